@@ -138,6 +138,28 @@ DIP_DEV float cvt_nibble_div16(uint32_t v) {
   return r;
 }
 
+// float(sext(byte n of v)) (v_cvt_f32_i32 reading the byte through SDWA).  With
+// a nibble in a byte's high half and zeros below, this is 16 q; times s / 16
+// (exact in fp32, subnormals included) it is q * s for every bf16 s, with no
+// overflow on the way.
+template <int N>
+DIP_DEV float cvt_sbyte(uint32_t v) {
+  float r;
+  if (N == 0)
+    asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0"
+        : "=v"(r) : "v"(v));
+  if (N == 1)
+    asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1"
+        : "=v"(r) : "v"(v));
+  if (N == 2)
+    asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2"
+        : "=v"(r) : "v"(v));
+  if (N == 3)
+    asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3"
+        : "=v"(r) : "v"(v));
+  return r;
+}
+
 // Sum over aligned groups of W lanes (W a power of two <= 64), every lane of
 // the group receiving the total: DPP within rows of 16 lanes (xor 1, xor 2,
 // half-row mirror, row mirror), then v_permlane16_swap / v_permlane32_swap to

@@ -92,8 +92,91 @@ __global__ __launch_bounds__(kAsmThreads) void ca_assemble_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Row dequantisation (bit-exact dequant check).
+// Row dequantisation.  Bound by the stores (bf16: 4 bytes out for each byte
+// in).  A thread turns one dword (8 columns) into one or two 128-bit stores,
+// kDqUnroll dwords apart by a block, so that a wave stores whole kilobytes and
+// has its loads in flight together; each value is one SDWA convert and one
+// multiply.  Rows in order are one flat run (the scale of dword e is e / 16).
+// 25600 x 5120 to bf16 (332 MB): 174 us with one byte per thread and two
+// 16-bit stores; 50 us in this form, 23 us for 5120 x 8192.
 // ---------------------------------------------------------------------------
+constexpr int kDqUnroll = 4;
+
+// 8 nibbles of w times the scale s16 / 16 (see dequant8_scale).
+DIP_DEV void dequant8(uint32_t w, float s16, float v[8]) {
+  const uint32_t lo = (w << 4) & 0xF0F0F0F0u, hi = w & 0xF0F0F0F0u;
+  v[0] = cvt_sbyte<0>(lo) * s16;
+  v[1] = cvt_sbyte<0>(hi) * s16;
+  v[2] = cvt_sbyte<1>(lo) * s16;
+  v[3] = cvt_sbyte<1>(hi) * s16;
+  v[4] = cvt_sbyte<2>(lo) * s16;
+  v[5] = cvt_sbyte<2>(hi) * s16;
+  v[6] = cvt_sbyte<3>(lo) * s16;
+  v[7] = cvt_sbyte<3>(hi) * s16;
+}
+
+template <int MODE>
+DIP_DEV void store_dequant8(uint32_t w, uint32_t s, bool bad, void* out, size_t dword) {
+  float v[8];
+  dequant8(w, bf16_to_f32(s) * 0.0625f, v);
+  if (bad) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = __builtin_nanf("");
+  }
+  if constexpr (MODE == 0) {
+    float4* o = reinterpret_cast<float4*>(out) + 2 * dword;
+    o[0] = make_float4(v[0], v[1], v[2], v[3]);
+    o[1] = make_float4(v[4], v[5], v[6], v[7]);
+  } else {
+    reinterpret_cast<uint4*>(out)[dword] =
+        make_uint4(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]),
+                   f32x2_to_bf16x2(v[4], v[5]), f32x2_to_bf16x2(v[6], v[7]));
+  }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(256) void dequant_flat_kernel(const uint32_t* __restrict__ qw,
+                                                           const uint16_t* __restrict__ sc,
+                                                           void* __restrict__ out, size_t ndwords) {
+  constexpr size_t kSpan = 256 * kDqUnroll;
+  for (size_t b = (size_t)blockIdx.x * kSpan; b < ndwords; b += (size_t)gridDim.x * kSpan) {
+    uint32_t w[kDqUnroll], s[kDqUnroll];
+#pragma unroll
+    for (int u = 0; u < kDqUnroll; ++u) {
+      const size_t e = b + threadIdx.x + 256 * u, c = e < ndwords ? e : ndwords - 1;
+      w[u] = qw[c];
+      s[u] = sc[c >> 4];
+    }
+#pragma unroll
+    for (int u = 0; u < kDqUnroll; ++u) {
+      const size_t e = b + threadIdx.x + 256 * u;
+      if (e < ndwords) store_dequant8<MODE>(w[u], s[u], false, out, e);
+    }
+  }
+}
+
+// Rows through an id list: workgroup y takes rows y, y + gridDim.y, ...
+template <int MODE>
+__global__ __launch_bounds__(256) void dequant_gather_kernel(const uint32_t* __restrict__ qw,
+                                                             const uint16_t* __restrict__ sc,
+                                                             const int32_t* __restrict__ indices,
+                                                             void* __restrict__ out, int n_out_rows,
+                                                             int rows, int row_dwords) {
+  for (int i = blockIdx.y; i < n_out_rows; i += gridDim.y) {
+    const int id = indices[i];
+    const bool bad = (unsigned)id >= (unsigned)rows;
+    if (bad && rows == 0) {
+      for (int c = blockIdx.x * 256 + threadIdx.x; c < row_dwords; c += gridDim.x * 256)
+        store_dequant8<MODE>(0u, 0u, true, out, (size_t)i * row_dwords + c);
+      continue;
+    }
+    const size_t r0 = (size_t)(bad ? 0 : id) * row_dwords;
+    for (int c = blockIdx.x * 256 + threadIdx.x; c < row_dwords; c += gridDim.x * 256)
+      store_dequant8<MODE>(qw[r0 + c], sc[(r0 + c) >> 4], bad, out, (size_t)i * row_dwords + c);
+  }
+}
+
+// One byte per thread: buffers that are not aligned for the vector forms.
 __global__ __launch_bounds__(256) void dequant_rows_kernel(
     const int8_t* __restrict__ qw, const uint16_t* __restrict__ sc,
     const int32_t* __restrict__ indices, void* __restrict__ out, int n_out_rows, int rows,
@@ -234,10 +317,34 @@ extern "C" int dip_dequant_rows(const int8_t* qweight, const uint16_t* scales,
   if (!indices && n_out_rows > rows) return DIP_ERR_SHAPE;
   if (mode != 0 && mode != 1) return DIP_ERR_ARG;
   if (n_out_rows == 0) return DIP_OK;
-  const size_t total = (size_t)n_out_rows * (size_t)(cols / 2);
-  const unsigned blocks = (unsigned)std::min<size_t>((total + 255) / 256, 4096);
-  hipLaunchKernelGGL(dequant_rows_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream,
-                     qweight, scales, indices, out, (int)n_out_rows, (int)rows, (int)cols, mode);
+  // The vector forms load dwords and store 128 bits; a caller's buffers need
+  // not be aligned for that.
+  const bool vec = (reinterpret_cast<uintptr_t>(qweight) & 3u) == 0 && aligned16(out);
+  hipStream_t s = (hipStream_t)stream;
+  if (vec && !indices) {
+    const size_t n = (size_t)n_out_rows * (size_t)(cols / 8);
+    const unsigned blocks = (unsigned)std::min<size_t>((n + 256 * kDqUnroll - 1) / (256 * kDqUnroll), 1u << 20);
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(qweight);
+    if (mode == 0)
+      hipLaunchKernelGGL(dequant_flat_kernel<0>, dim3(blocks), dim3(256), 0, s, q, scales, out, n);
+    else
+      hipLaunchKernelGGL(dequant_flat_kernel<1>, dim3(blocks), dim3(256), 0, s, q, scales, out, n);
+  } else if (vec) {
+    const int rd = (int)(cols / 8);
+    const dim3 grid((unsigned)((rd + 255) / 256), (unsigned)std::min<int64_t>(n_out_rows, 65535));
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(qweight);
+    if (mode == 0)
+      hipLaunchKernelGGL(dequant_gather_kernel<0>, grid, dim3(256), 0, s, q, scales, indices, out,
+                         (int)n_out_rows, (int)rows, rd);
+    else
+      hipLaunchKernelGGL(dequant_gather_kernel<1>, grid, dim3(256), 0, s, q, scales, indices, out,
+                         (int)n_out_rows, (int)rows, rd);
+  } else {
+    const size_t total = (size_t)n_out_rows * (size_t)(cols / 2);
+    const unsigned blocks = (unsigned)std::min<size_t>((total + 255) / 256, 4096);
+    hipLaunchKernelGGL(dequant_rows_kernel, dim3(blocks), dim3(256), 0, s, qweight, scales, indices,
+                       out, (int)n_out_rows, (int)rows, (int)cols, mode);
+  }
   return hip_status(hipGetLastError());
 }
 
