@@ -48,6 +48,14 @@ DIP_DEV uint32_t f32x2_to_bf16x2(float lo, float hi) {
   return r;
 }
 
+// The same without making NaN canonical, for values whose NaN bits nobody
+// sees: the conversion keeps a NaN a NaN.
+DIP_DEV uint32_t f32x2_to_bf16x2_nan(float lo, float hi) {
+  uint32_t r;
+  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(lo), "v"(hi));
+  return r;
+}
+
 // |v| as the bf16 key the top-k orders by: sign dropped, subnormal
 // magnitudes flushed to 0 (the reference's top-k kernels are built with
 // --use_fast_math, so fabsf flushes them).  NaN keys (> 0x7F80) are kept
