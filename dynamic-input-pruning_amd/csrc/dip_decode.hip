@@ -25,7 +25,7 @@ namespace {
 constexpr int kNormThreads = 256;
 constexpr int kNormVecs = 4;              // 16-byte vectors per thread: n <= 8192
 constexpr int kHeadDim = 128;
-constexpr int kAttnChunk = 32;            // cache positions per attention workgroup
+constexpr int kAttnChunk = 32;            // cache positions a wave takes at a time
 constexpr int kPartFloats = 2 + kHeadDim; // m, l, acc[128] per (kv head, chunk, query head)
 
 // Wave-wide reductions on DPP / permlane exchanges (no LDS round trips).
@@ -157,163 +157,243 @@ __global__ __launch_bounds__(64) void qk_rope_cache_kernel(
     reinterpret_cast<uint32_t*>(k_cache)[((size_t)(head - nh) * max_len + pos) * 64 + l] = o;
 }
 
-// Attention, pass 1: workgroup (one wave) = (32-row chunk c, kv head): the
-// scores of the G query heads over the chunk's rows up to pos on bf16 MFMA
-// (A = 16 cache rows, B = the q heads; exact products, fp32 sums), softmax
-// in fp32, the value sum in fp32 on the VALU (lane l: dimensions 2l, 2l + 1).
-// Writes per query head the chunk's max score m, sum of exp(s - m) and the
-// unnormalised value sum.
+// Attention over a long cache, pass 1.  The rows 0 .. pos are cut into
+// attn_rows_per_wave rows per wave, 4 waves to a workgroup (split) and
+// attn_splits splits per kv head at most, from pos itself: a cache that is
+// mostly empty still spreads over the chip.  A wave walks its rows 32 at a
+// time with a running (max, sum, value sum) per query head of the group:
+//   * scores on bf16 MFMA (A = 16 cache rows, B = the q heads, exact products,
+//     fp32 sums), both operands in memory order (slice j: lane quarter kb holds
+//     dims 32 j + 8 kb ..), so one load covers 64 contiguous bytes of a row;
+//   * softmax in fp32; the weights reach the value lanes through LDS;
+//   * values in fp32 on the VALU: lane l holds dims 8 (l % 16) .. + 7 of rows
+//     4 i + l / 16, a 128-bit load per four rows' worth of a wave.
+// At the end the four lane groups and the four waves are merged in a fixed
+// order and the split stores per query head its max, sum of exp and
+// unnormalised value sum.  Bound by HBM: 64 query / 8 kv heads, 20011 rows
+// (82 MB) 23 us, and 4.5 us for the merge of 63 splits.  (One wave and one
+// partial per 32 rows: 26 us, and 60 us to merge 626 of them in series.)
+constexpr int kAttnWaves = 4;
+constexpr int kAttnMaxSplits = 256;
+
+// Splits per kv head that fill the chip about twice over.
+inline int attn_splits(int nkv, int max_len) {
+  const int want = (2 * device_cus() + nkv - 1) / nkv;
+  const int most = (max_len + kAttnChunk * kAttnWaves - 1) / (kAttnChunk * kAttnWaves);
+  return max(1, min(min(want, most), kAttnMaxSplits));
+}
+
+// Cache rows attended at position pos: 0 .. pos, none before the first.
+DIP_DEV int attn_rows(int64_t pos, int max_len) {
+  return pos < 0 ? 0 : (pos < (int64_t)max_len ? (int)pos + 1 : max_len);
+}
+
+// Rows a wave takes of `rows`, never fewer than one chunk.
+DIP_DEV int attn_rows_per_wave(int rows, int splits) {
+  return max(kAttnChunk, (rows + splits * kAttnWaves - 1) / (splits * kAttnWaves));
+}
+
 template <int G>
-__global__ __launch_bounds__(64) void attn_partial_kernel(
+__global__ __launch_bounds__(kAttnWaves * 64) void attn_partial_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache,
     const uint16_t* __restrict__ v_cache, const int64_t* __restrict__ pos_p,
-    float* __restrict__ part, int max_len, int nchunks, float scale) {
+    float* __restrict__ part, int max_len, int splits, float scale) {
   static_assert(G <= 16, "one MFMA column per query head");
-  __shared__ __align__(16) uint32_t qb[16][64 + 4];  // q as bf16 pairs; heads >= G are 0
-  __shared__ float ps[G][kAttnChunk];
-  __shared__ float cm[G], cl[G];
-  const int c = blockIdx.x, kvh = blockIdx.y, l = threadIdx.x;
+  constexpr int GP = G <= 2 ? G : (G + 3) / 4 * 4;  // LDS row of weights
+  __shared__ __align__(16) float ps[kAttnWaves][kAttnChunk][GP];
+  __shared__ __align__(16) float fac[kAttnWaves][GP];
+  __shared__ float wm[kAttnWaves][G], wl[kAttnWaves][G];
+  __shared__ __align__(16) float wacc[kAttnWaves][G][kHeadDim];
+  const int split = blockIdx.x, kvh = blockIdx.y;
+  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int l16 = l & 15, kb = l >> 4;
   const int64_t pos = *pos_p;
-  const int64_t last = pos < (int64_t)max_len ? pos : (int64_t)max_len - 1;
-  const int start = c * kAttnChunk;
-  if ((int64_t)start > last) return;  // no position of this chunk is attended
-  const int npos = (int)((last - start + 1) < kAttnChunk ? (last - start + 1) : kAttnChunk);
-
-  uint4 ka[2][4];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int row = start + 16 * t + l16;
-    if ((int64_t)row <= last) {
-      const uint4* src = reinterpret_cast<const uint4*>(
-          k_cache + ((size_t)kvh * max_len + row) * kHeadDim + 32 * kb);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) ka[t][j] = src[j];
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) ka[t][j] = make_uint4(0, 0, 0, 0);
-    }
-  }
-  const uint32_t* vcol =
-      reinterpret_cast<const uint32_t*>(v_cache + ((size_t)kvh * max_len + start) * kHeadDim) + l;
-  uint32_t vv[kAttnChunk];
-#pragma unroll
-  for (int j = 0; j < kAttnChunk; ++j) vv[j] = j < npos ? vcol[(size_t)j * 64] : 0u;
-  const uint32_t* qsrc = reinterpret_cast<const uint32_t*>(q + (size_t)kvh * G * kHeadDim);
-  for (int i = l; i < 16 * 64; i += 64) qb[i >> 6][i & 63] = (i >> 6) < G ? qsrc[i] : 0u;
-  __syncthreads();
+  const int rows = attn_rows(pos, max_len);
+  const int rpw = attn_rows_per_wave(rows, splits);
+  if (rows <= 0 || split >= (rows + kAttnWaves * rpw - 1) / (kAttnWaves * rpw)) return;
+  const int r0 = min((split * kAttnWaves + wave) * rpw, rows), r1 = min(r0 + rpw, rows);
+  const uint16_t* kbase = k_cache + (size_t)kvh * max_len * kHeadDim;
+  const uint16_t* vbase = v_cache + (size_t)kvh * max_len * kHeadDim;
 
   uint4 bq[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) bq[j] = *reinterpret_cast<const uint4*>(&qb[l16][16 * kb + 4 * j]);
-  float sc[2][4];
+  for (int j = 0; j < 4; ++j)
+    bq[j] = l16 < G ? reinterpret_cast<const uint4*>(q + (size_t)(kvh * G + l16) * kHeadDim)[4 * j + kb]
+                    : make_uint4(0, 0, 0, 0);
+  float acc[G][8];
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    floatx4 d = {0.f, 0.f, 0.f, 0.f};
+  for (int g = 0; g < G; ++g)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(ka[t][j]), as_bf16x8(bq[j]), d, 0, 0,
-                                                  0);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) sc[t][r] = 16 * t + 4 * kb + r < npos ? d[r] * scale : -INFINITY;
-  }
-  float mx = -INFINITY;
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[t][r]);
-  mx = row_pair_max32(row_pair_max16(mx));
-  float sum = 0.f;
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float e = sc[t][r] == -INFINITY ? 0.f : expf(sc[t][r] - mx);
-      sum += e;
-      if (l16 < G) ps[l16][16 * t + 4 * kb + r] = e;
-    }
-  sum = row_pair_sum32(row_pair_sum16(sum));
-  if (kb == 0 && l16 < G) {
-    cm[l16] = mx;
-    cl[l16] = sum;
-  }
-  __syncthreads();
+    for (int d = 0; d < 8; ++d) acc[g][d] = 0.f;
+  float m = -INFINITY, den = 0.f;  // of head l16
 
-  float a0[G], a1[G];
+  for (int start = r0; start < r1; start += kAttnChunk) {
+    const int npos = min(r1 - start, kAttnChunk);
+    uint4 ka[2][4], vv[8];
 #pragma unroll
-  for (int g = 0; g < G; ++g) a0[g] = a1[g] = 0.f;
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-  for (int j = 0; j < kAttnChunk; ++j) {
-    if (j < npos) {
-      const float v0 = bf16_to_f32(vv[j] & 0xFFFFu), v1 = bf16_to_f32(vv[j] >> 16);
+      for (int j = 0; j < 4; ++j) {
+        ka[t][j] = make_uint4(0, 0, 0, 0);
+        if (16 * t + l16 < npos)
+          ka[t][j] = ldg_nt(reinterpret_cast<const uint4*>(
+                                kbase + (size_t)(start + 16 * t + l16) * kHeadDim) + 4 * j + kb);
+      }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      vv[i] = make_uint4(0, 0, 0, 0);
+      if (4 * i + kb < npos)
+        vv[i] = ldg_nt(reinterpret_cast<const uint4*>(
+                           vbase + (size_t)(start + 4 * i + kb) * kHeadDim) + l16);
+    }
+    float sc[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      floatx4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(ka[t][j]), as_bf16x8(bq[j]), d, 0, 0,
+                                                    0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sc[t][r] = 16 * t + 4 * kb + r < npos ? d[r] * scale : -INFINITY;
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[t][r]);
+    mx = fmaxf(m, row_pair_max32(row_pair_max16(mx)));
+    const float f = m == -INFINITY ? 0.f : expf(m - mx);  // what the sums so far are worth
+    float sum = 0.f;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float e = sc[t][r] == -INFINITY ? 0.f : expf(sc[t][r] - mx);
+        sum += e;
+        if (l16 < G) ps[wave][16 * t + 4 * kb + r][l16] = e;
+      }
+    if (kb == 0 && l16 < G) fac[wave][l16] = f;
+    den = den * f + row_pair_sum32(row_pair_sum16(sum));
+    m = mx;
+    // the wave's own LDS writes before its reads
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const float fg = fac[wave][g];
+#pragma unroll
+      for (int d = 0; d < 8; ++d) acc[g][d] *= fg;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t w[4] = {vv[i].x, vv[i].y, vv[i].z, vv[i].w};
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[2 * e] = bf16_to_f32(w[e] & 0xFFFFu);
+        v[2 * e + 1] = __uint_as_float(w[e] & 0xFFFF0000u);
+      }
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        a0[g] = fmaf(ps[g][j], v0, a0[g]);
-        a1[g] = fmaf(ps[g][j], v1, a1[g]);
+        const float pg = ps[wave][4 * i + kb][g];
+#pragma unroll
+        for (int d = 0; d < 8; ++d) acc[g][d] = fmaf(pg, v[d], acc[g][d]);
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
-  float* out = part + ((size_t)kvh * nchunks + c) * G * kPartFloats;
+
+  if (kb == 0 && l16 < G) {
+    wm[wave][l16] = m;
+    wl[wave][l16] = den;
+  }
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    float* o = out + g * kPartFloats;
-    if (l == 0) {
-      o[0] = cm[g];
-      o[1] = cl[g];
+#pragma unroll
+    for (int d = 0; d < 8; ++d) acc[g][d] = row_pair_sum32(row_pair_sum16(acc[g][d]));
+    if (kb == (g & 3)) {
+      float4* o = reinterpret_cast<float4*>(&wacc[wave][g][8 * l16]);
+      o[0] = make_float4(acc[g][0], acc[g][1], acc[g][2], acc[g][3]);
+      o[1] = make_float4(acc[g][4], acc[g][5], acc[g][6], acc[g][7]);
     }
-    o[2 + 2 * l] = a0[g];
-    o[3 + 2 * l] = a1[g];
+  }
+  __syncthreads();
+  float* out = part + ((size_t)kvh * splits + split) * G * kPartFloats;
+  for (int e = threadIdx.x; e < G * kHeadDim; e += kAttnWaves * 64) {
+    const int g = e / kHeadDim, d = e % kHeadDim;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kAttnWaves; ++w) mx = fmaxf(mx, wm[w][g]);
+    float s = 0.f, o = 0.f;
+#pragma unroll
+    for (int w = 0; w < kAttnWaves; ++w) {
+      const float f = wl[w][g] > 0.f ? expf(wm[w][g] - mx) : 0.f;
+      s = fmaf(f, wl[w][g], s);
+      o = fmaf(f, wacc[w][g][d], o);
+    }
+    if (d == 0) {
+      out[g * kPartFloats] = mx;
+      out[g * kPartFloats + 1] = s;
+    }
+    out[g * kPartFloats + 2 + d] = o;
   }
 }
 
-// Attention, pass 2: one workgroup per query head merges the chunks
-// 0 .. pos/32: wave w takes chunks w, w + 4, ... with a one-pass running
-// rescale (max, sum, value sum), then the 4 waves merge through LDS in a
-// fixed order and write bf16(sum / l).
-__global__ __launch_bounds__(256) void attn_combine_kernel(
+// Attention, pass 2: one workgroup per query head.  The splits' weights first
+// (one thread per split), then dimension d on the threads d, d + 128, ...,
+// which sum every fourth split; the four sums are added in order.
+__global__ __launch_bounds__(4 * kHeadDim) void attn_combine_kernel(
     const float* __restrict__ part, const int64_t* __restrict__ pos_p, uint16_t* __restrict__ out,
-    int G, int max_len, int nchunks) {
-  __shared__ float wm[4], wl[4];
-  __shared__ float wa[4][kHeadDim];
-  const int qh = blockIdx.x, wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int kvh = qh / G, g = qh % G;
+    int G, int max_len, int splits) {
+  __shared__ float wgt[kAttnMaxSplits];
+  __shared__ float red[8][2];
+  __shared__ float so[4][kHeadDim];
+  const int qh = blockIdx.x, kvh = qh / G, g = qh % G, tid = threadIdx.x;
   const int64_t pos = *pos_p;
-  const int64_t last = pos < (int64_t)max_len ? pos : (int64_t)max_len - 1;
-  const int nc = last < 0 ? 0 : (int)(last / kAttnChunk) + 1;
-  const float* base = part + (size_t)kvh * nchunks * G * kPartFloats + (size_t)g * kPartFloats;
+  const int rows = attn_rows(pos, max_len);
+  const int rpw = attn_rows_per_wave(max(rows, 1), splits);
+  const int ns = rows <= 0 ? 0 : (rows + kAttnWaves * rpw - 1) / (kAttnWaves * rpw);
   const size_t stride = (size_t)G * kPartFloats;
-  float mx = -INFINITY, den = 0.f, a0 = 0.f, a1 = 0.f;
-  for (int c = wave; c < nc; c += 4) {
-    const float* pc = base + c * stride;
-    const float mc = pc[0], lc = pc[1], v0 = pc[2 + 2 * l], v1 = pc[3 + 2 * l];
-    const float mn = fmaxf(mx, mc);
-    const float fo = expf(mx - mn), fn = expf(mc - mn);
-    den = den * fo + lc * fn;
-    a0 = a0 * fo + v0 * fn;
-    a1 = a1 * fo + v1 * fn;
-    mx = mn;
-  }
-  if (l == 0) {
-    wm[wave] = mx;
-    wl[wave] = den;
-  }
-  wa[wave][2 * l] = a0;
-  wa[wave][2 * l + 1] = a1;
+  const float* base = part + (size_t)kvh * splits * stride + (size_t)g * kPartFloats;
+  const int d = tid % kHeadDim, p = tid / kHeadDim;
+  const float ms = tid < ns ? base[tid * stride] : -INFINITY;
+  const float ls = tid < ns ? base[tid * stride + 1] : 0.f;
+  float mx = wave_max(ms);
+  if ((tid & 63) == 0) red[tid >> 6][0] = mx;
   __syncthreads();
-  if (wave != 0) return;
-  float m = -INFINITY;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) m = fmaxf(m, wm[w]);
-  float d = 0.f, o0 = 0.f, o1 = 0.f;
+  for (int w = 0; w < 8; ++w) mx = fmaxf(mx, red[w][0]);
+  const float f = ls > 0.f ? expf(ms - mx) : 0.f;
+  if (tid < kAttnMaxSplits) wgt[tid] = f;
+  const float dsum = wave_sum(f * ls);
+  if ((tid & 63) == 0) red[tid >> 6][1] = dsum;
+  __syncthreads();
+  float den = 0.f;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const float f = wl[w] > 0.f ? expf(wm[w] - m) : 0.f;
-    d = fmaf(f, wl[w], d);
-    o0 = fmaf(f, wa[w][2 * l], o0);
-    o1 = fmaf(f, wa[w][2 * l + 1], o1);
+  for (int w = 0; w < 8; ++w) den += red[w][1];
+  float o = 0.f;
+  for (int s0 = p; s0 < ns; s0 += 32) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = base[min(s0 + 4 * u, ns - 1) * stride + 2 + d];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (s0 + 4 * u < ns) o = fmaf(wgt[s0 + 4 * u], v[u], o);
   }
-  reinterpret_cast<uint32_t*>(out)[(size_t)qh * 64 + l] =
-      f32_to_bf16(o0 / d) | (f32_to_bf16(o1 / d) << 16);
+  so[p][d] = o;
+  __syncthreads();
+  if (tid < kHeadDim / 2) {
+    float r[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int c = 2 * tid + e;
+      r[e] = ((so[0][c] + so[1][c]) + so[2][c]) + so[3][c];
+    }
+    reinterpret_cast<uint32_t*>(out)[(size_t)qh * 64 + tid] =
+        f32_to_bf16(r[0] / den) | (f32_to_bf16(r[1] / den) << 16);
+  }
 }
 
 // Norm + rotary + cache write + attention in one launch, for caches of at
@@ -566,12 +646,13 @@ __global__ __launch_bounds__(NW * 64) void attn_fused_kernel(
 
 template <int G>
 void launch_attention(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int64_t* pos,
-                      uint16_t* out, int nkv, int max_len, int nchunks, float scale, float* part,
+                      uint16_t* out, int nkv, int max_len, float scale, float* part,
                       hipStream_t stream) {
-  hipLaunchKernelGGL((attn_partial_kernel<G>), dim3(nchunks, nkv), dim3(64), 0, stream, q, kc, vc,
-                     pos, part, max_len, nchunks, scale);
-  hipLaunchKernelGGL(attn_combine_kernel, dim3(nkv * G), dim3(256), 0, stream, part, pos, out, G,
-                     max_len, nchunks);
+  const int splits = attn_splits(nkv, max_len);
+  hipLaunchKernelGGL((attn_partial_kernel<G>), dim3(splits, nkv), dim3(kAttnWaves * 64), 0, stream,
+                     q, kc, vc, pos, part, max_len, splits, scale);
+  hipLaunchKernelGGL(attn_combine_kernel, dim3(nkv * G), dim3(4 * kHeadDim), 0, stream, part, pos,
+                     out, G, max_len, splits);
 }
 
 }  // namespace
@@ -674,17 +755,16 @@ extern "C" int dip_decode_attention(const uint16_t* q, const uint16_t* k_cache,
   if (!aligned16(workspace)) return DIP_ERR_ALIGN;
   const int nkv = (int)n_kv_heads;
   const int G = (int)(n_heads / n_kv_heads);
-  const int nchunks = (int)((max_len + kAttnChunk - 1) / kAttnChunk);
   float* part = static_cast<float*>(workspace);
   hipStream_t s = (hipStream_t)stream;
   const int ml = (int)max_len;
   switch (G) {
-    case 1: launch_attention<1>(q, k_cache, v_cache, pos, out, nkv, ml, nchunks, scale, part, s); break;
-    case 2: launch_attention<2>(q, k_cache, v_cache, pos, out, nkv, ml, nchunks, scale, part, s); break;
-    case 4: launch_attention<4>(q, k_cache, v_cache, pos, out, nkv, ml, nchunks, scale, part, s); break;
-    case 5: launch_attention<5>(q, k_cache, v_cache, pos, out, nkv, ml, nchunks, scale, part, s); break;
-    case 8: launch_attention<8>(q, k_cache, v_cache, pos, out, nkv, ml, nchunks, scale, part, s); break;
-    case 16: launch_attention<16>(q, k_cache, v_cache, pos, out, nkv, ml, nchunks, scale, part, s); break;
+    case 1: launch_attention<1>(q, k_cache, v_cache, pos, out, nkv, ml, scale, part, s); break;
+    case 2: launch_attention<2>(q, k_cache, v_cache, pos, out, nkv, ml, scale, part, s); break;
+    case 4: launch_attention<4>(q, k_cache, v_cache, pos, out, nkv, ml, scale, part, s); break;
+    case 5: launch_attention<5>(q, k_cache, v_cache, pos, out, nkv, ml, scale, part, s); break;
+    case 8: launch_attention<8>(q, k_cache, v_cache, pos, out, nkv, ml, scale, part, s); break;
+    case 16: launch_attention<16>(q, k_cache, v_cache, pos, out, nkv, ml, scale, part, s); break;
     default: return DIP_ERR_UNSUPPORTED;
   }
   return hip_status(hipGetLastError());

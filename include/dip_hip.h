@@ -535,7 +535,7 @@ int dip_qk_norm_rope_cache(const uint16_t* qkv, const uint16_t* q_norm_w,
  * dip_decode_attention: out[h] = softmax(scale * q[h] . K[j]) V over cache
  * rows j = 0 .. pos of kv head h / (n_heads / n_kv_heads) (grouped-query
  * attention of one token; fp32 scores, softmax and sums, bf16 output).
- * Two launches: per (32-row chunk, kv head) partial sums into the workspace
+ * Two launches: per (range of rows, kv head) partial sums into the workspace
  * (dip_decode_attention_workspace_size bytes), then one merge per query
  * head.  head_dim 128 and n_heads / n_kv_heads in {1, 2, 4, 5, 8, 16}
  * (else DIP_ERR_UNSUPPORTED).
