@@ -6,30 +6,16 @@
 // dip_stream_predispatch.py:206-215 for gate and up): it writes a bf16 copy
 // of W and reads it back in a GEMM.  Here each weight is read once, as
 // packed nibbles, and turned into an MFMA operand in registers:
-//   * a nibble u (two's complement q) becomes the bf16 value 136 + q, exact:
-//     0x4300 | (u ^ 8) is 128 + (q + 8), so 8 nibbles need a few bit ops;
-//   * v_mfma_f32_16x16x32_bf16 sums (136 + q) * x over one 128-column group
-//     in fp32; subtracting 136 * sum(x) of the group leaves sum(q * x),
-//     which is scaled by the group's scale and added to the fp32 total.
+//   * a nibble u (two's complement q) in mantissa bits 3..6 of bf16 16.0, its
+//     top bit flipped, is 24 + q exactly; nibbles j and j + 4 of a dword sit
+//     16 bits apart, so two weights cost a shift and one v_bitop3;
+//   * x is paired the same way, (x[c + j], x[c + j + 4]), on its way into LDS;
+//   * v_mfma_f32_16x16x32_bf16 sums (24 + q) * x over one 128-column group in
+//     fp32, starting from -24 * sum(x) of the group, which the same MFMA gives
+//     with a constant operand: the result is sum(q * x), scaled by the group's
+//     scale into the fp32 total.
 // So the weights enter exactly as q * s in fp32 (the reference rounds q * s
 // to bf16 first); the output is rounded to bf16 once.
-//
-// Tiling: a wave owns RW tiles of 16 weight rows and 16 * TM tokens, so each
-// x operand it loads feeds RW row tiles (x comes from L2, and with one row
-// tile per wave its re-reads, not the weights, bounded the kernel: the
-// 32-token 25600 x 5120 product took 91 us with RW = 1, 46 us with RW = 4);
-// the 136 * sum(x) term is computed once per x operand.  A workgroup is 4
-// waves on RT such row super-tiles; the 4 / RT waves of one super-tile
-// split the K groups between them (wave ks takes groups ks, ks + KS, ...)
-// and add their partial sums through LDS at the end, in a fixed order.
-// Nothing else is shared: each lane loads its own 16 bytes of nibbles per
-// row tile and 64 bytes of x per group, weights and scales PW groups ahead
-// and x two groups ahead, so no barrier sits in the main loop.  RW is 4 for
-// at least 8192 rows, else 2 (fewer, larger tiles leave CUs idle there).  Inside a 32-column MFMA slice the k
-// order is permuted identically for both operands (lane quarter kb holds
-// columns 32 kb .. 32 kb + 31 and slice j uses its 8 columns 8j .. 8j + 7),
-// so a lane's nibbles are one contiguous 16-byte load.  The offset term
-// 136 * sum(x) comes from the same MFMA with a constant operand.
 #include <algorithm>
 
 #include "dip_common.h"
@@ -42,210 +28,524 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kGemmThreads = 256;
-constexpr uint32_t kOffsetPair = 0x43084308u;  // bf16 136.0, twice
-
-// 8 nibbles (element p = nibble p of w) -> the 8 bf16 values 136 + q.
-DIP_DEV bf16x8_t offset_bf16x8(uint32_t w) {
-  const uint32_t t = w ^ 0x88888888u;  // q + 8 in every nibble
-  u32x4_t p;
-  p.x = 0x43004300u | (t & 0xFu) | ((t & 0xF0u) << 12);
-  p.y = 0x43004300u | ((t >> 8) & 0xFu) | ((t & 0xF000u) << 4);
-  p.z = 0x43004300u | ((t >> 16) & 0xFu) | ((t >> 4) & 0xF0000u);
-  p.w = 0x43004300u | ((t >> 24) & 0xFu) | ((t >> 12) & 0xF0000u);
-  return __builtin_bit_cast(bf16x8_t, p);
-}
+constexpr uint32_t kPair24 = 0x41C041C0u;    // bf16 16.0 twice, the nibbles' top bits flipped
+constexpr uint32_t kMinus24 = 0xC1C0C1C0u;   // bf16 -24.0, twice
 
 DIP_DEV bf16x8_t as_bf16x8(const uint4& v) {
   return __builtin_bit_cast(bf16x8_t, u32x4_t{v.x, v.y, v.z, v.w});
 }
 
-template <int TM, int RT, int PW, int RW>
-__global__ __launch_bounds__(kGemmThreads) void int4_gemm_kernel(
+// 8 nibbles -> 24 + q as bf16, in the order 0, 4, 1, 5, 2, 6, 3, 7.
+DIP_DEV bf16x8_t weights24(uint32_t w) {
+  return __builtin_bit_cast(
+      bf16x8_t, u32x4_t{((w << 3) & kPairMask) ^ kPair24, ((w >> 1) & kPairMask) ^ kPair24,
+                        ((w >> 5) & kPairMask) ^ kPair24, ((w >> 9) & kPairMask) ^ kPair24});
+}
+
+constexpr size_t kGemmLds = 160 * 1024;
+constexpr int kXcds = 8;  // workgroups go to the 8 XCDs round-robin
+
+// ---------------------------------------------------------------------------
+// Few tokens (or few rows): K split over a workgroup's waves.  16 TM tokens and
+// RW tiles of 16 weight rows per workgroup, whose KS waves take the K groups ks,
+// ks + KS, ... and add their sums through LDS at the end, in a fixed order.
+// Bound by HBM, or by the launch.  Per group a wave
+//   * has its RW x 16 rows' nibbles in flight D groups ahead (lane: row l16,
+//     columns 32 kb ..: 16 bytes, so 64 contiguous bytes of each row; cached,
+//     since the next wave reads the other half of the same lines: with
+//     streaming loads 25600 x 5120 took 30 us instead of 25);
+//   * stages its own x tile in LDS, loaded a group ahead by whole 256-byte token
+//     rows (read as operands from memory, 16 bytes of 64 different lines per
+//     load, x bounds the kernel), chunk c of token t at slot c ^ (t % 16), which
+//     is free of bank conflicts on both sides; nothing is shared, so the loop
+//     has no barrier;
+//   * works on UB row tiles at a time, UB * TM independent chains of MFMAs (one
+//     chain at a time left the matrix cores waiting: 20.6 us of 25 us).
+// 25600 x 5120: 2 tokens 27.8 -> 22 us, 32 tokens 45.5 -> 30 us; 10240 x 5120,
+// 7 tokens 17.1 -> 12 us; 5120 x 8192, 32 tokens 24.5 -> 16 us (before: RW
+// tiles and K parts by the matrix alone, x and 16-bit scales from memory).
+// Tokens are the MFMA's rows, so that a lane's 4 sums belong to one weight row
+// and share its scale.  The scales of the workgroup's rows are one contiguous
+// run, staged in LDS once (SCL) unless K is too long for that or they are not
+// 4-byte aligned.
+// ---------------------------------------------------------------------------
+constexpr int kScaleRegs = 5;  // scale dwords a thread holds before the first barrier
+
+template <int TM, int RW, int KS, int D, bool SCL>
+__global__ __launch_bounds__(KS * 64, 2) void int4_gemm_split_kernel(
     const int8_t* __restrict__ qw, const uint16_t* __restrict__ sc, const uint16_t* __restrict__ x,
-    uint16_t* __restrict__ out, int M, int N, int K) {
-  static_assert(PW % 2 == 0, "x ring of 2 inside the weight ring");
-  constexpr int KS = 4 / RT;  // waves per row super-tile (K split)
-  __shared__ float red[KS > 1 ? 4 : 1][RW][TM][4][64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int rt = wave / KS, ks = wave % KS;
-  // this wave's RW 16-row tiles: rows row0 + 16 u + ...
-  const int row0 = (blockIdx.x * RT + rt) * (16 * RW);
-  const int tok0 = blockIdx.y * TM * 16;
-  const int ngroups = K >> 7;
-  const int ng = ngroups > ks ? (ngroups - ks + KS - 1) / KS : 0;  // this wave's groups
+    uint16_t* __restrict__ out, int M, int N, int K, int row_blocks) {
+  extern __shared__ __align__(16) uint4 gemm_lds[];
+  constexpr int kThreads = KS * 64;
+  constexpr int XT = TM * 256;         // 16-byte chunks of a wave's x tile
+  constexpr int UB = TM == 1 ? 4 : 2;  // row tiles worked on together
+  const int ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int kb = lane >> 4, l16 = lane & 15;
+  // Row tile u starts at a row that leaves it 16 rows (a matrix of fewer than
+  // 16: its lanes past the last row repeat it); tiles that overlap compute and
+  // store the same values.
+  const int row0 = max(0, min((int)(blockIdx.x % row_blocks) * (16 * RW), N - 16));
+  auto tile_row = [&](int u) { return max(0, min(row0 + 16 * u, N - 16)); };
+  const int lrow = min(l16, N - 1);
+  const int tok0 = (int)(blockIdx.x / row_blocks) * (16 * TM);
+  const int ngroups = K >> 7;
+  const int ng = ngroups > ks ? (ngroups - ks + KS - 1) / KS : 0;
+  const int glast = ks + (ng - 1) * KS;  // loads past the end repeat the last group
+  uint4* xt = gemm_lds + ks * XT;
+  uint32_t* ssc = reinterpret_cast<uint32_t*>(gemm_lds + KS * XT);
 
-  // A operand: weight row l16 of tile u, columns 32 kb .. 32 kb + 31 of each group
-  const uint4* wp[RW];
-  // D: token l16, rows 4 kb + r of tile u; their scales
-  const uint16_t* sp[RW][4];
+  [[maybe_unused]] uint32_t sreg[kScaleRegs];
+  const int n_sc = min(16 * RW, N - row0) * ngroups;  // this workgroup's scales
+  const uint16_t* sc0 = sc + (size_t)row0 * ngroups;
+  if constexpr (SCL) {
 #pragma unroll
-  for (int u = 0; u < RW; ++u) {
-    wp[u] = reinterpret_cast<const uint4*>(qw + (size_t)min(row0 + 16 * u + l16, N - 1) *
-                                                     (K >> 1)) + kb;
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      sp[u][r] = sc + (size_t)min(row0 + 16 * u + 4 * kb + r, N - 1) * ngroups;
-  }
-  // B operand: token l16 of each 16-token tile, the same columns
-  const uint4* xp[TM];
-#pragma unroll
-  for (int t = 0; t < TM; ++t)
-    xp[t] = reinterpret_cast<const uint4*>(x + (size_t)min(tok0 + t * 16 + l16, M - 1) * K) +
-            4 * kb;
-
-  uint4 wq[PW][RW];
-  uint32_t sq[PW][RW][4];
-  uint4 xq[2][TM][4];
-#pragma unroll
-  for (int p = 0; p < PW; ++p) {
-    if (p < ng) {
-      const int g = ks + p * KS;
-#pragma unroll
-      for (int u = 0; u < RW; ++u) {
-        wq[p][u] = wp[u][4 * g];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sq[p][u][r] = sp[u][r][g];
-      }
+    for (int i = 0; i < kScaleRegs; ++i) {
+      const int e = 2 * (i * kThreads + (int)threadIdx.x);
+      // an odd count's last value is loaded alone: the run may end the matrix
+      sreg[i] = e + 1 < n_sc ? *reinterpret_cast<const uint32_t*>(sc0 + e) : e < n_sc ? sc0[e] : 0u;
     }
   }
+  const uint32_t woff = (uint32_t)lrow * (uint32_t)(K >> 1) + 16u * kb;
+  const char* xbase = reinterpret_cast<const char*>(x + (size_t)tok0 * K);
+  const int tlast = M - 1 - tok0;
+  uint4 xr[TM * 4], w[D][RW];
+  [[maybe_unused]] uint32_t s[D][RW];
+  auto load_x = [&](int g) {
 #pragma unroll
-  for (int p = 0; p < 2; ++p) {
-    if (p < ng) {
-      const int g = ks + p * KS;
+    for (int i = 0; i < TM * 4; ++i)
+      xr[i] = *reinterpret_cast<const uint4*>(
+          xbase + (size_t)g * 256 +
+          ((uint32_t)min(4 * i + kb, tlast) * (uint32_t)(2 * K) + (uint32_t)(16 * l16)));
+  };
+  auto stage_x = [&] {
 #pragma unroll
-      for (int t = 0; t < TM; ++t)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) xq[p][t][v] = xp[t][16 * g + v];
+    for (int i = 0; i < TM * 4; ++i) {
+      const int t = 4 * i + kb;
+      uint32_t p[4];
+      make_xpairs(xr[i].x, xr[i].y, xr[i].z, xr[i].w, p);
+      xt[t * 16 + (l16 ^ (t & 15))] = make_uint4(p[0], p[1], p[2], p[3]);
     }
-  }
-
-  const bf16x8_t c136 = __builtin_bit_cast(
-      bf16x8_t, u32x4_t{kOffsetPair, kOffsetPair, kOffsetPair, kOffsetPair});
+  };
+  auto load_w = [&](int d, int u, int g) {
+    const int8_t* p = qw + (size_t)tile_row(u) * (K >> 1) + (size_t)g * 64;
+    w[d][u] = *reinterpret_cast<const uint4*>(p + woff);
+    if constexpr (!SCL) s[d][u] = sc[(size_t)(tile_row(u) + lrow) * ngroups + g];
+  };
   floatx4 acc[RW][TM];
 #pragma unroll
   for (int u = 0; u < RW; ++u)
 #pragma unroll
     for (int t = 0; t < TM; ++t) acc[u][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  if (ng > 0) {
+    load_x(ks);
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+#pragma unroll
+      for (int u = 0; u < RW; ++u) load_w(d, u, min(ks + d * KS, glast));
+    stage_x();
+  }
+  if constexpr (SCL) {
+#pragma unroll
+    for (int i = 0; i < kScaleRegs; ++i) {
+      const int e = i * kThreads + (int)threadIdx.x;
+      if (2 * e < n_sc) ssc[e] = sreg[i];
+    }
+    for (int e = kScaleRegs * kThreads + (int)threadIdx.x; 2 * e < n_sc; e += kThreads)
+      ssc[e] = 2 * e + 1 < n_sc ? *reinterpret_cast<const uint32_t*>(sc0 + 2 * e) : sc0[2 * e];
+    __syncthreads();
+  }
 
-  for (int i0 = 0; i0 < ng; i0 += PW) {
+  const bf16x8_t m24 = __builtin_bit_cast(bf16x8_t, u32x4_t{kMinus24, kMinus24, kMinus24, kMinus24});
+  for (int i0 = 0; i0 < ng; i0 += D) {
 #pragma unroll
-    for (int p = 0; p < PW; ++p) {
-      const int i = i0 + p;
+    for (int d = 0; d < D; ++d) {
+      const int i = i0 + d;
       if (i < ng) {
-        // 136 * (sum of the group's x) per token: shared by the RW row tiles
-        floatx4 d1[TM];
+        const int g = ks + i * KS;
+        load_x(min(g + KS, glast));
+        bf16x8_t xa[TM][4];
+        floatx4 c[TM];  // -24 * (the group's sum of x) per token
 #pragma unroll
-        for (int t = 0; t < TM; ++t) {
-          d1[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int v = 0; v < 4; ++v)
-            d1[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c136, as_bf16x8(xq[p & 1][t][v]),
-                                                            d1[t], 0, 0, 0);
-        }
-#pragma unroll
-        for (int u = 0; u < RW; ++u) {
-          const bf16x8_t a0 = offset_bf16x8(wq[p][u].x), a1 = offset_bf16x8(wq[p][u].y);
-          const bf16x8_t a2 = offset_bf16x8(wq[p][u].z), a3 = offset_bf16x8(wq[p][u].w);
-          float s4[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) s4[r] = bf16_to_f32(sq[p][u][r]);
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
           for (int t = 0; t < TM; ++t) {
-            floatx4 d = {0.f, 0.f, 0.f, 0.f};
-            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, as_bf16x8(xq[p & 1][t][0]), d, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, as_bf16x8(xq[p & 1][t][1]), d, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, as_bf16x8(xq[p & 1][t][2]), d, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a3, as_bf16x8(xq[p & 1][t][3]), d, 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              acc[u][t][r] = fmaf(s4[r], d[r] - d1[t][r], acc[u][t][r]);
+            xa[t][j] = as_bf16x8(xt[(16 * t + l16) * 16 + ((4 * kb + j) ^ l16)]);
+            c[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                xa[t][j], m24, j ? c[t] : floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
           }
-        }
-        if (i + PW < ng) {
-          const int g = ks + (i + PW) * KS;
 #pragma unroll
-          for (int u = 0; u < RW; ++u) {
-            wq[p][u] = wp[u][4 * g];
+        for (int u0 = 0; u0 < RW; u0 += UB) {
+          float sf[UB];
+          bf16x8_t b[UB][4];
+          floatx4 v[UB][TM];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) sq[p][u][r] = sp[u][r][g];
+          for (int q = 0; q < UB; ++q) {
+            const int u = u0 + q;
+            if (u < RW) {
+              if constexpr (SCL)
+                sf[q] = bf16_to_f32(
+                    reinterpret_cast<const uint16_t*>(ssc)[(tile_row(u) - row0 + lrow) * ngroups + g]);
+              else
+                sf[q] = bf16_to_f32(s[d][u]);
+              b[q][0] = weights24(w[d][u].x);
+              b[q][1] = weights24(w[d][u].y);
+              b[q][2] = weights24(w[d][u].z);
+              b[q][3] = weights24(w[d][u].w);
+              load_w(d, u, min(g + D * KS, glast));
+            }
           }
-        }
-        if (i + 2 < ng) {
-          const int g = ks + (i + 2) * KS;
 #pragma unroll
-          for (int t = 0; t < TM; ++t)
+          for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) xq[p & 1][t][v] = xp[t][16 * g + v];
+            for (int q = 0; q < UB; ++q)
+#pragma unroll
+              for (int t = 0; t < TM; ++t)
+                if (u0 + q < RW)
+                  v[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                      xa[t][j], b[q][j], j ? v[q][t] : c[t], 0, 0, 0);
+          if (u0 + UB >= RW) stage_x();  // the next group's tile over this one's
+#pragma unroll
+          for (int q = 0; q < UB; ++q)
+#pragma unroll
+            for (int t = 0; t < TM; ++t)
+              if (u0 + q < RW)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                  acc[u0 + q][t][r] = fmaf(sf[q], v[q][t][r], acc[u0 + q][t][r]);
         }
       }
     }
   }
 
+  // the waves' sums, in wave order; wave k takes every KS-th of the values
+  constexpr int F = RW * TM * 4;
+  float* red = reinterpret_cast<float*>(gemm_lds) + lane;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < RW; ++u)
+#pragma unroll
+    for (int t = 0; t < TM; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[(ks * F + (u * TM + t) * 4 + r) * 64] = acc[u][t][r];
+  __syncthreads();
+  for (int f = ks; f < F; f += KS) {
+    float v = red[f * 64];
+#pragma unroll
+    for (int k = 1; k < KS; ++k) v += red[(k * F + f) * 64];
+    const int r = f & 3, t = (f >> 2) % TM, u = (f >> 2) / TM;
+    const int tok = tok0 + 16 * t + 4 * kb + r;
+    if (tok < M && l16 < N) out[(size_t)tok * N + tile_row(u) + l16] = (uint16_t)f32_to_bf16(v);
+  }
+}
+
+constexpr size_t split_lds_bytes(int tm, int rw, int ks, int scale_groups) {
+  const size_t x = (size_t)ks * tm * 4096 + (size_t)16 * rw * scale_groups * 2;
+  const size_t red = (size_t)ks * rw * tm * 4 * 256;
+  return x > red ? x : red;
+}
+
+template <int TM, int RW, int KS, int D, bool SCL>
+int launch_split(const int8_t* qw, const uint16_t* sc, const uint16_t* x, uint16_t* out, int M, int N,
+                 int K, hipStream_t s) {
+  static const bool lds_ok =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&int4_gemm_split_kernel<TM, RW, KS, D, SCL>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemmLds) == hipSuccess;
+  if (!lds_ok) return hip_status(hipGetLastError());
+  const int row_blocks = (N + 16 * RW - 1) / (16 * RW);
+  const unsigned grid = (unsigned)row_blocks * (unsigned)((M + 16 * TM - 1) / (16 * TM));
+  hipLaunchKernelGGL((int4_gemm_split_kernel<TM, RW, KS, D, SCL>), dim3(grid), dim3(KS * 64),
+                     split_lds_bytes(TM, RW, KS, SCL ? K / kGroupSize : 0), s, qw, sc, x, out, M, N, K,
+                     row_blocks);
+  return hip_status(hipGetLastError());
+}
+
+// Row tiles per workgroup: the count that leaves the busiest CU the least to
+// do, with 0.6 of a row tile as a workgroup's own share (its x tile).
+int split_row_tiles(int n, int token_blocks) {
+  const long long tiles = (n + 15) / 16;
+  const int cus = device_cus();
+  int best = 1;
+  long long cost = 0;
+  for (int rw = 1; rw <= 4; ++rw) {
+    const long long wgs = (tiles + rw - 1) / rw * token_blocks;
+    const long long c = (wgs + cus - 1) / cus * (10 * rw + 6);
+    if (rw == 1 || c <= cost) {
+      best = rw;
+      cost = c;
+    }
+  }
+  return best;
+}
+
+// Scale runs are staged by dwords, so they start at even values.
+bool scales_by_dword(const uint16_t* sc, int N, int K) {
+  return (reinterpret_cast<uintptr_t>(sc) & 3u) == 0 && (K / kGroupSize % 2 == 0 || N % 2 == 0);
+}
+
+template <int TM>
+int launch_split_tokens(const int8_t* qw, const uint16_t* sc, const uint16_t* x, uint16_t* out, int M,
+                        int N, int K, hipStream_t s) {
+  const int blocks = (M + 16 * TM - 1) / (16 * TM);
+  const int rw = split_row_tiles(N, blocks);
+  // at most one workgroup per CU: twice the waves, on half as many groups each
+  const bool few = (long long)(((N + 15) / 16 + rw - 1) / rw) * blocks <= device_cus();
+  if (!scales_by_dword(sc, N, K) ||
+      split_lds_bytes(TM, rw, few ? 8 : 4, K / kGroupSize) > kGemmLds / (few ? 1 : 2))
+    return launch_split<TM, 2, 4, 1, false>(qw, sc, x, out, M, N, K, s);
+#define DIP_SPLIT(R)                                                                    \
+  if (rw == (R))                                                                        \
+    return few ? launch_split<TM, R, 8, 2, true>(qw, sc, x, out, M, N, K, s)            \
+               : launch_split<TM, R, 4, 2, true>(qw, sc, x, out, M, N, K, s);
+  DIP_SPLIT(1) DIP_SPLIT(2) DIP_SPLIT(3) DIP_SPLIT(4)
+#undef DIP_SPLIT
+  return DIP_ERR_UNSUPPORTED;
+}
+
+// ---------------------------------------------------------------------------
+// Enough tokens and rows to fill the chip: 64 RW weight rows and 64 tokens per
+// workgroup, 4 waves side by side with RW tiles of 16 rows each, times KS parts
+// of K (part ks takes groups ks, ks + KS, ...) whose sums are added through LDS
+// at the end, in a fixed order.  Per group (one step, one barrier):
+//   * a part's 4 waves stage its x tile in LDS, P steps ahead in registers, as
+//     above, and each token's -24 * sum(x) beside it;
+//   * a wave has its rows' nibbles in flight P steps ahead and turns each into
+//     an operand once for all 64 tokens;
+//   * per 32-column slice, 4 operands from LDS feed 4 RW independent MFMAs.
+// Bound by instruction issue (RW 4: 64 MFMAs and 283 other vector instructions
+// a step, half of them the nibbles) and below about 500 workgroups by a step's
+// latency: 25600 x 5120, 64 tokens 68 -> 35 us, 100 tokens 57 us (dequantize
+// and the library's product: 119), 333 tokens 132 us (159), 512 tokens 180 us
+// (191); 2048 tokens 639 us, 840 TFLOP/s (540).  The token blocks of a row block run on one XCD, whose
+// L2 then reads the rows once.
+// ---------------------------------------------------------------------------
+// x pairs of 8 values, and their sum.
+DIP_DEV uint4 pair8(const uint4& v, float& sum) {
+  uint32_t p[4];
+  make_xpairs(v.x, v.y, v.z, v.w, p);
+  sum = dot2_bf16(v.x, 0x3F803F80u, 0.f);
+  sum = dot2_bf16(v.y, 0x3F803F80u, sum);
+  sum = dot2_bf16(v.z, 0x3F803F80u, sum);
+  sum = dot2_bf16(v.w, 0x3F803F80u, sum);
+  return make_uint4(p[0], p[1], p[2], p[3]);
+}
+
+constexpr int kTileTokens = 64;
+
+template <int RW, int KS>
+__global__ __launch_bounds__(KS * 256, 2) void int4_gemm_kernel(
+    const int8_t* __restrict__ qw, const uint16_t* __restrict__ sc, const uint16_t* __restrict__ x,
+    uint16_t* __restrict__ out, int M, int N, int K, int row_blocks, int token_blocks) {
+  extern __shared__ __align__(16) uint4 gemm_lds[];
+  constexpr int TM = kTileTokens / 16;
+  constexpr int P = RW == 4 ? 1 : 2;
+  constexpr int XT = TM * 256;  // 16-byte chunks of an x tile
+  const int bi = blockIdx.x / kXcds;
+  const int rb = blockIdx.x % kXcds + kXcds * (bi / token_blocks);
+  if (rb >= row_blocks) return;
+  const int tok0 = (bi % token_blocks) * kTileTokens;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int ks = wave >> 2, wr = wave & 3;
+  const int kb = lane >> 4, l16 = lane & 15;
+  // row tiles at the end of the matrix overlap, as in the kernel above
+  const int row0 = max(0, min(rb * (64 * RW), N - 16));
+  auto tile_row = [&](int u) { return max(0, min(row0 + 16 * (RW * wr + u), N - 16)); };
+  const int lrow = min(l16, N - 1);
+  const int ngroups = K >> 7;
+  const int steps = (ngroups + KS - 1) / KS;
+  uint4* xt = gemm_lds + ks * 2 * XT;  // two buffers
+  float* xs = reinterpret_cast<float*>(gemm_lds + KS * 2 * XT) + ks * 2 * kTileTokens;
+  uint32_t* ssc = reinterpret_cast<uint32_t*>(gemm_lds + KS * 2 * (XT + kTileTokens / 4));
+
+  const int xtok = (threadIdx.x & 255) >> 4;  // the thread's token of every 16
+  const char* xbase = reinterpret_cast<const char*>(x + (size_t)tok0 * K);
+  uint32_t xoff[TM];
+#pragma unroll
+  for (int e = 0; e < TM; ++e)
+    xoff[e] = (uint32_t)min(16 * e + xtok, M - 1 - tok0) * (uint32_t)(2 * K) + (uint32_t)(16 * l16);
+  const uint32_t woff = (uint32_t)lrow * (uint32_t)(K >> 1) + 16u * kb;
+  uint4 xr[P][TM], w[P][RW];
+  auto group = [&](int i) { return min(ks + i * KS, ngroups - 1); };  // past the end: the last again
+  auto load_x = [&](int p, int i) {
+    const char* b = xbase + (size_t)group(i) * 256;
+#pragma unroll
+    for (int e = 0; e < TM; ++e) xr[p][e] = *reinterpret_cast<const uint4*>(b + xoff[e]);
+  };
+  auto stage_x = [&](int p, int buf) {
+#pragma unroll
+    for (int e = 0; e < TM; ++e) {
+      const int t = 16 * e + xtok;
+      float sum;
+      xt[buf * XT + t * 16 + (l16 ^ (t & 15))] = pair8(xr[p][e], sum);
+      sum = group_sum<16>(sum);
+      if (l16 == 0) xs[buf * kTileTokens + t] = -24.0f * sum;
+    }
+  };
+  auto load_w = [&](int p, int u, int i) {
+    const int8_t* q = qw + (size_t)tile_row(u) * (K >> 1) + (size_t)group(i) * 64;
+    w[p][u] = *reinterpret_cast<const uint4*>(q + woff);
+  };
+  load_x(0, 0);
+#pragma unroll
+  for (int p = 0; p < P; ++p)
+#pragma unroll
+    for (int u = 0; u < RW; ++u) load_w(p, u, p);
+  {
+    const int n_sc = min(64 * RW, N - row0) * ngroups;  // this workgroup's scales
+    const uint16_t* src = sc + (size_t)row0 * ngroups;
+    for (int e0 = threadIdx.x; 2 * e0 < n_sc; e0 += 8 * KS * 256) {
+      uint32_t r[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {  // an odd count's last value is loaded alone: it may end the matrix
+        const int e = 2 * (e0 + i * KS * 256);
+        r[i] = e + 1 < n_sc ? *reinterpret_cast<const uint32_t*>(src + e) : e < n_sc ? src[e] : 0u;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (2 * (e0 + i * KS * 256) < n_sc) ssc[e0 + i * KS * 256] = r[i];
+    }
+  }
+  stage_x(0, 0);
+#pragma unroll
+  for (int p = 0; p < P; ++p) load_x((p + 1) % P, p + 1);
+  __syncthreads();
+
+  floatx4 acc[RW][TM];
+#pragma unroll
+  for (int u = 0; u < RW; ++u)
+#pragma unroll
+    for (int t = 0; t < TM; ++t) acc[u][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  // two steps per turn: the register slots and the buffers are constants
+  for (int i0 = 0; i0 < steps; i0 += 2) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int i = i0 + e;
+      if (i < steps) {
+        const int p = e % P;
+        // the next step's x into the other buffer, which every wave has left
+        stage_x((e + 1) % P, e ^ 1);
+        load_x((e + 1) % P, i + 1 + P);
+        if (ks + i * KS < ngroups) {
+          float sf[RW];
+#pragma unroll
+          for (int u = 0; u < RW; ++u)
+            sf[u] = bf16_to_f32(reinterpret_cast<const uint16_t*>(
+                ssc)[(tile_row(u) - row0 + lrow) * ngroups + ks + i * KS]);
+          floatx4 v[RW][TM];
+#pragma unroll
+          for (int t = 0; t < TM; ++t) {
+            const floatx4 c = *reinterpret_cast<const floatx4*>(&xs[e * kTileTokens + 16 * t + 4 * kb]);
+#pragma unroll
+            for (int u = 0; u < RW; ++u) v[u][t] = c;
+          }
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            bf16x8_t xa[TM], b[RW];
+#pragma unroll
+            for (int t = 0; t < TM; ++t)
+              xa[t] = as_bf16x8(xt[e * XT + (16 * t + l16) * 16 + ((4 * kb + j) ^ l16)]);
+#pragma unroll
+            for (int u = 0; u < RW; ++u)
+              b[u] = weights24(j == 0 ? w[p][u].x : j == 1 ? w[p][u].y : j == 2 ? w[p][u].z : w[p][u].w);
+#pragma unroll
+            for (int u = 0; u < RW; ++u)
+#pragma unroll
+              for (int t = 0; t < TM; ++t)
+                v[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[t], b[u], v[u][t], 0, 0, 0);
+          }
+#pragma unroll
+          for (int u = 0; u < RW; ++u) load_w(p, u, i + P);
+#pragma unroll
+          for (int u = 0; u < RW; ++u)
+#pragma unroll
+            for (int t = 0; t < TM; ++t)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[u][t][r] = fmaf(sf[u], v[u][t][r], acc[u][t][r]);
+        }
+        __syncthreads();
+      }
+    }
+  }
+
+  // the K parts' sums, in order, on part 0
   if constexpr (KS > 1) {
-#pragma unroll
-    for (int u = 0; u < RW; ++u)
-#pragma unroll
-      for (int t = 0; t < TM; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) red[wave][u][t][r][lane] = acc[u][t][r];
-    __syncthreads();
-    if (ks != 0) return;
-#pragma unroll
-    for (int w = 1; w < KS; ++w)
+    constexpr int F = RW * TM * 4;
+    float* red = reinterpret_cast<float*>(gemm_lds) + lane;
+    if (ks > 0) {
 #pragma unroll
       for (int u = 0; u < RW; ++u)
 #pragma unroll
         for (int t = 0; t < TM; ++t)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[u][t][r] += red[wave + w][u][t][r][lane];
+          for (int r = 0; r < 4; ++r)
+            red[((wave - 4) * F + (u * TM + t) * 4 + r) * 64] = acc[u][t][r];
+    }
+    __syncthreads();
+    if (ks > 0) return;
+#pragma unroll
+    for (int k = 1; k < KS; ++k)
+#pragma unroll
+      for (int u = 0; u < RW; ++u)
+#pragma unroll
+        for (int t = 0; t < TM; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            acc[u][t][r] += red[((4 * (k - 1) + wr) * F + (u * TM + t) * 4 + r) * 64];
   }
 #pragma unroll
-  for (int t = 0; t < TM; ++t) {
-    const int tok = tok0 + t * 16 + l16;
-    if (tok >= M) continue;
+  for (int t = 0; t < TM; ++t)
 #pragma unroll
-    for (int u = 0; u < RW; ++u)
+    for (int r = 0; r < 4; ++r) {
+      const int tok = tok0 + 16 * t + 4 * kb + r;
+      if (tok < M && l16 < N) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = row0 + 16 * u + 4 * kb + r;
-        if (row < N) out[(size_t)tok * N + row] = (uint16_t)f32_to_bf16(acc[u][t][r]);
+        for (int u = 0; u < RW; ++u)
+          out[(size_t)tok * N + tile_row(u) + l16] = (uint16_t)f32_to_bf16(acc[u][t][r]);
       }
-  }
+    }
 }
 
-template <int TM, int PW, int RW>
-void launch_gemm(const int8_t* qw, const uint16_t* sc, const uint16_t* x, uint16_t* out, int M,
-                 int N, int K, hipStream_t s) {
-  // 16 * RW rows per wave; 16 * RW * RT rows per workgroup: as many rows as
-  // keep at least two workgroups per CU, the rest of the 4 waves splitting K
-  const int cus = device_cus();
-  const unsigned gy = (unsigned)((M + 16 * TM - 1) / (16 * TM));
-  const long long tile = 16LL * RW;
-  if ((long long)N >= tile * 4 * 2 * cus)
-    hipLaunchKernelGGL((int4_gemm_kernel<TM, 4, PW, RW>), dim3((N + tile * 4 - 1) / (tile * 4), gy),
-                       dim3(kGemmThreads), 0, s, qw, sc, x, out, M, N, K);
-  else if ((long long)N >= tile * 2 * 2 * cus)
-    hipLaunchKernelGGL((int4_gemm_kernel<TM, 2, PW, RW>), dim3((N + tile * 2 - 1) / (tile * 2), gy),
-                       dim3(kGemmThreads), 0, s, qw, sc, x, out, M, N, K);
-  else
-    hipLaunchKernelGGL((int4_gemm_kernel<TM, 1, PW, RW>), dim3((N + tile - 1) / tile, gy),
-                       dim3(kGemmThreads), 0, s, qw, sc, x, out, M, N, K);
+constexpr size_t gemm_lds_bytes(int rw, int ks, int ngroups) {
+  const size_t x = (size_t)ks * 2 * kTileTokens * (256 + 4) + (size_t)64 * rw * ngroups * 2;
+  const size_t red = (size_t)(ks - 1) * 4 * rw * kTileTokens * 64;
+  return x > red ? x : red;
 }
 
-// The token tiling for M tokens, RW row tiles per wave; the weight prefetch
-// depth shrinks as RW grows so the wave stays within 256 VGPRs.
-template <int RW>
-void launch_tokens(const int8_t* qw, const uint16_t* sc, const uint16_t* x, uint16_t* out, int M,
-                   int N, int K, hipStream_t s) {
-  constexpr int kPW8 = 8 / RW >= 2 ? 8 / RW : 2, kPW4 = 4 / RW >= 2 ? 4 / RW : 2;
-  if (M <= 16)
-    launch_gemm<1, kPW8, RW>(qw, sc, x, out, M, N, K, s);
-  else if (M <= 32)
-    launch_gemm<2, kPW8, RW>(qw, sc, x, out, M, N, K, s);
-  else
-    launch_gemm<4, kPW4, RW>(qw, sc, x, out, M, N, K, s);
+template <int RW, int KS>
+int launch_gemm(const int8_t* qw, const uint16_t* sc, const uint16_t* x, uint16_t* out, int M, int N,
+                int K, hipStream_t s) {
+  static const bool lds_ok =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&int4_gemm_kernel<RW, KS>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemmLds) == hipSuccess;
+  if (!lds_ok) return hip_status(hipGetLastError());
+  const int rbs = (N + 64 * RW - 1) / (64 * RW), tbs = (M + kTileTokens - 1) / kTileTokens;
+  const unsigned grid = (unsigned)((rbs + kXcds - 1) / kXcds * kXcds) * (unsigned)tbs;
+  hipLaunchKernelGGL((int4_gemm_kernel<RW, KS>), dim3(grid), dim3(KS * 256),
+                     gemm_lds_bytes(RW, KS, K / kGroupSize), s, qw, sc, x, out, M, N, K, rbs, tbs);
+  return hip_status(hipGetLastError());
+}
+
+// The kernel for a product (us measured on both sides of each line): up to 32
+// tokens the split kernel.  Beyond, the tiled one once 128-row blocks give 160
+// workgroups (12288 x 4096: 96 workgroups 28 against 19 split, 192 28 against
+// 32): with two K parts, 8 waves a workgroup, while every CU gets at most one
+// (25600 x 5120, 64 tokens, 200 workgroups: 35, with one part 41), else with one
+// (100 tokens, 400 workgroups: 57, with two parts 63; 5120 x 8192, 400 tokens,
+// 280 workgroups: two parts 93), and with four row tiles per wave from 1024
+// workgroups of them (25600 x 5120: 333 tokens, 600 of them, 151 against 138
+// with two; 2048 tokens, 3200 of them, 639 against 718).
+int launch_int4_gemm(const int8_t* qw, const uint16_t* sc, const uint16_t* x, uint16_t* out, int M,
+                     int N, int K, hipStream_t s) {
+  if (M <= 16) return launch_split_tokens<1>(qw, sc, x, out, M, N, K, s);
+  const long long tbs = (M + kTileTokens - 1) / kTileTokens;
+  const long long wgs2 = (N + 127) / 128 * tbs, wgs4 = (N + 255) / 256 * tbs;
+  const int cus = device_cus(), ngroups = K / kGroupSize;
+  if (M <= 32 || 8 * wgs2 < 5 * cus || !scales_by_dword(sc, N, K) ||
+      gemm_lds_bytes(2, 2, ngroups) > kGemmLds)
+    return launch_split_tokens<2>(qw, sc, x, out, M, N, K, s);
+  if (wgs4 >= 4 * cus && gemm_lds_bytes(4, 1, ngroups) <= kGemmLds / 2)
+    return launch_gemm<4, 1>(qw, sc, x, out, M, N, K, s);
+  if (wgs2 > cus) return launch_gemm<2, 1>(qw, sc, x, out, M, N, K, s);
+  return launch_gemm<2, 2>(qw, sc, x, out, M, N, K, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -267,6 +567,7 @@ void launch_tokens(const int8_t* qw, const uint16_t* sc, const uint16_t* x, uint
 //   * wave w reads A = 16 columns x 8 consecutive k (one 16-byte LDS read
 //     per slice) and B = x[token][k .. k + 7] straight from L2, and
 //     accumulates on v_mfma_f32_16x16x32_bf16.
+constexpr int kGemmThreads = 256;
 constexpr int kGemmTStep = 128;     // K rows per step
 constexpr int kGemmTStride = 128 + 8;  // LDS row of one column: 128 k + 16 B of padding
 constexpr int kGemmTPrefetch = 4;
@@ -456,11 +757,7 @@ extern "C" int dip_int4_gemm(const int8_t* qweight, const uint16_t* scales, cons
   if (!aligned16(qweight) || !aligned16(x)) return DIP_ERR_ALIGN;
   const int M = (int)m, N = (int)out_features, K = (int)in_features;
   hipStream_t s = (hipStream_t)stream;
-  if (N >= 8192)
-    launch_tokens<4>(qweight, scales, x, out, M, N, K, s);
-  else
-    launch_tokens<2>(qweight, scales, x, out, M, N, K, s);
-  return hip_status(hipGetLastError());
+  return launch_int4_gemm(qweight, scales, x, out, M, N, K, s);
 }
 
 namespace {

@@ -34,8 +34,27 @@ _QUANT_SUBSTRINGS = ("q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_pr
 _GEMV_COLS = frozenset((128, 256, 512, 1024, 1536, 2048, 2560, 3072, 4096, 5120, 6144, 8192))
 # Prompts of up to this many tokens run the int4 MFMA GEMM (weights read
 # once as nibbles); longer ones dequantize once and use the library GEMM,
-# which wins once the bf16 copy is amortised over enough tokens.
-GEMM_MAX_TOKENS = 64
+# which wins once the bf16 copy is amortised over enough tokens (us, int4
+# GEMM against both steps of the library route: 25600 x 5120, 512 tokens 180
+# / 191, 700 tokens 228 / 237, 1024 tokens 313 / 300; 12288 x 4096, 512 tokens
+# 69 / 77, 700 tokens 104 / 95).
+GEMM_MAX_TOKENS = 512
+# Up to this many rows it takes any input, rounded to bf16; beyond, plain bf16
+# tensors only (_plain_bf16).
+_ANY_INPUT_TOKENS = 64
+# The transposed GEMM's limit.
+GEMM_T_MAX_TOKENS = 64
+
+
+def _plain_bf16(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether x is a plain bf16 tensor beside `weight` that nothing
+    differentiates, batches or traces: what a kernel called on its data may
+    take in place of torch ops."""
+    return (type(x) is torch.Tensor and x.dtype == torch.bfloat16 and x.device == weight.device
+            and not (x.requires_grad and torch.is_grad_enabled())
+            and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+            and torch.autograd.forward_ad._current_level < 0
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
 
 
 def int4_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor) -> torch.Tensor:
@@ -48,7 +67,8 @@ def int4_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor) ->
     if rows == 1 and in_f in _GEMV_COLS:
         y = K.int4_gemv(qweight, scales, x.reshape(-1).to(torch.bfloat16))
         return y.to(x.dtype).reshape(*x.shape[:-1], qweight.shape[0])
-    if 1 < rows <= GEMM_MAX_TOKENS:
+    if 1 < rows <= _ANY_INPUT_TOKENS or (1 < rows <= GEMM_MAX_TOKENS and x.shape[-1] == in_f
+                                         and _plain_bf16(x, qweight)):
         y = K.int4_gemm(qweight, scales, x.reshape(rows, in_f).to(torch.bfloat16))
         return y.to(x.dtype).reshape(*x.shape[:-1], qweight.shape[0])
     return F.linear(x, dequantize(qweight, scales).to(x.dtype))
@@ -57,11 +77,11 @@ def int4_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor) ->
 def int4_linear_t(x: torch.Tensor, qweight_t: torch.Tensor, scales_t: torch.Tensor) -> torch.Tensor:
     """x @ bf16(q*s) for a matrix stored as rows of the input dimension (the
     transposed down matrix) on the device, in x's dtype: the int4 MFMA GEMM
-    for up to GEMM_MAX_TOKENS rows of x, else x @ dequantize (the reference's
+    for up to GEMM_T_MAX_TOKENS rows of x, else x @ dequantize (the reference's
     route, dip_stream_predispatch.py:213-215)."""
     import _dip_hip as K
     rows = x.numel() // x.shape[-1]
-    if rows <= GEMM_MAX_TOKENS:
+    if rows <= GEMM_T_MAX_TOKENS:
         return K.int4_gemm_t(qweight_t, scales_t, x.to(torch.bfloat16)).to(x.dtype)
     return x @ dequantize(qweight_t, scales_t).to(x.dtype)
 
