@@ -261,7 +261,9 @@ def int4_gemm_t(qweight_t, scales_t, x, out=None):
           or out.device != dev):
         raise RuntimeError(f"out must be a contiguous bf16 tensor of {m} x {n} values")
     nbytes = lib.dip_int4_gemm_t_workspace_size(m, n, k_rows)
-    ws = workspace(dev, nbytes, "gemm_t") if nbytes else None
+    # scratch that nothing has to clear: the caching allocator's, so calls on
+    # several streams or in a captured graph each have their own
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
     _check(lib.dip_int4_gemm_t(_ptr(qweight_t), _ptr(scales_t), _ptr(x2), _ptr(out), m, n, k_rows,
                                _ptr(ws), 0 if ws is None else ws.numel(), _stream(dev)),
            "dip_int4_gemm_t")

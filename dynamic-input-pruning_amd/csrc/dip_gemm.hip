@@ -554,189 +554,288 @@ int launch_int4_gemm(const int8_t* qw, const uint16_t* sc, const uint16_t* x, ui
 // down matrix down_t of the dense route's h @ down_t
 // (dip_stream_predispatch.py:213-215).  The scale varies along k here, so
 // each weight becomes the reference's bf16(q * s) (qlinear.dequantize's
-// rounding, exact to it) on its way into LDS:
-//   * a workgroup owns 64 output columns x 16 * TM tokens and a K range
-//     (the K ranges of a split are added by int4_gemm_t_reduce_kernel, in
-//     a fixed order);
-//   * per 128-row step the 256 threads read 128 rows x 32 bytes of nibbles
-//     (thread t: rows 2 (t / 4) and 2 (t / 4) + 1, 16 columns) and their
-//     scales, and write the dequantised values transposed into LDS
-//     [column][k], one 32-bit word (the two rows) per column: each pair is
-//     one v_cvt_pk_bf16_f32 (double-buffered, one barrier per step);
-//     nibbles and scales run kGemmTPrefetch steps ahead in registers;
-//   * wave w reads A = 16 columns x 8 consecutive k (one 16-byte LDS read
-//     per slice) and B = x[token][k .. k + 7] straight from L2, and
-//     accumulates on v_mfma_f32_16x16x32_bf16.
-constexpr int kGemmThreads = 256;
-constexpr int kGemmTStep = 128;     // K rows per step
-constexpr int kGemmTStride = 128 + 8;  // LDS row of one column: 128 k + 16 B of padding
-constexpr int kGemmTPrefetch = 4;
+// rounding, exact to it) in registers:
+//   * a wave owns 128 columns (one scale group), lane l16 the 8 columns 8 l16 ..:
+//     a dword of each row.  An MFMA slice is 32 rows; the lane quarter kb loads
+//     rows 8 kb .. + 7 (64 contiguous bytes of each row), and column c of the
+//     16 lanes' 8 is one 16-column operand whose k pairs are two rows' values
+//     rounded by one v_cvt_pk_bf16_f32: the transposition costs nothing;
+//   * q * s: a nibble in the low mantissa bits of an fp16 1024.0 is 1032 + q (or
+//     1152 + 16 q, four bits higher), read as fp16 by v_fma_mix_f32, which
+//     multiplies by s and takes 1032 s (72 s) away with one rounding of an
+//     exactly representable result: 17 instructions per 8 weights.  Scales of
+//     2^118 or more, infinite or NaN, take plain products instead;
+//   * x comes from memory as operands, 64 contiguous bytes of each token, so
+//     nothing is staged and the loop has no barrier;
+//   * a row's four factors are read from LDS, 256 rows of them prepared at a
+//     time by the wave itself.
+// A workgroup is 2 such column blocks (whole 128-byte lines) times 4 parts of
+// K, added through LDS; blockIdx.z splits K further, its fp32 partials added in
+// a fixed order by int4_gemm_t_reduce_kernel.  Bound by instruction issue (136
+// vector instructions to 8 TM MFMAs a slice).  25600 x 5120: 2 tokens 63 -> 32
+// us, 32 tokens 112 -> 39 us, 64 tokens 201 -> 49 us (before: values transposed
+// through LDS a barrier at a time, 64 columns a workgroup), 333 tokens 143 us
+// (dequantize and the library's product: 234), 1024 tokens 418 us (401).
+// ---------------------------------------------------------------------------
+constexpr int kGemmTThreads = 512;
+constexpr int kGemmTCols = 256;  // columns of a workgroup
+constexpr int kGemmTParts = 4;   // K parts of a workgroup
+constexpr int kChunkSlices = 8;  // slices per round of prepared factors
+
+// fp16 half H of v times a plus c, in fp32.
+template <int H>
+DIP_DEV float fma_mix(uint32_t v, float a, float c) {
+  float r;
+  if (H == 0)
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,0,0] op_sel_hi:[1,0,0]"
+        : "=v"(r) : "v"(v), "v"(a), "v"(c));
+  else
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+        : "=v"(r) : "v"(v), "v"(a), "v"(c));
+  return r;
+}
+
+// The 8 columns' q * s of one row; f = (s, s / 16, -1032 s, -72 s).
+template <bool PLAIN>
+DIP_DEV void row_values(uint32_t w, const float4& f, float v[8]) {
+  if constexpr (PLAIN) {
+#pragma unroll
+    for (int p = 0; p < 8; ++p) v[p] = (float)(int)__builtin_amdgcn_sbfe(w, 4 * p, 4) * f.x;
+    return;
+  }
+  const uint32_t t = w >> 8;
+  const uint32_t a = (w & 0x000F000Fu) ^ 0x64086408u, b = (w & 0x00F000F0u) ^ 0x64806480u;
+  const uint32_t c = (t & 0x000F000Fu) ^ 0x64086408u, d = (t & 0x00F000F0u) ^ 0x64806480u;
+  v[0] = fma_mix<0>(a, f.x, f.z);
+  v[4] = fma_mix<1>(a, f.x, f.z);
+  v[1] = fma_mix<0>(b, f.y, f.w);
+  v[5] = fma_mix<1>(b, f.y, f.w);
+  v[2] = fma_mix<0>(c, f.x, f.z);
+  v[6] = fma_mix<1>(c, f.x, f.z);
+  v[3] = fma_mix<0>(d, f.y, f.w);
+  v[7] = fma_mix<1>(d, f.y, f.w);
+}
+
+// A lane's 8 rows x 8 columns as 8 operands.
+template <bool PLAIN>
+DIP_DEV void slice_operands(const uint32_t w[8], const float4* f, bf16x8_t b[8]) {
+  uint32_t r[8][4];
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) {
+    float v0[8], v1[8];
+    row_values<PLAIN>(w[i], f[i], v0);
+    row_values<PLAIN>(w[i + 1], f[i + 1], v1);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) r[c][i / 2] = f32x2_to_bf16x2_nan(v0[c], v1[c]);
+  }
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+    b[c] = __builtin_bit_cast(bf16x8_t, u32x4_t{r[c][0], r[c][1], r[c][2], r[c][3]});
+}
 
 template <int TM>
-__global__ __launch_bounds__(kGemmThreads) void int4_gemm_t_kernel(
+__global__ __launch_bounds__(kGemmTThreads, 2) void int4_gemm_t_kernel(
     const int8_t* __restrict__ qw, const uint16_t* __restrict__ sc, const uint16_t* __restrict__ x,
-    uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int K, int kchunk) {
-  __shared__ __align__(16) uint16_t wt[2][64][kGemmTStride];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int K, int part_slices) {
+  constexpr int D = TM == 4 ? 2 : 4;  // slices of weights in flight
+  constexpr int DX = 2;               // slices of x in flight
+  constexpr int F = 8 * TM * 4;       // sums of a lane
+  extern __shared__ __align__(16) float4 gemmt_lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int kb = lane >> 4, l16 = lane & 15;
-  const int n0 = blockIdx.x * 64;
-  const int tok0 = blockIdx.y * TM * 16;
-  const int k0 = blockIdx.z * kchunk;
-  const int k1 = min(K, k0 + kchunk);
-  const int nsteps = (k1 - k0 + kGemmTStep - 1) / kGemmTStep;
+  const int col0 = blockIdx.x * kGemmTCols + (wave & 1) * 128;
+  const int kp = wave >> 1;
+  const int tok0 = blockIdx.y * (16 * TM);
+  const int slices = (K + 31) / 32;
+  const int s0 = min(((int)blockIdx.z * kGemmTParts + kp) * part_slices, slices);
+  const int s1 = col0 < N ? min(s0 + part_slices, slices) : s0;
+  const size_t row_bytes = (size_t)(N >> 1);
   const int ngroups_n = N >> 7;
+  float4* fac = gemmt_lds + wave * (32 * kChunkSlices);
 
-  // staging role: rows sr, sr + 1 of the step, columns n0 + scol .. + 15
-  const int sr = 2 * (threadIdx.x >> 2), scol = 16 * (threadIdx.x & 3);
-  const bool col_ok = n0 + scol < N;
-  struct WPair {
-    uint2 w0, w1;   // 16 nibbles of each row
-    uint32_t s01;   // the two rows' scales (row sr low)
-  };
-  auto load_w = [&](int step, WPair& wp) {
-    const int row = k0 + step * kGemmTStep + sr;
-    const size_t off = (size_t)((n0 + scol) >> 1);
-    const int g = (n0 + scol) >> 7;
-    wp.w0 = make_uint2(0, 0);
-    wp.w1 = make_uint2(0, 0);
-    wp.s01 = 0u;
-    if (row < k1 && col_ok) {
-      wp.w0 = *reinterpret_cast<const uint2*>(qw + (size_t)row * (N >> 1) + off);
-      wp.s01 = sc[(size_t)row * ngroups_n + g];
-    }
-    if (row + 1 < k1 && col_ok) {
-      wp.w1 = *reinterpret_cast<const uint2*>(qw + (size_t)(row + 1) * (N >> 1) + off);
-      wp.s01 |= (uint32_t)sc[(size_t)(row + 1) * ngroups_n + g] << 16;
-    }
-  };
-  // bf16(q * s) of both rows for each of the 16 columns, as one word per
-  // column: the signed nibble is one bit-field extract, and the pair of
-  // roundings one f32x2_to_bf16x2 (f32_to_bf16's bits, NaN included).
-  auto stage = [&](int buf, const WPair& wp) {
-    const float s0 = bf16_to_f32(wp.s01 & 0xFFFFu), s1 = bf16_to_f32(wp.s01 >> 16);
-    const uint32_t a4[2] = {wp.w0.x, wp.w0.y}, b4[2] = {wp.w1.x, wp.w1.y};
-    // word k/2 of column c sits at (k/2) ^ (16 * ((c / 16) & 3)): the four
-    // 16-column groups written by one instruction land in different banks
-    uint32_t* dst = reinterpret_cast<uint32_t*>(&wt[buf][scol][0]) + ((sr >> 1) ^ (scol & 48));
-    constexpr int kColWords = kGemmTStride / 2;
+  // K is a multiple of 8, so a lane's 8 rows are all inside or all past the end
+  const int tail8 = K - 32 * (slices - 1);  // rows of the last slice
+  const bool in_tail = 8 * kb < tail8;
+  const uint32_t off_full = 8u * kb * (uint32_t)row_bytes + 4u * l16;
+  const uint32_t off_tail = (in_tail ? 8u * kb : 0u) * (uint32_t)row_bytes + 4u * l16;
+  const int8_t* wbase = qw + (col0 >> 1);
+  const char* xp[TM];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+  for (int t = 0; t < TM; ++t)
+    xp[t] = reinterpret_cast<const char*>(x + (size_t)min(tok0 + 16 * t + l16, M - 1) * K + 8 * kb);
+  uint32_t w[D][8], sreg[4];
+  uint4 xr[DX][TM];
+  auto load_w = [&](int d, int s) {
+    const int8_t* b = wbase + (size_t)s * 32 * row_bytes;
+    const uint32_t o = s == slices - 1 ? off_tail : off_full;
 #pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        const float va = (float)(int)__builtin_amdgcn_sbfe(a4[i], 4 * b, 4) * s0;
-        const float vb = (float)(int)__builtin_amdgcn_sbfe(b4[i], 4 * b, 4) * s1;
-        dst[(8 * i + b) * kColWords] = f32x2_to_bf16x2(va, vb);
-      }
+    for (int i = 0; i < 8; ++i) w[d][i] = *reinterpret_cast<const uint32_t*>(b + i * row_bytes + o);
+  };
+  auto load_x = [&](int d, int s) {
+    const bool in = s < slices - 1 || in_tail;
+#pragma unroll
+    for (int t = 0; t < TM; ++t) {
+      xr[d][t] = make_uint4(0, 0, 0, 0);
+      if (in) xr[d][t] = *reinterpret_cast<const uint4*>(xp[t] + (size_t)s * 64);
     }
   };
-  // B operand: token l16 of each tile, k .. k + 7 at column quarter kb
-  const uint16_t* xrow[TM];
+  auto load_s = [&](int s) {  // the factors' scales of rows 32 s .. + 255
 #pragma unroll
-  for (int t = 0; t < TM; ++t) xrow[t] = x + (size_t)min(tok0 + t * 16 + l16, M - 1) * K;
+    for (int e = 0; e < 4; ++e) {
+      const int row = min(32 * s + 64 * e + lane, K - 1);
+      sreg[e] = sc[(size_t)row * ngroups_n + (col0 >> 7)];
+    }
+  };
+  floatx4 acc[8][TM];
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+#pragma unroll
+    for (int t = 0; t < TM; ++t) acc[c][t] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  // x operands of one step: slice j, token tile t (zeros past the K range)
-  auto load_x = [&](int step, uint4 (&dst)[kGemmTStep / 32][TM]) {
+  if (s0 < s1) {
+    load_s(s0);
 #pragma unroll
-    for (int j = 0; j < kGemmTStep / 32; ++j) {
-      const int kk = k0 + step * kGemmTStep + 32 * j + 8 * kb;
+    for (int d = 0; d < DX; ++d) load_x(d, min(s0 + d, s1 - 1));
 #pragma unroll
-      for (int t = 0; t < TM; ++t)
-        dst[j][t] = (step < nsteps && kk < k1) ? *reinterpret_cast<const uint4*>(xrow[t] + kk)
-                                               : make_uint4(0, 0, 0, 0);
-    }
-  };
-  // x one step ahead in registers for up to 32 tokens; the 64-token tiling
-  // loads it in place (the extra registers would cost it occupancy)
-  constexpr bool kXAhead = TM <= 2;
-  [[maybe_unused]] uint4 xc[kGemmTStep / 32][TM];
-  if constexpr (kXAhead) load_x(0, xc);
-
-  WPair wq[kGemmTPrefetch];
-#pragma unroll
-  for (int p = 0; p < kGemmTPrefetch; ++p) {
-    if (p < nsteps) load_w(p, wq[p]);
+    for (int d = 0; d < D; ++d) load_w(d, min(s0 + d, s1 - 1));
   }
-  floatx4 acc[TM];
+  for (int sb = s0; sb < s1; sb += kChunkSlices) {
+    bool plain = false;
 #pragma unroll
-  for (int t = 0; t < TM; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-  if (nsteps > 0) stage(0, wq[0]);
-  if (kGemmTPrefetch < nsteps) load_w(kGemmTPrefetch, wq[0]);
-  __syncthreads();
-
-  for (int i0 = 0; i0 < nsteps; i0 += kGemmTPrefetch) {
+    for (int e = 0; e < 4; ++e) {
+      const int row = 32 * sb + 64 * e + lane;
+      const float f = row < K ? bf16_to_f32(sreg[e]) : 0.f;  // rows past the end weigh nothing
+      plain |= row < K && (sreg[e] & 0x7FFFu) >= 0x7A80u;
+      fac[64 * e + lane] = make_float4(f, f * 0.0625f, f * -1032.0f, f * -72.0f);
+    }
+    plain = __any(plain);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    load_s(min(sb + kChunkSlices, slices - 1));
+    for (int q0 = 0; q0 < kChunkSlices; q0 += D) {
 #pragma unroll
-    for (int p = 0; p < kGemmTPrefetch; ++p) {
-      const int i = i0 + p;
-      if (i < nsteps) {
-        const int buf = i & 1;
-        // stage step i + 1 into the other buffer while this one is read
-        if (i + 1 < nsteps) {
-          const int pn = (p + 1) % kGemmTPrefetch;
-          stage(buf ^ 1, wq[pn]);
-          if (i + 1 + kGemmTPrefetch < nsteps) load_w(i + 1 + kGemmTPrefetch, wq[pn]);
-        }
-        if constexpr (kXAhead) {
-          // the next step's x operands, in flight while this step multiplies
-          uint4 xn[kGemmTStep / 32][TM];
-          load_x(i + 1, xn);
+      for (int d = 0; d < D; ++d) {
+        const int s = sb + q0 + d;
+        if (s < s1) {
+          bf16x8_t b[8];
+          const float4* fr = fac + 32 * (q0 + d) + 8 * kb;
+          if (plain) slice_operands<true>(w[d], fr, b);
+          else slice_operands<false>(w[d], fr, b);
+          load_w(d, min(s + D, s1 - 1));
+          bf16x8_t xa[TM];
 #pragma unroll
-          for (int j = 0; j < kGemmTStep / 32; ++j) {
-            const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(
-                &wt[buf][16 * wave + l16][(32 * j + 8 * kb) ^ (32 * (wave & 3))]);
+          for (int t = 0; t < TM; ++t) xa[t] = as_bf16x8(xr[d % DX][t]);
+#pragma unroll
+          for (int c = 0; c < 8; ++c)
 #pragma unroll
             for (int t = 0; t < TM; ++t)
-              acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, as_bf16x8(xc[j][t]), acc[t], 0,
-                                                               0, 0);
-          }
-#pragma unroll
-          for (int j = 0; j < kGemmTStep / 32; ++j)
-#pragma unroll
-            for (int t = 0; t < TM; ++t) xc[j][t] = xn[j][t];
-        } else {
-          const int kbase = k0 + i * kGemmTStep;
-#pragma unroll
-          for (int j = 0; j < kGemmTStep / 32; ++j) {
-            const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(
-                &wt[buf][16 * wave + l16][(32 * j + 8 * kb) ^ (32 * (wave & 3))]);
-            const int kk = kbase + 32 * j + 8 * kb;
-#pragma unroll
-            for (int t = 0; t < TM; ++t) {
-              uint4 bv = make_uint4(0, 0, 0, 0);
-              if (kk < k1) bv = *reinterpret_cast<const uint4*>(xrow[t] + kk);
-              acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, as_bf16x8(bv), acc[t], 0, 0, 0);
-            }
-          }
+              acc[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[t], b[c], acc[c][t], 0, 0, 0);
+          load_x(d % DX, min(s + DX, s1 - 1));
         }
-        __syncthreads();
       }
     }
+    // this round's reads of the factors before the next round's writes
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
 
+  // (part 0 + part 2) + (part 1 + part 3)
+  float* red = reinterpret_cast<float*>(gemmt_lds);
 #pragma unroll
-  for (int t = 0; t < TM; ++t) {
-    const int tok = tok0 + t * 16 + l16;
-    if (tok >= M) continue;
+  for (int h = kGemmTParts / 2; h >= 1; h /= 2) {
+    __syncthreads();
+    if (kp >= h && kp < 2 * h) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+#pragma unroll
+        for (int t = 0; t < TM; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            red[((wave - 2 * h) * F + (c * TM + t) * 4 + r) * 64 + lane] = acc[c][t][r];
+    }
+    __syncthreads();
+    if (kp < h) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+#pragma unroll
+        for (int t = 0; t < TM; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            acc[c][t][r] += red[(wave * F + (c * TM + t) * 4 + r) * 64 + lane];
+    }
+  }
+  if (kp > 0 || col0 >= N) return;
+  const bool wide = (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
+#pragma unroll
+  for (int t = 0; t < TM; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int col = n0 + 16 * wave + 4 * kb + r;
-      if (col >= N) continue;
-      if (part)
-        part[((size_t)blockIdx.z * M + tok) * N + col] = acc[t][r];
-      else
-        out[(size_t)tok * N + col] = (uint16_t)f32_to_bf16(acc[t][r]);
+      const int tok = tok0 + 16 * t + 4 * kb + r;
+      if (tok >= M) continue;
+      if (part) {
+        float4* o = reinterpret_cast<float4*>(part + ((size_t)blockIdx.z * M + tok) * N + col0 + 8 * l16);
+        o[0] = make_float4(acc[0][t][r], acc[1][t][r], acc[2][t][r], acc[3][t][r]);
+        o[1] = make_float4(acc[4][t][r], acc[5][t][r], acc[6][t][r], acc[7][t][r]);
+      } else {
+        uint16_t* o = out + (size_t)tok * N + col0 + 8 * l16;
+        uint32_t v[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = f32x2_to_bf16x2(acc[2 * c][t][r], acc[2 * c + 1][t][r]);
+        if (wide) {
+          *reinterpret_cast<uint4*>(o) = make_uint4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+          for (int c = 0; c < 8; ++c) o[c] = (uint16_t)(v[c / 2] >> (16 * (c & 1)));
+        }
+      }
+    }
+}
+
+constexpr size_t gemm_t_lds_bytes(int tm) {
+  const size_t red = (size_t)4 * 8 * tm * 4 * 256, fac = (size_t)8 * 32 * kChunkSlices * 16;
+  return red > fac ? red : fac;
+}
+
+// Sum of the K split's fp32 partials in split order, rounded to bf16: four
+// values a thread (M * N is a multiple of 128).
+__global__ __launch_bounds__(256) void int4_gemm_t_reduce_kernel(const float* __restrict__ part,
+                                                                 uint16_t* __restrict__ out,
+                                                                 size_t mn, int splits) {
+  const bool wide = (reinterpret_cast<uintptr_t>(out) & 7u) == 0;
+  for (size_t e = 4 * ((size_t)blockIdx.x * 256 + threadIdx.x); e < mn; e += 4 * (size_t)gridDim.x * 256) {
+    float4 v = *reinterpret_cast<const float4*>(part + e);
+#pragma unroll 4
+    for (int z = 1; z < splits; ++z) {
+      const float4 p = *reinterpret_cast<const float4*>(part + (size_t)z * mn + e);
+      v.x += p.x;
+      v.y += p.y;
+      v.z += p.z;
+      v.w += p.w;
+    }
+    const uint32_t lo = f32x2_to_bf16x2(v.x, v.y), hi = f32x2_to_bf16x2(v.z, v.w);
+    if (wide) {
+      *reinterpret_cast<uint2*>(out + e) = make_uint2(lo, hi);
+    } else {
+      out[e] = (uint16_t)lo;
+      out[e + 1] = (uint16_t)(lo >> 16);
+      out[e + 2] = (uint16_t)hi;
+      out[e + 3] = (uint16_t)(hi >> 16);
     }
   }
 }
 
-// Sum of the K split's fp32 partials in split order, rounded to bf16.
-__global__ __launch_bounds__(256) void int4_gemm_t_reduce_kernel(const float* __restrict__ part,
-                                                                 uint16_t* __restrict__ out,
-                                                                 size_t mn, int splits) {
-  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < mn; e += (size_t)gridDim.x * 256) {
-    float v = 0.f;
-    for (int z = 0; z < splits; ++z) v += part[(size_t)z * mn + e];
-    out[e] = (uint16_t)f32_to_bf16(v);
-  }
+template <int TM>
+int launch_gemm_t(const int8_t* qw, const uint16_t* sc, const uint16_t* x, uint16_t* out, float* part,
+                  int M, int N, int K, int splits, int part_slices, hipStream_t s) {
+  static const bool lds_ok =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&int4_gemm_t_kernel<TM>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemmLds) == hipSuccess;
+  if (!lds_ok) return hip_status(hipGetLastError());
+  const dim3 grid((unsigned)((N + kGemmTCols - 1) / kGemmTCols), (unsigned)((M + 16 * TM - 1) / (16 * TM)),
+                  (unsigned)splits);
+  hipLaunchKernelGGL(int4_gemm_t_kernel<TM>, grid, dim3(kGemmTThreads), gemm_t_lds_bytes(TM), s, qw, sc,
+                     x, out, part, M, N, K, part_slices);
+  return hip_status(hipGetLastError());
 }
 
 }  // namespace
@@ -761,14 +860,22 @@ extern "C" int dip_int4_gemm(const int8_t* qweight, const uint16_t* scales, cons
 }
 
 namespace {
-// K split of dip_int4_gemm_t: about two workgroups per CU over the
-// (64-column, 16*TM-token) tiles, at most 16 ranges, whole 128-row steps.
+int gemm_t_token_tiles(int64_t m) { return m <= 16 ? 1 : (m <= 32 ? 2 : 4); }
+
+// K split of dip_int4_gemm_t over blockIdx.z: as many as give every CU one
+// workgroup (8 waves fill it; us for 25600 x 5120: 64 tokens, 20 workgroups a
+// split, 12 splits 49, 10: 53, 16: 72; 200 tokens 3 splits 103, 4: 146; 333
+// tokens 2 splits 143, 3: 188).  Where one round of workgroups would leave a
+// third of the chip idle and two rounds would not, two (512 tokens, 160
+// workgroups: one split 279, three 210).
 int gemm_t_splits(int64_t m, int64_t n, int64_t k) {
-  const int64_t tm = m <= 16 ? 1 : (m <= 32 ? 2 : 4);
-  const int64_t tiles = ((n + 63) / 64) * ((m + 16 * tm - 1) / (16 * tm));
-  const int64_t want = (2LL * device_cus() + tiles - 1) / tiles;
-  const int64_t max_split = (k + kGemmTStep - 1) / kGemmTStep;
-  return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, 16), max_split));
+  const int64_t tm = gemm_t_token_tiles(m);
+  const int64_t tiles = ((n + kGemmTCols - 1) / kGemmTCols) * ((m + 16 * tm - 1) / (16 * tm));
+  const int64_t most = std::min<int64_t>(16, (k + 32 * kGemmTParts - 1) / (32 * kGemmTParts));
+  const int64_t cus = device_cus(), two = 2 * cus / tiles;
+  int64_t z = std::max<int64_t>(1, cus / tiles);
+  if (3 * z * tiles < 2 * cus && 20 * two * tiles >= 17 * 2 * cus) z = two;
+  return (int)std::max<int64_t>(1, std::min(z, most));
 }
 }  // namespace
 
@@ -792,30 +899,23 @@ extern "C" int dip_int4_gemm_t(const int8_t* qweight_t, const uint16_t* scales_t
   if (!x || !out) return DIP_ERR_NULL;
   if (!aligned16(qweight_t) || !aligned16(x)) return DIP_ERR_ALIGN;
   const int M = (int)m, N = (int)out_features, K = (int)in_features;
-  const int TM = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
-  const int gy = (M + 16 * TM - 1) / (16 * TM);
-  const int gx = (N + 63) / 64;
   int splits = gemm_t_splits(m, out_features, in_features);
   const size_t need = splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
   if (need > 0 && (!workspace || ws_bytes < need)) return DIP_ERR_WORKSPACE;
   if (splits > 1 && !aligned16(workspace)) return DIP_ERR_ALIGN;
-  const int kchunk = ((K + splits - 1) / splits + kGemmTStep - 1) / kGemmTStep * kGemmTStep;
-  splits = (K + kchunk - 1) / kchunk;
+  const int slices = (K + 31) / 32;
+  const int part_slices = (slices + splits * kGemmTParts - 1) / (splits * kGemmTParts);
   float* part = splits > 1 ? static_cast<float*>(workspace) : nullptr;
   hipStream_t s = (hipStream_t)stream;
-  const dim3 grid(gx, gy, splits);
-  if (TM == 1)
-    hipLaunchKernelGGL(int4_gemm_t_kernel<1>, grid, dim3(kGemmThreads), 0, s, qweight_t, scales_t,
-                       x, out, part, M, N, K, kchunk);
-  else if (TM == 2)
-    hipLaunchKernelGGL(int4_gemm_t_kernel<2>, grid, dim3(kGemmThreads), 0, s, qweight_t, scales_t,
-                       x, out, part, M, N, K, kchunk);
-  else
-    hipLaunchKernelGGL(int4_gemm_t_kernel<4>, grid, dim3(kGemmThreads), 0, s, qweight_t, scales_t,
-                       x, out, part, M, N, K, kchunk);
+  const int tm = gemm_t_token_tiles(m);
+  const int st =
+      tm == 1 ? launch_gemm_t<1>(qweight_t, scales_t, x, out, part, M, N, K, splits, part_slices, s)
+      : tm == 2 ? launch_gemm_t<2>(qweight_t, scales_t, x, out, part, M, N, K, splits, part_slices, s)
+                : launch_gemm_t<4>(qweight_t, scales_t, x, out, part, M, N, K, splits, part_slices, s);
+  if (st) return st;
   if (splits > 1) {
     const size_t mn = (size_t)M * N;
-    const unsigned blocks = (unsigned)std::min<size_t>((mn + 255) / 256, 2048);
+    const unsigned blocks = (unsigned)std::min<size_t>((mn / 4 + 255) / 256, 4096);
     hipLaunchKernelGGL(int4_gemm_t_reduce_kernel, dim3(blocks), dim3(256), 0, s, part, out, mn,
                        splits);
   }

@@ -42,8 +42,10 @@ GEMM_MAX_TOKENS = 512
 # Up to this many rows it takes any input, rounded to bf16; beyond, plain bf16
 # tensors only (_plain_bf16).
 _ANY_INPUT_TOKENS = 64
-# The transposed GEMM's limit.
-GEMM_T_MAX_TOKENS = 64
+# The transposed GEMM's limit (us, against dequantize and the library's
+# product: 25600 x 5120, 512 tokens 210 / 338, 1024 tokens 418 / 401; 12288 x
+# 4096, 512 tokens 85 / 128, 1024 tokens 147 / 148).
+GEMM_T_MAX_TOKENS = 768
 
 
 def _plain_bf16(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -81,7 +83,7 @@ def int4_linear_t(x: torch.Tensor, qweight_t: torch.Tensor, scales_t: torch.Tens
     route, dip_stream_predispatch.py:213-215)."""
     import _dip_hip as K
     rows = x.numel() // x.shape[-1]
-    if rows <= GEMM_T_MAX_TOKENS:
+    if rows <= _ANY_INPUT_TOKENS or (rows <= GEMM_T_MAX_TOKENS and _plain_bf16(x, qweight_t)):
         return K.int4_gemm_t(qweight_t, scales_t, x.to(torch.bfloat16)).to(x.dtype)
     return x @ dequantize(qweight_t, scales_t).to(x.dtype)
 
