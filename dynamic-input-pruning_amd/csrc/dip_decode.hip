@@ -397,8 +397,8 @@ __global__ __launch_bounds__(4 * kHeadDim) void attn_combine_kernel(
 }
 
 // Norm + rotary + cache write + attention in one launch, for caches of at
-// most kFusedMaxLen rows (4 waves up to 128 rows, 16 beyond, which walk the
-// 32-row chunks 16 at a time): workgroup = HPW consecutive query heads of one kv
+// most kFusedMaxLen rows (4 waves up to 128 rows, 8 beyond, which walk the
+// 32-row chunks 8 at a time): workgroup = HPW consecutive query heads of one kv
 // head (group = nh / nkv query heads share it).  Every workgroup of a group
 // normalises and rotates the group's k itself; only the group's first
 // workgroup writes k and v to cache row pos (the others take this token's
@@ -414,12 +414,17 @@ __global__ __launch_bounds__(4 * kHeadDim) void attn_combine_kernel(
 //      (v_mfma_f32_16x16x32_bf16, A = 16 cache rows, B = the q heads, exact
 //      products, fp32 sums; row pos from LDS, not read back), softmax in
 //      fp32, the value sum in fp32 on the VALU, merged into a running (max,
-//      sum, value sum) per query head;
+//      sum, value sum) per query head.  Keys and values come by 128-bit loads
+//      that cover 64 (256) contiguous bytes of a row, the next chunk's while
+//      this one is worked on;
 //   3. the NW waves' partials are merged through LDS in a fixed order.
-// One launch wins over the split path up to about 900 cache rows (64 query /
-// 8 kv heads: 11.9 against 15.6 us at 512 rows, 18.3 against 17.3 at 1024);
-// beyond, each query head's workgroup re-reading its kv head's rows costs
-// more than the split path's extra launches.
+// Bound by what one CU can fetch (each query head's workgroup reads its kv
+// head's rows).  64 / 8 heads, us in a graph: 121 rows of 128 7.1 -> 5.5, 101
+// rows of 1024 7.3 -> 5.5, 501 rows 11.8 -> 10.0, 701 rows 15.3 -> 11.9, 1021
+// rows 18.5 -> 14.7 (before: 16 waves without room for a chunk ahead, 16-byte
+// pieces of 64 lines per key load, 4-byte value loads; two chunks ahead on 8
+// waves 13.2 at 701 rows, 12 waves 12.5).  The split path takes 14.1 at 501 and
+// 14.5 at 1021 rows, so one launch serves caches of up to 1024 rows.
 constexpr int kFusedMaxLen = 1024;
 
 template <int HPW, int NW>
@@ -442,12 +447,14 @@ __global__ __launch_bounds__(NW * 64) void attn_fused_kernel(
   __shared__ float ps[NW][HPW][kAttnChunk];
   __shared__ float cm[NW][HPW], cl[NW][HPW];
   __shared__ float wm[NW][HPW], wl[NW][HPW];
-  __shared__ float wacc[NW][HPW][kHeadDim];
-  const int kvh = h0 / group, wave = threadIdx.x >> 6, l = threadIdx.x & 63;
+  __shared__ __align__(16) float wacc[NW][HPW][kHeadDim];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kvh = h0 / group, l = threadIdx.x & 63;
   const int l16 = l & 15, kb = l >> 4;
   const int64_t pos = *pos_p;
   const bool pos_ok = pos >= 0 && pos < max_len;
-  const int64_t last = pos < (int64_t)max_len ? pos : (int64_t)max_len - 1;
+  const int last = attn_rows(pos, max_len) - 1;  // the last attended row
+  const int own = pos_ok ? (int)pos : -1;        // this token's row
 
   // 0. loads
   for (int i = threadIdx.x; i < (HPW + 2) * 64; i += kThreads) {
@@ -465,29 +472,34 @@ __global__ __launch_bounds__(NW * 64) void attn_fused_kernel(
     tabs[wave][l] = *src;
   }
   int start = wave * kAttnChunk;
-  uint4 ka[2][4];       // A operand: cache rows start + 16t + l16, dims 32 kb .. 32 kb + 31
-  uint32_t vv[kAttnChunk];  // values: rows start + j, dims 2l, 2l + 1
-  auto load_chunk = [&](int st) {
+  const char* kbase = reinterpret_cast<const char*>(k_cache + (size_t)kvh * max_len * kHeadDim);
+  const char* vbase = reinterpret_cast<const char*>(v_cache + (size_t)kvh * max_len * kHeadDim);
+  uint4 ka[2][4];  // A operand: cache rows st + 16 t + l16, slice j: dims 32 j + 8 kb .. + 7
+  uint4 vv[8];     // values: rows st + 4 i + kb, dims 8 l16 .. + 7
+  auto load_k = [&](int st) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int row = st + 16 * t + l16;
-      if ((int64_t)row <= last) {
-        const uint4* src = reinterpret_cast<const uint4*>(
-            k_cache + ((size_t)kvh * max_len + row) * kHeadDim + 32 * kb);
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) ka[t][j] = src[j];
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) ka[t][j] = make_uint4(0, 0, 0, 0);
+      for (int j = 0; j < 4; ++j) {
+        const int row = st + 16 * t + l16;
+        ka[t][j] = make_uint4(0, 0, 0, 0);
+        if (row <= last)
+          ka[t][j] = *reinterpret_cast<const uint4*>(kbase + (uint32_t)(row * 256 + 64 * j + 16 * kb));
       }
-    }
-    const int np = (int)((last - st + 1) < kAttnChunk ? (last - st + 1) : kAttnChunk);
-    const uint32_t* vcol =
-        reinterpret_cast<const uint32_t*>(v_cache + ((size_t)kvh * max_len + st) * kHeadDim) + l;
-#pragma unroll
-    for (int j = 0; j < kAttnChunk; ++j) vv[j] = j < np ? vcol[(size_t)j * 64] : 0u;
   };
-  if ((int64_t)start <= last) load_chunk(start);
+  auto load_v = [&](int st) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int row = st + 4 * i + kb;
+      vv[i] = make_uint4(0, 0, 0, 0);
+      if (row <= last)
+        vv[i] = *reinterpret_cast<const uint4*>(vbase + (uint32_t)(row * 256 + 16 * l16));
+    }
+  };
+  if (start <= last) {
+    load_k(start);
+    load_v(start);
+  }
   __syncthreads();
 
   // 1. RMSNorm + rotary of the q heads and the k head; v and k to the cache
@@ -527,28 +539,30 @@ __global__ __launch_bounds__(NW * 64) void attn_fused_kernel(
   }
   __syncthreads();
 
-  // 2. B operand (q head l16, dims 32 kb .. 32 kb + 31) once; then the chunks
+  // 2. B operand (q head l16, the same dims per slice) once; then the chunks
   uint4 bq[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) bq[j] = *reinterpret_cast<const uint4*>(&qb[l16][16 * kb + 4 * j]);
-  float m[HPW], lsum[HPW], a0[HPW], a1[HPW];
+  for (int j = 0; j < 4; ++j) bq[j] = *reinterpret_cast<const uint4*>(&qb[l16][16 * j + 4 * kb]);
+  float m[HPW], lsum[HPW], acc[HPW][8];
 #pragma unroll
   for (int g = 0; g < HPW; ++g) {
     m[g] = -INFINITY;
-    lsum[g] = a0[g] = a1[g] = 0.f;
+    lsum[g] = 0.f;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) acc[g][d] = 0.f;
   }
-  for (; (int64_t)start <= last; start += NW * kAttnChunk) {
-    const int npos = (int)((last - start + 1) < kAttnChunk ? (last - start + 1) : kAttnChunk);
+  for (; start <= last; start += NW * kAttnChunk) {
+    const int npos = min(last - start + 1, kAttnChunk);
+    const int next = start + NW * kAttnChunk;
+    const bool more = next <= last;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      if ((int64_t)(start + 16 * t + l16) == pos) {  // this token's row from LDS
+      if (start + 16 * t + l16 == own) {  // this token's row from LDS
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          ka[t][j] = *reinterpret_cast<const uint4*>(&kv_new[0][16 * kb + 4 * j]);
+          ka[t][j] = *reinterpret_cast<const uint4*>(&kv_new[0][16 * j + 4 * kb]);
       }
     }
-    if ((int64_t)start <= pos && pos < (int64_t)start + npos) vv[pos - start] = kv_new[1][l];
-
     // scores: lane (head l16, rows 4 kb + r of tile t)
     float sc[2][4];
 #pragma unroll
@@ -564,6 +578,9 @@ __global__ __launch_bounds__(NW * 64) void attn_fused_kernel(
         sc[t][r] = ok ? d[r] * scale : -INFINITY;
       }
     }
+    // the next chunk's keys while this one's softmax and values run, and its
+    // values behind them
+    if (more) load_k(next);
     float mx = -INFINITY;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -587,33 +604,39 @@ __global__ __launch_bounds__(NW * 64) void attn_fused_kernel(
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
 
-    // values: lane l takes dimensions 2l, 2l + 1
-    float c0[HPW], c1[HPW];
+    // values: lane dims 8 l16 .. + 7 of every fourth row
+    float c[HPW][8];
 #pragma unroll
-    for (int g = 0; g < HPW; ++g) c0[g] = c1[g] = 0.f;
+    for (int g = 0; g < HPW; ++g)
 #pragma unroll
-    for (int j = 0; j < kAttnChunk; ++j) {
-      if (j < npos) {
-        const float v0 = bf16_to_f32(vv[j] & 0xFFFFu), v1 = bf16_to_f32(vv[j] >> 16);
+      for (int d = 0; d < 8; ++d) c[g][d] = 0.f;
 #pragma unroll
-        for (int g = 0; g < HPW; ++g) {
-          c0[g] = fmaf(ps[wave][g][j], v0, c0[g]);
-          c1[g] = fmaf(ps[wave][g][j], v1, c1[g]);
+    for (int i = 0; i < 8; ++i) {
+      if (start + 4 * i + kb == own)  // this token's row from LDS
+        vv[i] = *reinterpret_cast<const uint4*>(&kv_new[1][4 * l16]);
+      const uint32_t vw[4] = {vv[i].x, vv[i].y, vv[i].z, vv[i].w};
+#pragma unroll
+      for (int g = 0; g < HPW; ++g) {
+        const float pg = ps[wave][g][4 * i + kb];  // 0 for rows past the end
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          c[g][2 * e] = fmaf(pg, bf16_to_f32(vw[e] & 0xFFFFu), c[g][2 * e]);
+          c[g][2 * e + 1] = fmaf(pg, __uint_as_float(vw[e] & 0xFFFF0000u), c[g][2 * e + 1]);
         }
       }
     }
+    if (more) load_v(next);
 #pragma unroll
     for (int g = 0; g < HPW; ++g) {
       const float mc = cm[wave][g], lc = cl[wave][g];
       const float mn = fmaxf(m[g], mc);
       const float fo = expf(m[g] - mn), fn = expf(mc - mn);
       lsum[g] = lsum[g] * fo + lc * fn;
-      a0[g] = a0[g] * fo + c0[g] * fn;
-      a1[g] = a1[g] * fo + c1[g] * fn;
+#pragma unroll
+      for (int d = 0; d < 8; ++d) acc[g][d] = acc[g][d] * fo + c[g][d] * fn;
       m[g] = mn;
     }
     __builtin_amdgcn_wave_barrier();
-    if ((int64_t)(start + NW * kAttnChunk) <= last) load_chunk(start + NW * kAttnChunk);
   }
 
   // 3. merge the waves in a fixed order
@@ -623,8 +646,13 @@ __global__ __launch_bounds__(NW * 64) void attn_fused_kernel(
       wm[wave][g] = m[g];
       wl[wave][g] = lsum[g];
     }
-    wacc[wave][g][2 * l] = a0[g];
-    wacc[wave][g][2 * l + 1] = a1[g];
+#pragma unroll
+    for (int d = 0; d < 8; ++d) acc[g][d] = row_pair_sum32(row_pair_sum16(acc[g][d]));
+    if (kb == 0) {
+      float4* o = reinterpret_cast<float4*>(&wacc[wave][g][8 * l16]);
+      o[0] = make_float4(acc[g][0], acc[g][1], acc[g][2], acc[g][3]);
+      o[1] = make_float4(acc[g][4], acc[g][5], acc[g][6], acc[g][7]);
+    }
   }
   __syncthreads();
   for (int g = wave; g < HPW; g += NW) {
@@ -718,14 +746,14 @@ extern "C" int dip_decode_attention_fused(const uint16_t* qkv, const uint16_t* q
     return DIP_ERR_ALIGN;
   const int nh = (int)n_heads, nkv = (int)n_kv_heads, ml = (int)max_len;
   hipStream_t s = (hipStream_t)stream;
-  // one query head per workgroup; 16 waves (chunks 16 at a time) for caches
-  // of more than 128 rows
+  // one query head per workgroup; 8 waves (chunks 8 at a time) for caches of
+  // more than 128 rows
   if (ml <= 128)
     hipLaunchKernelGGL((attn_fused_kernel<1, 4>), dim3(nh), dim3(256), 0, s, qkv, q_norm_w,
                        k_norm_w, cos_table, sin_table, pos, k_cache, v_cache, out, nh, nkv, ml,
                        eps, scale);
   else
-    hipLaunchKernelGGL((attn_fused_kernel<1, 16>), dim3(nh), dim3(1024), 0, s, qkv, q_norm_w,
+    hipLaunchKernelGGL((attn_fused_kernel<1, 8>), dim3(nh), dim3(512), 0, s, qkv, q_norm_w,
                        k_norm_w, cos_table, sin_table, pos, k_cache, v_cache, out, nh, nkv, ml,
                        eps, scale);
   return hip_status(hipGetLastError());
