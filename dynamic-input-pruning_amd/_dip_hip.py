@@ -72,6 +72,7 @@ _SIGS = {
     "dip_host_gather_rows": ([_p, _p, _p, _i64, _i64, _i64, _i32], _i32),
     "dip_host_gather_rows_multi": ([_p, _p, _p, _i64, _p, _i64, _i64, _i32], _i32),
     "dip_host_stream_rows": ([_p, _p, _p, _p, _i64, _p, _i64, _i64, _i64, _i32, _p, _p], _i32),
+    "dip_stream_rows": ([_p, _p, _p, _i64, _p, _p, _i64, _i64, _p], _i32),
     "dip_int4_gemm": ([_p, _p, _p, _p, _i64, _i64, _i64, _p], _i32),
     "dip_int4_gemm_t_workspace_size": ([_i64, _i64, _i64], _sz),
     "dip_int4_gemm_t": ([_p, _p, _p, _p, _i64, _i64, _i64, _p, _sz, _p], _i32),
@@ -901,6 +902,38 @@ def host_gather_rows_multi(srcs, ids: torch.Tensor, dsts, threads: int = 8) -> N
     _check(lib.dip_host_gather_rows_multi(ctypes.addressof(src_arr), ctypes.addressof(dst_arr),
                                           ctypes.addressof(rb_arr), len(rbs), _ptr(ids), n, rows,
                                           int(threads)), "dip_host_gather_rows_multi")
+
+
+def stream_rows(srcs, ids: torch.Tensor, count: torch.Tensor, dsts) -> bool:
+    """dsts[p][i] = srcs[p][ids[i]] for i < count[0], read by the device from
+    the pinned host matrices srcs (ids and count: int32 on the device), queued
+    on the current stream.  False, with nothing queued, where a source is not
+    pinned."""
+    dev = _dev(*dsts, ids, count)
+    if ids.dtype != torch.int32 or count.dtype != torch.int32 or not ids.is_contiguous():
+        raise RuntimeError("ids and count must be contiguous int32 tensors")
+    rows, rbs = srcs[0].shape[0], []
+    max_rows = ids.numel()
+    if len(dsts) != len(srcs):
+        raise RuntimeError("need one device destination per source")
+    for s, d in zip(srcs, dsts):
+        if s.device.type != "cpu" or not s.is_contiguous() or not d.is_contiguous():
+            raise RuntimeError("stream_rows copies contiguous host rows to contiguous device rows")
+        rb = s.stride(0) * s.element_size()
+        if s.shape[0] != rows or d.stride(0) * d.element_size() != rb:
+            raise RuntimeError("row count or row size mismatch")
+        if d.shape[0] < max_rows:
+            raise RuntimeError("device destination too small")
+        rbs.append(rb)
+    src_arr, dst_arr = _ptr_array(srcs), _ptr_array(dsts)
+    rb_arr = (ctypes.c_int64 * len(rbs))(*rbs)
+    st = lib.dip_stream_rows(ctypes.addressof(src_arr), ctypes.addressof(dst_arr),
+                             ctypes.addressof(rb_arr), len(rbs), _ptr(ids), _ptr(count), max_rows,
+                             rows, _stream(dev))
+    if st == -4:  # DIP_ERR_UNSUPPORTED
+        return False
+    _check(st, "dip_stream_rows")
+    return True
 
 
 def host_stream_rows(srcs, ids: torch.Tensor, pinned, dsts, chunk_rows: int = 2048,

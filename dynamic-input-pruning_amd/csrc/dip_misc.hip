@@ -1,4 +1,4 @@
-// dip_misc.hip — cache-aware hit/miss assembly, row dequantisation, the
+// dip_misc.hip — cache-aware hit/miss assembly and miss stream, row dequantisation, the
 // host-side miss gather, the one-call resident MLP decode step and the
 // library's status helpers.
 #include <algorithm>
@@ -18,21 +18,30 @@
 namespace dip {
 
 // ---------------------------------------------------------------------------
-// Cache-aware assembly (dip_ca.py:137-171).  One workgroup: each thread owns a
-// contiguous segment of idx, counts its hits, a block scan gives every
-// element its place in [hits in idx order, misses in idx order].
+// Cache-aware assembly (dip_ca.py:137-171).  One workgroup, whose time is its
+// chains of dependent loads (idx, then the slot): each wave owns a contiguous
+// run of idx, 64 channels a step and kAsmUnroll steps in flight, counts its
+// hits by ballots, and a scan over the waves gives every element its place in
+// [hits in idx order, misses in idx order].  7373 channels: 20.9 us with a run
+// of single loads per thread, 8.4 us so.
 // ---------------------------------------------------------------------------
 namespace {
 constexpr int kAsmThreads = 1024;
 constexpr int kAsmWaves = kAsmThreads / 64;
+constexpr int kAsmUnroll = 8;
 
-DIP_DEV uint32_t wave_prefix32(uint32_t v, int lane) {
+// The channels at j0 + 64 u of a wave's run [.., end) and their slots, -1
+// where not resident.
+DIP_DEV void asm_load(const int64_t* id2slot, const int32_t* idx, int inter, uint32_t j0,
+                      uint32_t end, int c[kAsmUnroll], int slot[kAsmUnroll]) {
 #pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    uint32_t t = __shfl_up(v, d, 64);
-    if (lane >= d) v += t;
+  for (int u = 0; u < kAsmUnroll; ++u) {
+    const uint32_t j = j0 + 64 * u;
+    c[u] = j < end ? idx[j] : -1;
   }
-  return v;
+#pragma unroll
+  for (int u = 0; u < kAsmUnroll; ++u)
+    slot[u] = (unsigned)c[u] < (unsigned)inter ? (int)max(id2slot[c[u]], (int64_t)-1) : -1;
 }
 }  // namespace
 
@@ -40,54 +49,134 @@ __global__ __launch_bounds__(kAsmThreads) void ca_assemble_kernel(
     const int64_t* __restrict__ id2slot, const int32_t* __restrict__ idx, int inter, int k,
     int32_t* __restrict__ combined, int32_t* __restrict__ src, int32_t* __restrict__ row,
     int32_t* __restrict__ miss_ids, int32_t* __restrict__ counts) {
-  __shared__ uint32_t wave_excl[kAsmWaves];
-  __shared__ uint32_t total_hits;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int per = (k + kAsmThreads - 1) / kAsmThreads;
-  const int beg = min(k, tid * per);
-  const int end = min(k, beg + per);
+  __shared__ int wave_hits[kAsmWaves];
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  // (unsigned: a step past the last of 2^31 - 1 channels does not wrap)
+  const uint32_t steps = ((uint32_t)k + kAsmThreads - 1) / kAsmThreads;  // 64 channels each
+  const uint32_t beg = min((uint32_t)k, wave * steps * 64);
+  const uint32_t end = min((uint32_t)k, beg + steps * 64);
+  int c[kAsmUnroll], slot[kAsmUnroll];
 
-  uint32_t hits = 0;
-  for (int j = beg; j < end; ++j) {
-    const int c = idx[j];
-    const int64_t s = ((unsigned)c < (unsigned)inter) ? id2slot[c] : -1;
-    hits += s >= 0 ? 1u : 0u;
+  int hits = 0;
+  for (uint32_t s = 0; s < steps; s += kAsmUnroll) {
+    asm_load(id2slot, idx, inter, beg + s * 64 + lane, end, c, slot);
+#pragma unroll
+    for (int u = 0; u < kAsmUnroll; ++u) hits += __popcll(__ballot(slot[u] >= 0));
   }
-  const uint32_t incl = wave_prefix32(hits, lane);
-  if (lane == 63) wave_excl[wave] = incl;
+  if (lane == 0) wave_hits[wave] = hits;
   __syncthreads();
-  if (wave == 0) {
-    const uint32_t v = lane < kAsmWaves ? wave_excl[lane] : 0u;
-    const uint32_t p = wave_prefix32(v, lane);
-    if (lane < kAsmWaves) wave_excl[lane] = p - v;
-    const uint32_t tot = __shfl(p, kAsmWaves - 1, 64);
-    if (lane == 0) total_hits = tot;
+  int n_hit = 0, hit_pos = 0;  // of all waves; of the waves before this one
+#pragma unroll
+  for (int w = 0; w < kAsmWaves; ++w) {
+    const int v = wave_hits[w];
+    n_hit += v;
+    hit_pos += w < wave ? v : 0;
   }
-  __syncthreads();
-  const uint32_t n_hit = total_hits;
-  uint32_t hit_pos = wave_excl[wave] + incl - hits;  // hits before this segment
-  for (int j = beg; j < end; ++j) {
-    const int c = idx[j];
-    const int64_t s = ((unsigned)c < (unsigned)inter) ? id2slot[c] : -1;
-    if (s >= 0) {
-      combined[hit_pos] = c;
-      src[hit_pos] = 0;
-      row[hit_pos] = (int32_t)s;
-      ++hit_pos;
-    } else {
-      const uint32_t miss_rank = (uint32_t)j - hit_pos;  // misses before j
-      const uint32_t pos = n_hit + miss_rank;
-      combined[pos] = c;
-      src[pos] = 1;
-      row[pos] = (int32_t)miss_rank;
-      miss_ids[miss_rank] = c;
+  const uint64_t below = ((uint64_t)1 << lane) - 1;
+  for (uint32_t s = 0; s < steps; s += kAsmUnroll) {
+    const uint32_t j0 = beg + s * 64 + lane;
+    // (a run of one pass is still in the registers)
+    if (steps > kAsmUnroll) asm_load(id2slot, idx, inter, j0, end, c, slot);
+#pragma unroll
+    for (int u = 0; u < kAsmUnroll; ++u) {
+      const uint32_t j = j0 + 64 * u;
+      const uint64_t m = __ballot(slot[u] >= 0);
+      const int before = hit_pos + __popcll(m & below);  // hits before j
+      hit_pos += __popcll(m);
+      if (j >= end) continue;
+      if (slot[u] >= 0) {
+        combined[before] = c[u];
+        src[before] = 0;
+        row[before] = slot[u];
+      } else {
+        const int miss_rank = (int)j - before;
+        combined[n_hit + miss_rank] = c[u];
+        src[n_hit + miss_rank] = 1;
+        row[n_hit + miss_rank] = miss_rank;
+        miss_ids[miss_rank] = c[u];
+      }
     }
   }
-  if (tid == 0) {
-    counts[0] = (int32_t)n_hit;
-    counts[1] = k - (int32_t)n_hit;
+  if (threadIdx.x == 0) {
+    counts[0] = n_hit;
+    counts[1] = k - n_hit;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Miss rows straight from pinned host memory (the index_select and copies of
+// dip_ca.py:146-156 as one kernel).  Bound by the host link: the rows of all
+// pieces are one run of vectors (a channel's up row, up scales, down row and
+// down scales behind each other), dealt to the grid in order, so that
+// neighbouring lanes ask the link for neighbouring bytes, and the device's
+// own count ends the run: the host learns it only afterwards.  5161 rows of
+// 4224 bytes 420 us, 52 GB/s, the rate of a plain copy over the link (64 to
+// 1024 blocks and 1 to 8 vectors a lane are within 4 %).  A layer's whole
+// token, 12288 x 4096, 5161 misses: 765 us with host threads gathering into
+// staging for DMA copies, 500 us so.
+// ---------------------------------------------------------------------------
+constexpr int kStreamPieces = 8;
+constexpr int kStreamBlocks = 256;
+constexpr int kStreamUnroll = 4;
+
+struct StreamArgs {
+  const char* src[kStreamPieces];
+  char* dst[kStreamPieces];
+  uint32_t row_bytes[kStreamPieces];
+  uint32_t end[kStreamPieces];    // vectors of the pieces up to this one, in a row
+  uint32_t shift[kStreamPieces];  // log2 of the piece's vector bytes
+  int npieces;
+  uint32_t per_row;               // vectors of all pieces in a row
+};
+
+__global__ __launch_bounds__(256) void stream_rows_kernel(StreamArgs a,
+                                                          const int32_t* __restrict__ ids,
+                                                          const int32_t* __restrict__ count,
+                                                          uint32_t max_rows, uint32_t src_rows) {
+  const uint32_t n = (uint32_t)min(max(*count, 0), (int)max_rows);
+  const uint32_t total = n * a.per_row;
+  const uint32_t step = gridDim.x * blockDim.x;
+  for (uint32_t e0 = blockIdx.x * blockDim.x + threadIdx.x; e0 < total;
+       e0 += kStreamUnroll * step) {
+    uint4 v[kStreamUnroll];
+    char* to[kStreamUnroll];
+    uint32_t sh[kStreamUnroll];
+#pragma unroll
+    for (int u = 0; u < kStreamUnroll; ++u) {
+      const uint32_t e = e0 + u * step;
+      to[u] = nullptr;
+      v[u] = make_uint4(0, 0, 0, 0);
+      if (e >= total) continue;
+      const uint32_t i = e / a.per_row, o = e - i * a.per_row;
+      int p = 0;
+      while (o >= a.end[p]) ++p;
+      const uint32_t off = (o - (p ? a.end[p - 1] : 0u)) << a.shift[p];
+      const uint32_t id = (uint32_t)ids[i];
+      sh[u] = a.shift[p];
+      to[u] = a.dst[p] + (size_t)i * a.row_bytes[p] + off;
+      // an id past the matrix leaves a row of zeros
+      if (id >= src_rows) continue;
+      const char* from = a.src[p] + (size_t)id * a.row_bytes[p] + off;
+      switch (sh[u]) {
+        case 4: v[u] = *reinterpret_cast<const uint4*>(from); break;
+        case 3: *reinterpret_cast<uint2*>(&v[u]) = *reinterpret_cast<const uint2*>(from); break;
+        case 2: v[u].x = *reinterpret_cast<const uint32_t*>(from); break;
+        case 1: v[u].x = *reinterpret_cast<const uint16_t*>(from); break;
+        default: v[u].x = *reinterpret_cast<const uint8_t*>(from);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kStreamUnroll; ++u) {
+      if (!to[u]) continue;
+      switch (sh[u]) {
+        case 4: *reinterpret_cast<uint4*>(to[u]) = v[u]; break;
+        case 3: *reinterpret_cast<uint2*>(to[u]) = make_uint2(v[u].x, v[u].y); break;
+        case 2: *reinterpret_cast<uint32_t*>(to[u]) = v[u].x; break;
+        case 1: *reinterpret_cast<uint16_t*>(to[u]) = (uint16_t)v[u].x; break;
+        default: *reinterpret_cast<uint8_t*>(to[u]) = (uint8_t)v[u].x;
+      }
+    }
   }
 }
 
@@ -102,7 +191,7 @@ __global__ __launch_bounds__(kAsmThreads) void ca_assemble_kernel(
 // ---------------------------------------------------------------------------
 constexpr int kDqUnroll = 4;
 
-// 8 nibbles of w times the scale s16 / 16 (see dequant8_scale).
+// 8 nibbles of w (each converted as 16 times itself) times the scale s16 / 16.
 DIP_DEV void dequant8(uint32_t w, float s16, float v[8]) {
   const uint32_t lo = (w << 4) & 0xF0F0F0F0u, hi = w & 0xF0F0F0F0u;
   v[0] = cvt_sbyte<0>(lo) * s16;
@@ -304,6 +393,50 @@ extern "C" int dip_ca_assemble(const int64_t* id2slot, const int32_t* idx, int32
   if (k > 0 && (!idx || !combined || !src || !row || !miss_ids)) return DIP_ERR_NULL;
   hipLaunchKernelGGL(ca_assemble_kernel, dim3(1), dim3(kAsmThreads), 0, (hipStream_t)stream,
                      id2slot, idx, (int)inter, (int)k, combined, src, row, miss_ids, counts);
+  return hip_status(hipGetLastError());
+}
+
+extern "C" int dip_stream_rows(const void* const* src, void* const* dst, const int64_t* row_bytes,
+                               int64_t npieces, const int32_t* ids, const int32_t* count,
+                               int64_t max_rows, int64_t src_rows, void* stream) {
+  if (npieces < 0 || npieces > kStreamPieces || max_rows < 0 || src_rows < 0 ||
+      max_rows > INT32_MAX || src_rows > INT32_MAX)
+    return DIP_ERR_SHAPE;
+  if (npieces == 0 || max_rows == 0) return DIP_OK;
+  if (!src || !dst || !row_bytes || !ids || !count) return DIP_ERR_NULL;
+  StreamArgs a{};
+  uint64_t per_row = 0;
+  for (int p = 0; p < (int)npieces; ++p) {
+    if (row_bytes[p] < 0 || row_bytes[p] > INT32_MAX) return DIP_ERR_SHAPE;
+    if (row_bytes[p] == 0) continue;
+    if (!src[p] || !dst[p]) return DIP_ERR_NULL;
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, src[p]) != hipSuccess) {
+      (void)hipGetLastError();
+      return DIP_ERR_UNSUPPORTED;
+    }
+    // (only pinned memory has both; a kernel may read no other)
+    if (at.type != hipMemoryTypeHost || !at.devicePointer) return DIP_ERR_UNSUPPORTED;
+    const void* from = at.devicePointer;
+    // the widest vector that rows and both bases allow
+    const uint64_t al = reinterpret_cast<uintptr_t>(from) | reinterpret_cast<uintptr_t>(dst[p]) |
+                        (uint64_t)row_bytes[p] | 16u;
+    const int q = a.npieces++;
+    a.src[q] = static_cast<const char*>(from);
+    a.dst[q] = static_cast<char*>(dst[p]);
+    a.row_bytes[q] = (uint32_t)row_bytes[p];
+    a.shift[q] = (uint32_t)__builtin_ctzll(al);
+    per_row += (uint64_t)row_bytes[p] >> a.shift[q];
+    a.end[q] = (uint32_t)per_row;
+  }
+  if (a.npieces == 0) return DIP_OK;
+  // vector numbers, also those a stride past the last, stay within 32 bits
+  const uint64_t slack = (uint64_t)kStreamUnroll * kStreamBlocks * 256;
+  if (per_row > INT32_MAX || per_row * (uint64_t)max_rows + 2 * slack > UINT32_MAX)
+    return DIP_ERR_SHAPE;
+  a.per_row = (uint32_t)per_row;
+  hipLaunchKernelGGL(stream_rows_kernel, dim3(kStreamBlocks), dim3(256), 0, (hipStream_t)stream, a,
+                     ids, count, (uint32_t)max_rows, (uint32_t)src_rows);
   return hip_status(hipGetLastError());
 }
 

@@ -6,11 +6,16 @@ resident in HBM; each decode token splits its k selected channels into hits
 
     GPU : gate GEMV + SiLU + top-k (bit-exact reference order)
           -> hit/miss assembly through id2slot            (dip_ca_assemble)
-    host: read n_hit/n_miss and the miss ids (the one sync the reference also
-          has, dip_ca.py:139-146); gather the miss rows into pinned staging
-          with native threads
-    GPU : hits' up GEMV + h runs while the misses cross PCIe on a side stream
-          -> misses' up GEMV + h -> dual-source transposed-down gather
+          -> the misses' up and down rows read straight from pinned host
+          memory (dip_stream_rows), as the device's own count says
+          -> up GEMV + h of hits and misses -> dual-source transposed-down
+          gather
+    host: queues all of that at once, then reads n_hit/n_miss back (the sync
+          the reference also has, dip_ca.py:139-146) and waits for the rows
+
+Where a matrix is not in pinned memory (a caller replaced it), the host reads
+the miss ids too and gathers the rows into pinned staging with native threads,
+whose copies run beside the hits' GEMV.
 
 The combined order is [hits in idx order, misses in idx order] with
 src 0 = hit / 1 = miss and row = resident slot / staging row, exactly as the
@@ -77,9 +82,10 @@ class CABuffers:
         # statistics of the last forward (hit rate, bytes streamed)
         self.last_n_hit = 0
         self.last_n_miss = 0
-        # when a list: one (bytes, seconds of the gather-and-queue call, ms
-        # of copy-stream time of its H2D copies) per streamed miss set; the
-        # call then also waits for its copies
+        # when a list: one (bytes, seconds from queueing the stream until its
+        # rows are there, ms of device time of the stream) per streamed miss
+        # set (a host gather: seconds of the gather-and-queue call, ms of its
+        # H2D copies, which the call then waits for)
         self.transfers = None
 
     def g(self, inter: int) -> torch.Tensor:
@@ -156,7 +162,7 @@ class CADIPMlp(nn.Module):
         while the next chunk is gathered."""
         b = self.buf
         pins = (b.pin_up_qw, b.pin_up_sc, b.pin_dn_qw, b.pin_dn_sc)
-        # No wait on the compute stream: _decode_one synchronised it on the
+        # No wait on the compute stream: _decode_host_gather synchronised it on the
         # host before the read-back, so the previous layer's reads of the
         # staging rows are done, and the hits' GEMV queued since reads only
         # resident rows.  The copies therefore overlap that GEMV.
@@ -173,8 +179,41 @@ class CADIPMlp(nn.Module):
 
     def _decode_one(self, xv: torch.Tensor) -> torch.Tensor:
         b = self.buf
+        if self.k not in (1, b.k):
+            raise RuntimeError(f"the buffers stage {b.k} channels, the module selects {self.k}")
         g, idx = K.gate_silu_topk(self.gate_qw, self.gate_sc, xv, self.k, g=b.g(self.inter))
         combined, src, row, miss, counts = K.ca_assemble(self.id2slot, idx)
+        stream = torch.cuda.current_stream(self.device)
+        assembled = stream.record_event()
+        timing = b.transfers is not None
+        t0 = time.perf_counter()
+        start = stream.record_event(torch.cuda.Event(enable_timing=True)) if timing else None
+        if not K.stream_rows((self.up_qw, self.up_sc, self.down_t_qw, self.down_t_sc), miss,
+                             counts[1:], (b.gpu_up_qw, b.gpu_up_sc, b.gpu_dn_qw, b.gpu_dn_sc)):
+            return self._decode_host_gather(xv, g, combined, src, row, miss, counts)
+        streamed = stream.record_event(torch.cuda.Event(enable_timing=timing))
+        h = b.h[: self.k]
+        if self.k:
+            K.ca_fused_gemv(self._res_up_qw, self._res_up_sc, b.gpu_up_qw, b.gpu_up_sc, xv, src,
+                            row, g=g, gid=combined, out=h)
+        y = K.ca_down(self._res_dn_qw, self._res_dn_sc, b.gpu_dn_qw, b.gpu_dn_sc, h, src, row)
+        # the counts come back beside the rows; the host rows are the caller's
+        # again once they have been read
+        b.copy_stream.wait_event(assembled)
+        with torch.cuda.stream(b.copy_stream):
+            b.host_counts.copy_(counts, non_blocking=True)
+        b.copy_stream.synchronize()
+        b.last_n_hit, b.last_n_miss = b.host_counts.tolist()
+        streamed.synchronize()
+        if timing and b.last_n_miss:
+            rows = (b.gpu_up_qw, b.gpu_up_sc, b.gpu_dn_qw, b.gpu_dn_sc)
+            nbytes = b.last_n_miss * sum(r.stride(0) * r.element_size() for r in rows)
+            b.transfers.append((nbytes, time.perf_counter() - t0, start.elapsed_time(streamed)))
+        return y
+
+    def _decode_host_gather(self, xv, g, combined, src, row, miss, counts):
+        """The rest of _decode_one where the device cannot read the matrices."""
+        b = self.buf
         # one read-back of the counts and the miss ids (the host sync the
         # reference also has, dip_ca.py:139-146)
         b.host_counts.copy_(counts, non_blocking=True)

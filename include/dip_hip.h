@@ -449,6 +449,20 @@ int dip_host_stream_rows(const void* const* src, void* const* pinned, void* cons
                          void* stream, float* copy_ms);
 
 /*
+ * The cache-aware miss stream (dip_ca.py:146-156) by the device itself:
+ * dst[p] + i * row_bytes[p] <- src[p] + ids[i] * row_bytes[p] for every piece
+ * p < npieces (at most 8) and i < *count, where src[p] is pinned host memory
+ * (src_rows rows), dst[p] device memory (max_rows rows, which bounds *count),
+ * and ids and count lie in device memory: nothing comes back to the host and
+ * no host thread gathers.  An id outside [0, src_rows) leaves its rows zero.
+ * Returns DIP_ERR_UNSUPPORTED, having queued nothing, where a source is not
+ * pinned.
+ */
+int dip_stream_rows(const void* const* src, void* const* dst, const int64_t* row_bytes,
+                    int64_t npieces, const int32_t* ids, const int32_t* count,
+                    int64_t max_rows, int64_t src_rows, void* stream);
+
+/*
  * dip_int4_gemv with the input RMSNorm of a decoder layer folded in:
  * v = bf16(h + add) (add may be NULL), x = bf16(norm_w * bf16(v * rsqrt(
  * mean(v^2) + eps))) (transformers' Qwen3RMSNorm, fp32 mean), out = the
