@@ -78,6 +78,9 @@ _SIGS = {
     "dip_int4_gemm_t": ([_p, _p, _p, _p, _i64, _i64, _i64, _p, _sz, _p], _i32),
     "dip_int4_gemv_rmsnorm": ([_p, _p, _p, _p, _p, ctypes.c_float, _p, _p, _i64, _i64, _p],
                               _i32),
+    "dip_add_rmsnorm_rows": ([_p, _p, _p, _p, _i64, _i64, ctypes.c_float, _p], _i32),
+    "dip_qk_norm_rope_cache_rows": ([_p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64,
+                                     ctypes.c_float, _p], _i32),
     "dip_add_rmsnorm": ([_p, _p, _p, _p, _i64, ctypes.c_float, _p], _i32),
     "dip_qk_norm_rope_cache": ([_p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64,
                                 ctypes.c_float, _p], _i32),
@@ -649,22 +652,52 @@ def _pos_tensor(pos: torch.Tensor, dev) -> torch.Tensor:
     return pos
 
 
-def add_rmsnorm(h, add, weight, out, eps: float):
-    """In place h = bf16(h + add) (when add is given), then
-    out = bf16(weight * bf16(h * rsqrt(mean(h^2) + eps)))."""
+def _add_rmsnorm(h, add, weight, out, eps: float, rows: int, n: int):
     dev = _dev(h, weight, out)
-    n = h.numel()
-    _bf16_vec(h, n, "h")
+    _bf16_vec(h, rows * n, "h")
     _bf16_vec(weight, n, "weight")
-    _bf16_vec(out, n, "out")
+    _bf16_vec(out, rows * n, "out")
     if add is not None:
         _dev(add)
         if add.device != dev:
             raise RuntimeError("add must be on h's device")
-        _bf16_vec(add, n, "add")
-    _check(lib.dip_add_rmsnorm(_ptr(h), _ptr(add), _ptr(weight), _ptr(out), n, float(eps),
-                               _stream(dev)), "dip_add_rmsnorm")
+        _bf16_vec(add, rows * n, "add")
+    _check(lib.dip_add_rmsnorm_rows(_ptr(h), _ptr(add), _ptr(weight), _ptr(out), rows, n,
+                                    float(eps), _stream(dev)), "dip_add_rmsnorm")
     return out
+
+
+def add_rmsnorm(h, add, weight, out, eps: float):
+    """In place h = bf16(h + add) (when add is given), then
+    out = bf16(weight * bf16(h * rsqrt(mean(h^2) + eps)))."""
+    return _add_rmsnorm(h, add, weight, out, eps, 1, h.numel())
+
+
+def add_rmsnorm_rows(h, add, weight, out, eps: float):
+    """add_rmsnorm of each row of h [rows, n] (a prompt's tokens)."""
+    return _add_rmsnorm(h, add, weight, out, eps, *h.shape)
+
+
+def _qk_check(qkv, q_norm_w, k_norm_w, cos, sin, q_out, k_cache, v_cache, n_heads, n_kv_heads,
+              tokens):
+    dev = _dev(qkv, q_out, k_cache, v_cache)
+    hd = q_norm_w.numel()
+    if k_cache.dim() != 3 or k_cache.shape != v_cache.shape or k_cache.shape[0] != n_kv_heads \
+            or k_cache.shape[2] != hd:
+        raise RuntimeError("k_cache / v_cache must be [n_kv_heads, max_len, head_dim]")
+    max_len = k_cache.shape[1]
+    _bf16_vec(qkv, tokens * (n_heads + 2 * n_kv_heads) * hd, "qkv")
+    _bf16_vec(q_norm_w, hd, "q_norm_w")
+    _bf16_vec(k_norm_w, hd, "k_norm_w")
+    _bf16_vec(cos, max_len * hd, "cos")
+    _bf16_vec(sin, max_len * hd, "sin")
+    _bf16_vec(q_out, tokens * n_heads * hd, "q_out")
+    _bf16_vec(k_cache, n_kv_heads * max_len * hd, "k_cache")
+    _bf16_vec(v_cache, n_kv_heads * max_len * hd, "v_cache")
+    for t in (q_norm_w, k_norm_w, cos, sin):
+        if t.device != dev:
+            raise RuntimeError("all tensors must be on one device")
+    return dev, hd, max_len
 
 
 def qk_norm_rope_cache(qkv, q_norm_w, k_norm_w, cos, sin, pos, q_out, k_cache, v_cache,
@@ -672,28 +705,27 @@ def qk_norm_rope_cache(qkv, q_norm_w, k_norm_w, cos, sin, pos, q_out, k_cache, v
     """q/k head RMSNorm + rotary embedding at `pos` for one token's q|k|v;
     q -> q_out, k and v -> row pos of the [n_kv_heads, max_len, head_dim]
     caches."""
-    dev = _dev(qkv, q_out, k_cache, v_cache)
-    hd = q_norm_w.numel()
-    if k_cache.dim() != 3 or k_cache.shape != v_cache.shape or k_cache.shape[0] != n_kv_heads \
-            or k_cache.shape[2] != hd:
-        raise RuntimeError("k_cache / v_cache must be [n_kv_heads, max_len, head_dim]")
-    max_len = k_cache.shape[1]
-    _bf16_vec(qkv, (n_heads + 2 * n_kv_heads) * hd, "qkv")
-    _bf16_vec(q_norm_w, hd, "q_norm_w")
-    _bf16_vec(k_norm_w, hd, "k_norm_w")
-    _bf16_vec(cos, max_len * hd, "cos")
-    _bf16_vec(sin, max_len * hd, "sin")
-    _bf16_vec(q_out, n_heads * hd, "q_out")
-    _bf16_vec(k_cache, n_kv_heads * max_len * hd, "k_cache")
-    _bf16_vec(v_cache, n_kv_heads * max_len * hd, "v_cache")
-    for t in (q_norm_w, k_norm_w, cos, sin):
-        if t.device != dev:
-            raise RuntimeError("all tensors must be on one device")
+    dev, hd, max_len = _qk_check(qkv, q_norm_w, k_norm_w, cos, sin, q_out, k_cache, v_cache,
+                                 n_heads, n_kv_heads, 1)
     _pos_tensor(pos, dev)
     _check(lib.dip_qk_norm_rope_cache(_ptr(qkv), _ptr(q_norm_w), _ptr(k_norm_w), _ptr(cos),
                                       _ptr(sin), _ptr(pos), _ptr(q_out), _ptr(k_cache),
                                       _ptr(v_cache), n_heads, n_kv_heads, hd, max_len,
                                       float(eps), _stream(dev)), "dip_qk_norm_rope_cache")
+    return q_out
+
+
+def qk_norm_rope_cache_rows(qkv, q_norm_w, k_norm_w, cos, sin, q_out, k_cache, v_cache,
+                            n_heads: int, n_kv_heads: int, eps: float):
+    """qk_norm_rope_cache for the tokens of a prompt: row t of qkv [tokens, ..]
+    at position t, q to row t of q_out, k and v to row t of the caches."""
+    tokens = qkv.shape[0]
+    dev, hd, max_len = _qk_check(qkv, q_norm_w, k_norm_w, cos, sin, q_out, k_cache, v_cache,
+                                 n_heads, n_kv_heads, tokens)
+    _check(lib.dip_qk_norm_rope_cache_rows(_ptr(qkv), _ptr(q_norm_w), _ptr(k_norm_w), _ptr(cos),
+                                           _ptr(sin), _ptr(q_out), _ptr(k_cache), _ptr(v_cache),
+                                           tokens, n_heads, n_kv_heads, hd, max_len, float(eps),
+                                           _stream(dev)), "dip_qk_norm_rope_cache_rows")
     return q_out
 
 

@@ -384,6 +384,61 @@ class DIPDecoder:
         K.add_rmsnorm(h, y, inner.norm.weight, self._x, inner.norm.variance_epsilon)
         return self._x.view(1, 1, H)
 
+    # -- a prompt through the fused kernels --------------------------------------
+    def _prefill_fusible(self) -> bool:
+        """Whether a prompt may pass by the HF modules around the projections
+        and MLPs: the attention is the one _prefill_fused makes, without
+        dropout, and nobody observes or replaced a module it passes by."""
+        from dip_ca import CADIPMlp
+        from dip_stream_predispatch import StreamingDIPMlp
+        from torch.nn.modules import module as M
+        if self.model.config._attn_implementation != "sdpa" or M._global_forward_hooks \
+                or M._global_forward_pre_hooks:
+            return False
+        inner = self.model.model
+        passed = [self.model, inner, inner.norm, inner.rotary_emb]
+        for L in self.layers:
+            a = L.self_attn
+            if not isinstance(L.mlp, (StreamingDIPMlp, CADIPMlp)) or \
+                    (a.training and a.attention_dropout):
+                return False
+            passed += [L, L.input_layernorm, L.post_attention_layernorm, a, a.q_norm, a.k_norm,
+                       a.q_proj, a.k_proj, a.v_proj]
+        return not any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__
+                       for m in passed)
+
+    def _prefill_fused(self, ids: torch.Tensor) -> torch.Tensor:
+        """prefill with the decode kernels' prompt forms around the
+        projections: one q|k|v product; q/k norm, rotary embedding and the
+        static cache's rows in one launch; residual add and RMSNorm in one; and
+        the head for the last token alone."""
+        from qlinear import int4_linear
+        K, inner, hd, nh = self._K, self.model.model, self.hd, self.nh
+        plen = ids.shape[1]
+        h = inner.embed_tokens(ids).view(plen, self.hidden)
+        x = torch.empty_like(h)
+        q = torch.empty(plen, nh * hd, dtype=self.dtype, device=self.device)
+        y = None
+        for i, L in enumerate(self.layers):
+            a, n_in, pn = L.self_attn, L.input_layernorm, L.post_attention_layernorm
+            kc, vc = self.k_cache[i], self.v_cache[i]
+            K.add_rmsnorm_rows(h, y, n_in.weight, x, n_in.variance_epsilon)
+            qkv = int4_linear(x, *self._qkv_w[i])
+            K.qk_norm_rope_cache_rows(qkv, a.q_norm.weight, a.k_norm.weight, self.cos, self.sin, q,
+                                      kc, vc, nh, self.nkv, a.q_norm.variance_epsilon)
+            o = F.scaled_dot_product_attention(
+                q.view(1, plen, nh, hd).transpose(1, 2), kc[None, :, :plen], vc[None, :, :plen],
+                is_causal=plen > 1, scale=a.scaling, enable_gqa=nh != self.nkv)
+            o = a.o_proj(o.transpose(1, 2).reshape(1, plen, nh * hd))
+            K.add_rmsnorm_rows(h, o.reshape(plen, -1), pn.weight, x, pn.variance_epsilon)
+            y = L.mlp(x.view(1, plen, -1)).reshape(plen, -1)
+        n = inner.norm
+        last = torch.empty(self.hidden, dtype=self.dtype, device=self.device)
+        K.add_rmsnorm(h[-1], y[-1], n.weight, last, n.variance_epsilon)
+        logits = self._head(last.view(1, 1, -1))
+        self.pos.fill_(plen)
+        return logits
+
     # -- one decode step (device-side token and position) ---------------------
     def _body(self) -> torch.Tensor:
         if self.fused:
@@ -454,14 +509,17 @@ class DIPDecoder:
     # -- prompt ---------------------------------------------------------------
     @torch.no_grad()
     def prefill(self, input_ids: torch.Tensor) -> torch.Tensor:
-        """Run the prompt [1, P] through the HF forward, copy its key/value
-        cache into the static cache, set `tok` to the argmax of the last
-        logits and `pos` to P.  Returns the last logits."""
+        """Run the prompt [1, P] through the model (with the fused kernels
+        where they serve, else the HF forward, whose key/value cache is copied
+        into the static cache), set `tok` to the argmax of the last logits and
+        `pos` to P.  Returns the last logits."""
         from transformers import DynamicCache
         ids = input_ids.to(self.device).view(1, -1)
         plen = ids.shape[1]
         if plen < 1 or plen >= self.max_len:
             raise ValueError(f"prompt length {plen} outside [1, {self.max_len})")
+        if self.fused and self._prefill_fusible():
+            return self._prefill_fused(ids)
         cache = DynamicCache(config=self.model.config)
         out = self.model(input_ids=ids, past_key_values=cache, use_cache=True)
         for i, layer in enumerate(cache.layers):

@@ -545,6 +545,18 @@ int dip_qk_norm_rope_cache(const uint16_t* qkv, const uint16_t* q_norm_w,
                            int64_t n_kv_heads, int64_t head_dim, int64_t max_len, float eps,
                            void* stream);
 
+/* Both of the above for the tokens of a prompt: `rows` rows of n values, and
+ * `tokens` tokens at positions 0 .. tokens - 1 (at most max_len), token t's
+ * q|k|v at row t of qkv and its q at row t of q_out. */
+int dip_add_rmsnorm_rows(uint16_t* h, const uint16_t* add, const uint16_t* weight,
+                         uint16_t* out, int64_t rows, int64_t n, float eps, void* stream);
+int dip_qk_norm_rope_cache_rows(const uint16_t* qkv, const uint16_t* q_norm_w,
+                                const uint16_t* k_norm_w, const uint16_t* cos_table,
+                                const uint16_t* sin_table, uint16_t* q_out, uint16_t* k_cache,
+                                uint16_t* v_cache, int64_t tokens, int64_t n_heads,
+                                int64_t n_kv_heads, int64_t head_dim, int64_t max_len, float eps,
+                                void* stream);
+
 /*
  * dip_decode_attention: out[h] = softmax(scale * q[h] . K[j]) V over cache
  * rows j = 0 .. pos of kv head h / (n_heads / n_kv_heads) (grouped-query
