@@ -72,6 +72,7 @@ _SIGS = {
     "dip_host_gather_rows": ([_p, _p, _p, _i64, _i64, _i64, _i32], _i32),
     "dip_host_gather_rows_multi": ([_p, _p, _p, _i64, _p, _i64, _i64, _i32], _i32),
     "dip_host_stream_rows": ([_p, _p, _p, _p, _i64, _p, _i64, _i64, _i64, _i32, _p, _p], _i32),
+    "dip_swiglu": ([_p, _p, _p, _i64, _p], _i32),
     "dip_stream_rows": ([_p, _p, _p, _i64, _p, _p, _i64, _i64, _p], _i32),
     "dip_int4_gemm": ([_p, _p, _p, _p, _i64, _i64, _i64, _p], _i32),
     "dip_int4_gemm_t_workspace_size": ([_i64, _i64, _i64], _sz),
@@ -475,6 +476,16 @@ def ca_assemble(id2slot: torch.Tensor, idx: torch.Tensor):
                                _ptr(miss), _ptr(counts), id2slot.numel(), k, _stream(dev)),
            "dip_ca_assemble")
     return combined, src, row, miss, counts
+
+
+def swiglu(g, u):
+    """bf16(bf16(silu(g)) * u) of two contiguous bf16 tensors of one shape."""
+    dev = _dev(g, u)
+    g = _want(g, torch.bfloat16, "g")
+    u = _want(u, torch.bfloat16, "u", g.shape)
+    out = torch.empty_like(g)
+    _check(lib.dip_swiglu(_ptr(g), _ptr(u), _ptr(out), g.numel(), _stream(dev)), "dip_swiglu")
+    return out
 
 
 def dequant_rows(qweight, scales, indices=None, mode: int = 0):

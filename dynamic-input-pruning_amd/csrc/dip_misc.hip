@@ -1,4 +1,4 @@
-// dip_misc.hip — cache-aware hit/miss assembly and miss stream, row dequantisation, the
+// dip_misc.hip — cache-aware hit/miss assembly and miss stream, SwiGLU, row dequantisation, the
 // host-side miss gather, the one-call resident MLP decode step and the
 // library's status helpers.
 #include <algorithm>
@@ -437,6 +437,67 @@ extern "C" int dip_stream_rows(const void* const* src, void* const* dst, const i
   a.per_row = (uint32_t)per_row;
   hipLaunchKernelGGL(stream_rows_kernel, dim3(kStreamBlocks), dim3(256), 0, (hipStream_t)stream, a,
                      ids, count, (uint32_t)max_rows, (uint32_t)src_rows);
+  return hip_status(hipGetLastError());
+}
+
+// ---------------------------------------------------------------------------
+// SwiGLU of a prompt's gate and up products, h = bf16(bf16(silu(g)) * u), with
+// the roundings of the two torch ops it takes the place of.  Bound by memory
+// beside expf and a division per value.  A block takes kSwigluUnroll runs of
+// 256 vectors, all loaded first.  2048 x 25600 values 64 us (4.9 TB/s; the two
+// ops 95), 333 x 12288 8.6 us (12.1).
+// ---------------------------------------------------------------------------
+namespace {
+constexpr int kSwigluUnroll = 2;
+
+DIP_DEV uint32_t swiglu2(uint32_t g, uint32_t u) {
+  const float g0 = bf16_to_f32(g & 0xFFFFu), g1 = bf16_to_f32(g >> 16);
+  const float s0 = bf16_to_f32(f32_to_bf16(g0 / (1.0f + expf(-g0))));
+  const float s1 = bf16_to_f32(f32_to_bf16(g1 / (1.0f + expf(-g1))));
+  return f32_to_bf16(s0 * bf16_to_f32(u & 0xFFFFu)) | (f32_to_bf16(s1 * bf16_to_f32(u >> 16)) << 16);
+}
+
+__global__ __launch_bounds__(256) void swiglu_kernel(const uint16_t* __restrict__ g,
+                                                     const uint16_t* __restrict__ u,
+                                                     uint16_t* __restrict__ out, size_t n) {
+  const size_t nv = n / 8;
+  const size_t v0 = (size_t)blockIdx.x * (256 * kSwigluUnroll) + threadIdx.x;
+  uint4 a[kSwigluUnroll], b[kSwigluUnroll];
+#pragma unroll
+  for (int i = 0; i < kSwigluUnroll; ++i) {
+    const size_t v = v0 + 256 * i;
+    if (v < nv) {
+      a[i] = reinterpret_cast<const uint4*>(g)[v];
+      b[i] = reinterpret_cast<const uint4*>(u)[v];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kSwigluUnroll; ++i) {
+    const size_t v = v0 + 256 * i;
+    if (v < nv)
+      reinterpret_cast<uint4*>(out)[v] =
+          make_uint4(swiglu2(a[i].x, b[i].x), swiglu2(a[i].y, b[i].y), swiglu2(a[i].z, b[i].z),
+                     swiglu2(a[i].w, b[i].w));
+  }
+  // the values past the last vector
+  if (blockIdx.x == 0 && threadIdx.x < (n & 7)) {
+    const size_t e = 8 * nv + threadIdx.x;
+    out[e] = (uint16_t)swiglu2(g[e], u[e]);
+  }
+}
+
+}  // namespace
+
+extern "C" int dip_swiglu(const uint16_t* g, const uint16_t* u, uint16_t* out, int64_t n,
+                          void* stream) {
+  if (n < 0) return DIP_ERR_SHAPE;
+  if (n == 0) return DIP_OK;
+  if (!g || !u || !out) return DIP_ERR_NULL;
+  if (!aligned16(g) || !aligned16(u) || !aligned16(out)) return DIP_ERR_ALIGN;
+  const size_t blocks = ((size_t)n / 8 + 256 * kSwigluUnroll - 1) / (256 * kSwigluUnroll);
+  if (blocks > INT32_MAX) return DIP_ERR_SHAPE;
+  hipLaunchKernelGGL(swiglu_kernel, dim3((unsigned)std::max<size_t>(blocks, 1)), dim3(256), 0,
+                     (hipStream_t)stream, g, u, out, (size_t)n);
   return hip_status(hipGetLastError());
 }
 

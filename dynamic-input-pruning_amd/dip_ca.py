@@ -30,10 +30,9 @@ import time
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 import _dip_hip as K
-from qlinear import GROUP_SIZE, dequantize, int4_linear, int4_linear_t
+from qlinear import GROUP_SIZE, dequantize, int4_linear, int4_linear_t, swiglu
 from dip_stream_predispatch import _transpose_down_to_int4, _use_gather, _use_down  # noqa: F401
 
 _use_ca_fused = True
@@ -241,9 +240,9 @@ class CADIPMlp(nn.Module):
 
     def _dense(self, x):
         """Prefill route (dip_ca.py:190-196), as StreamingDIPMlp._dense."""
-        g = F.silu(self._gate(x))
+        g = self._gate(x)
         u = int4_linear(x, self.up_qw.to(self.device), self.up_sc.to(self.device))
-        h = g * u
+        h = swiglu(g, u)
         return int4_linear_t(h, self.down_t_qw.to(self.device), self.down_t_sc.to(self.device))
 
 

@@ -25,10 +25,9 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 import _dip_hip as K
-from qlinear import GROUP_SIZE, dequantize, int4_linear, int4_linear_t, _unpack_int4
+from qlinear import GROUP_SIZE, dequantize, int4_linear, int4_linear_t, swiglu, _unpack_int4
 from quantize import pack_int4
 
 # The reference decides these from which kernel .so files it found; here the
@@ -208,9 +207,9 @@ class StreamingDIPMlp(nn.Module):
         """Prefill route (dip_stream_predispatch.py:206-215): every channel; the
         gate and up projections through int4_linear (the int4 GEMM for short
         prompts), down through its dequantized transpose."""
-        g = F.silu(self._gate(x))
+        g = self._gate(x)
         u = int4_linear(x, self.up_qw, self.up_sc)
-        h = g * u
+        h = swiglu(g, u)
         return int4_linear_t(h, self.down_t_qw, self.down_t_sc)
 
     # Introspection used by tests: the intermediates of the last decode call.

@@ -88,6 +88,15 @@ def int4_linear_t(x: torch.Tensor, qweight_t: torch.Tensor, scales_t: torch.Tens
     return x @ dequantize(qweight_t, scales_t).to(x.dtype)
 
 
+def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
+    """F.silu(gate) * up, in one launch for plain bf16 tensors on the device
+    (the same roundings)."""
+    if gate.is_cuda and gate.shape == up.shape and _plain_bf16(gate, up) and _plain_bf16(up, gate):
+        import _dip_hip as K
+        return K.swiglu(gate, up)
+    return F.silu(gate) * up
+
+
 def _unpack_int4(qweight: torch.Tensor) -> torch.Tensor:
     """int8 [R, C/2] -> int8 [R, C] in [-8, 7] (qlinear.py:28-50)."""
     q = qweight.view(torch.uint8) if qweight.dtype == torch.int8 else qweight.to(torch.uint8)

@@ -241,6 +241,11 @@ int dip_ca_down(const int8_t* res_qw, const uint16_t* res_sc, const int8_t* str_
                 int64_t out_features, int64_t k, void* workspace, size_t ws_bytes,
                 void* stream);
 
+/* h[i] = bf16(bf16(silu(g[i])) * u[i]), i < n: the SwiGLU between the
+ * projections of the dense route (dip_stream_predispatch.py:206-215), rounded
+ * as its two torch ops round. */
+int dip_swiglu(const uint16_t* g, const uint16_t* u, uint16_t* out, int64_t n, void* stream);
+
 /*
  * Cache-aware hit/miss assembly (dip_ca.py:137-171): from idx[k] and
  * id2slot[inter] (int64, -1 = not resident) write, in the order
