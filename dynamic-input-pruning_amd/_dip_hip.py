@@ -72,6 +72,7 @@ _SIGS = {
     "dip_host_gather_rows": ([_p, _p, _p, _i64, _i64, _i64, _i32], _i32),
     "dip_host_gather_rows_multi": ([_p, _p, _p, _i64, _p, _i64, _i64, _i32], _i32),
     "dip_host_stream_rows": ([_p, _p, _p, _p, _i64, _p, _i64, _i64, _i64, _i32, _p, _p], _i32),
+    "dip_int4_gemm_swiglu": ([_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p], _i32),
     "dip_swiglu": ([_p, _p, _p, _i64, _p], _i32),
     "dip_stream_rows": ([_p, _p, _p, _i64, _p, _p, _i64, _i64, _p], _i32),
     "dip_int4_gemm": ([_p, _p, _p, _p, _i64, _i64, _i64, _p], _i32),
@@ -247,6 +248,23 @@ def int4_gemm(qweight, scales, x, out=None):
     _check(lib.dip_int4_gemm(_ptr(qweight), _ptr(scales), _ptr(x2), _ptr(out), m, rows, cols,
                              _stream(dev)), "dip_int4_gemm")
     return out.view(*x.shape[:-1], rows)
+
+
+def int4_gemm_swiglu(gate_qw, gate_sc, up_qw, up_sc, x):
+    """swiglu(int4_gemm(gate, x), int4_gemm(up, x)) in one launch."""
+    gate_qw, gate_sc, rows, cols = _weights(gate_qw, gate_sc, "int4_gemm_swiglu.gate")
+    up_qw, up_sc, rows2, cols2 = _weights(up_qw, up_sc, "int4_gemm_swiglu.up")
+    if (rows2, cols2) != (rows, cols):
+        raise RuntimeError("gate and up differ in shape")
+    dev = _dev(gate_qw, gate_sc, up_qw, up_sc, x)
+    if x.dtype != torch.bfloat16 or x.shape[-1] != cols:
+        raise RuntimeError(f"x must be bf16 [..., {cols}]")
+    x2 = _want(x.reshape(-1, cols), torch.bfloat16, "x")
+    out = torch.empty(*x.shape[:-1], rows, dtype=torch.bfloat16, device=dev)
+    _check(lib.dip_int4_gemm_swiglu(_ptr(gate_qw), _ptr(gate_sc), _ptr(up_qw), _ptr(up_sc),
+                                    _ptr(x2), _ptr(out), x2.shape[0], rows, cols, _stream(dev)),
+           "dip_int4_gemm_swiglu")
+    return out
 
 
 def int4_gemm_t(qweight_t, scales_t, x, out=None):

@@ -287,4 +287,11 @@ DIP_DEV uint4 ldg_nt(const uint4* p) {
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+// bf16(bf16(silu(g)) * u) of bf16 values.
+DIP_DEV uint32_t swiglu_bf16(uint32_t g, uint32_t u) {
+  const float f = bf16_to_f32(g);
+  const float s = bf16_to_f32(f32_to_bf16(f / (1.0f + expf(-f))));
+  return f32_to_bf16(s * bf16_to_f32(u));
+}
+
 }  // namespace dip

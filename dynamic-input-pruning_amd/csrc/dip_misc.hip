@@ -451,10 +451,7 @@ namespace {
 constexpr int kSwigluUnroll = 2;
 
 DIP_DEV uint32_t swiglu2(uint32_t g, uint32_t u) {
-  const float g0 = bf16_to_f32(g & 0xFFFFu), g1 = bf16_to_f32(g >> 16);
-  const float s0 = bf16_to_f32(f32_to_bf16(g0 / (1.0f + expf(-g0))));
-  const float s1 = bf16_to_f32(f32_to_bf16(g1 / (1.0f + expf(-g1))));
-  return f32_to_bf16(s0 * bf16_to_f32(u & 0xFFFFu)) | (f32_to_bf16(s1 * bf16_to_f32(u >> 16)) << 16);
+  return swiglu_bf16(g & 0xFFFFu, u & 0xFFFFu) | (swiglu_bf16(g >> 16, u >> 16) << 16);
 }
 
 __global__ __launch_bounds__(256) void swiglu_kernel(const uint16_t* __restrict__ g,

@@ -32,7 +32,7 @@ import torch
 import torch.nn as nn
 
 import _dip_hip as K
-from qlinear import GROUP_SIZE, dequantize, int4_linear, int4_linear_t, swiglu
+from qlinear import GROUP_SIZE, dequantize, int4_gate_up, int4_linear, int4_linear_t, swiglu
 from dip_stream_predispatch import _transpose_down_to_int4, _use_gather, _use_down  # noqa: F401
 
 _use_ca_fused = True
@@ -240,9 +240,12 @@ class CADIPMlp(nn.Module):
 
     def _dense(self, x):
         """Prefill route (dip_ca.py:190-196), as StreamingDIPMlp._dense."""
-        g = self._gate(x)
-        u = int4_linear(x, self.up_qw.to(self.device), self.up_sc.to(self.device))
-        h = swiglu(g, u)
+        up_qw, up_sc = self.up_qw.to(self.device), self.up_sc.to(self.device)
+        h = None
+        if x.dim() != 3 or x.shape[1] > 1:  # _gate takes the GEMV token by token
+            h = int4_gate_up(x, self.gate_qw, self.gate_sc, up_qw, up_sc)
+        if h is None:
+            h = swiglu(self._gate(x), int4_linear(x, up_qw, up_sc))
         return int4_linear_t(h, self.down_t_qw.to(self.device), self.down_t_sc.to(self.device))
 
 

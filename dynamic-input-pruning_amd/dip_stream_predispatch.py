@@ -27,7 +27,7 @@ import torch
 import torch.nn as nn
 
 import _dip_hip as K
-from qlinear import GROUP_SIZE, dequantize, int4_linear, int4_linear_t, swiglu, _unpack_int4
+from qlinear import GROUP_SIZE, dequantize, int4_gate_up, int4_linear, int4_linear_t, swiglu, _unpack_int4
 from quantize import pack_int4
 
 # The reference decides these from which kernel .so files it found; here the
@@ -204,12 +204,14 @@ class StreamingDIPMlp(nn.Module):
         return torch.stack(ys).to(xdt).reshape(x.shape[0], 1, -1)
 
     def _dense(self, x):
-        """Prefill route (dip_stream_predispatch.py:206-215): every channel; the
-        gate and up projections through int4_linear (the int4 GEMM for short
-        prompts), down through its dequantized transpose."""
-        g = self._gate(x)
-        u = int4_linear(x, self.up_qw, self.up_sc)
-        h = swiglu(g, u)
+        """Prefill route (dip_stream_predispatch.py:206-215): every channel;
+        gate, up and the SwiGLU in one int4 GEMM launch for short prompts, else
+        through int4_linear; down through int4_linear_t."""
+        h = None
+        if x.dim() != 3 or x.shape[1] > 1:  # _gate takes the GEMV token by token
+            h = int4_gate_up(x, self.gate_qw, self.gate_sc, self.up_qw, self.up_sc)
+        if h is None:
+            h = swiglu(self._gate(x), int4_linear(x, self.up_qw, self.up_sc))
         return int4_linear_t(h, self.down_t_qw, self.down_t_sc)
 
     # Introspection used by tests: the intermediates of the last decode call.

@@ -97,6 +97,18 @@ def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     return F.silu(gate) * up
 
 
+def int4_gate_up(x, gate_qw, gate_sc, up_qw, up_sc):
+    """F.silu(x @ gate^T) * (x @ up^T), or None where that is not one launch: it
+    is for the prompts that int4_linear runs on the int4 MFMA GEMM."""
+    import _dip_hip as K
+    in_f = gate_qw.shape[1] * 2
+    rows = x.numel() // in_f
+    if not (1 < rows <= GEMM_MAX_TOKENS and x.shape[-1] == in_f
+            and gate_qw.shape == up_qw.shape and _plain_bf16(x, gate_qw)):
+        return None
+    return K.int4_gemm_swiglu(gate_qw, gate_sc, up_qw, up_sc, x)
+
+
 def _unpack_int4(qweight: torch.Tensor) -> torch.Tensor:
     """int8 [R, C/2] -> int8 [R, C] in [-8, 7] (qlinear.py:28-50)."""
     q = qweight.view(torch.uint8) if qweight.dtype == torch.int8 else qweight.to(torch.uint8)

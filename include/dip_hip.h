@@ -496,6 +496,13 @@ int dip_int4_gemm(const int8_t* qweight, const uint16_t* scales, const uint16_t*
                   uint16_t* out, int64_t m, int64_t out_features, int64_t in_features,
                   void* stream);
 
+/* out[m, inter] = bf16(bf16(silu(bf16(x . gate^T))) * bf16(x . up^T)): both
+ * projections of the dense MLP and the SwiGLU between them in one launch, each
+ * product and rounding as dip_int4_gemm and dip_swiglu make it. */
+int dip_int4_gemm_swiglu(const int8_t* gate_qw, const uint16_t* gate_sc, const int8_t* up_qw,
+                         const uint16_t* up_sc, const uint16_t* x, uint16_t* out, int64_t m,
+                         int64_t inter, int64_t hidden, void* stream);
+
 /*
  * out[m, n] = bf16( sum_c x[m, c] * bf16(q*s)[c, n] ) for W stored as rows
  * of in_features (qweight_t int8 [in_features, out_features/2], scales_t
