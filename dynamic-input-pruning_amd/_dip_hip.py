@@ -155,13 +155,21 @@ def _weights(qw: torch.Tensor, sc: torch.Tensor, name: str):
     cols = half * 2
     if cols % GROUP_SIZE != 0:
         raise RuntimeError(f"{name}: in_features {cols} is not a multiple of {GROUP_SIZE}")
+    # resident weights pass as they are: the checks of _want, without its calls
+    if (qw.dtype is torch.int8 and sc.dtype is torch.bfloat16
+            and sc.shape == (rows, cols // GROUP_SIZE) and qw.is_contiguous()
+            and sc.is_contiguous() and not (qw.data_ptr() | sc.data_ptr()) & 15):
+        return qw, sc, rows, cols
     qw = _want(qw, torch.int8, f"{name}.qweight")
     sc = _want(sc, torch.bfloat16, f"{name}.scales", (rows, cols // GROUP_SIZE))
     return qw, sc, rows, cols
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the handle alone: a Stream object costs 2 us of a small call's 15
+    if device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _ptr(t):
@@ -236,18 +244,19 @@ def int4_gemm(qweight, scales, x, out=None):
     dev = _dev(qweight, scales, x)
     if x.dtype != torch.bfloat16 or x.shape[-1] != cols:
         raise RuntimeError(f"x must be bf16 [..., {cols}]")
-    x2 = x.reshape(-1, cols)
+    x2 = x if x.dim() == 2 else x.reshape(-1, cols)
     if not x2.is_contiguous() or x2.data_ptr() % 16:
         x2 = x2.contiguous().clone() if x2.data_ptr() % 16 else x2.contiguous()
     m = x2.shape[0]
+    shape = (*x.shape[:-1], rows)
     if out is None:
-        out = torch.empty(m, rows, dtype=torch.bfloat16, device=dev)
+        out = torch.empty(shape, dtype=torch.bfloat16, device=dev)
     elif (out.dtype != torch.bfloat16 or out.numel() != m * rows or not out.is_contiguous()
           or out.device != dev):
         raise RuntimeError(f"out must be a contiguous bf16 tensor of {m} x {rows} values")
     _check(lib.dip_int4_gemm(_ptr(qweight), _ptr(scales), _ptr(x2), _ptr(out), m, rows, cols,
                              _stream(dev)), "dip_int4_gemm")
-    return out.view(*x.shape[:-1], rows)
+    return out if out.shape == shape else out.view(shape)
 
 
 def int4_gemm_swiglu(gate_qw, gate_sc, up_qw, up_sc, x):

@@ -235,6 +235,10 @@ class CADIPMlp(nn.Module):
         if x.dim() != 3 or x.shape[1] != 1 or self.keep_ratio >= 0.999 or self._res_up_qw is None:
             return self._dense(x)
         xdt = x.dtype
+        if x.shape[0] == 1:
+            v = x.reshape(-1)
+            y = self._decode_one(v if xdt is torch.bfloat16 else v.to(torch.bfloat16))
+            return (y if xdt is torch.bfloat16 else y.to(xdt)).view(1, 1, -1)
         ys = [self._decode_one(x[i, 0].to(torch.bfloat16)) for i in range(x.shape[0])]
         return torch.stack(ys).to(xdt).reshape(x.shape[0], 1, -1)
 

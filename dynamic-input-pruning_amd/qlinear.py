@@ -67,10 +67,15 @@ def int4_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor) ->
     in_f = qweight.shape[1] * 2
     rows = x.numel() // in_f
     if rows == 1 and in_f in _GEMV_COLS:
-        y = K.int4_gemv(qweight, scales, x.reshape(-1).to(torch.bfloat16))
-        return y.to(x.dtype).reshape(*x.shape[:-1], qweight.shape[0])
+        v = x.reshape(-1)
+        y = K.int4_gemv(qweight, scales, v if v.dtype is torch.bfloat16 else v.to(torch.bfloat16))
+        if y.dtype is not x.dtype:
+            y = y.to(x.dtype)
+        return y.view(*x.shape[:-1], qweight.shape[0])
     if 1 < rows <= _ANY_INPUT_TOKENS or (1 < rows <= GEMM_MAX_TOKENS and x.shape[-1] == in_f
                                          and _plain_bf16(x, qweight)):
+        if x.dtype is torch.bfloat16 and x.shape[-1] == in_f:
+            return K.int4_gemm(qweight, scales, x)
         y = K.int4_gemm(qweight, scales, x.reshape(rows, in_f).to(torch.bfloat16))
         return y.to(x.dtype).reshape(*x.shape[:-1], qweight.shape[0])
     return F.linear(x, dequantize(qweight, scales).to(x.dtype))
