@@ -54,6 +54,7 @@ _SIGS = {
     "dip_ca_down": ([_p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _p, _sz, _p], _i32),
     "dip_ca_assemble": ([_p, _p, _p, _p, _p, _p, _p, _i64, _i64, _p], _i32),
     "dip_dequant_rows": ([_p, _p, _p, _p, _i64, _i64, _i64, _i32, _p], _i32),
+    "dip_dequant_t": ([_p, _p, _p, _i64, _i64, _p], _i32),
     "dip_mlp_workspace_size": ([_i64, _i64, _i64], _sz),
     "dip_mlp_decode": ([_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p,
                         _sz, _p, _p], _i32),
@@ -512,6 +513,17 @@ def swiglu(g, u):
     u = _want(u, torch.bfloat16, "u", g.shape)
     out = torch.empty_like(g)
     _check(lib.dip_swiglu(_ptr(g), _ptr(u), _ptr(out), g.numel(), _stream(dev)), "dip_swiglu")
+    return out
+
+
+def dequant_t(qweight, scales):
+    """The transpose of bf16(q*s), contiguous [cols, rows] (rows a multiple of
+    8)."""
+    qweight, scales, rows, cols = _weights(qweight, scales, "dequant_t")
+    dev = _dev(qweight, scales)
+    out = torch.empty(cols, rows, dtype=torch.bfloat16, device=dev)
+    _check(lib.dip_dequant_t(_ptr(qweight), _ptr(scales), _ptr(out), rows, cols, _stream(dev)),
+           "dip_dequant_t")
     return out
 
 

@@ -90,6 +90,8 @@ def int4_linear_t(x: torch.Tensor, qweight_t: torch.Tensor, scales_t: torch.Tens
     rows = x.numel() // x.shape[-1]
     if rows <= _ANY_INPUT_TOKENS or (rows <= GEMM_T_MAX_TOKENS and _plain_bf16(x, qweight_t)):
         return K.int4_gemm_t(qweight_t, scales_t, x.to(torch.bfloat16)).to(x.dtype)
+    if qweight_t.is_cuda and qweight_t.shape[0] % 8 == 0:
+        return F.linear(x, K.dequant_t(qweight_t, scales_t).to(x.dtype))
     return x @ dequantize(qweight_t, scales_t).to(x.dtype)
 
 

@@ -268,6 +268,12 @@ int dip_dequant_rows(const int8_t* qweight, const uint16_t* scales, const int32_
                      void* out, int64_t n_out_rows, int64_t rows, int64_t cols, int mode,
                      void* stream);
 
+/* out bf16 [cols, rows] = the transpose of bf16(q*s): what a library product
+ * with the transposed down matrix reads fastest.  qweight and out 16-byte
+ * aligned; rows a multiple of 8 (else DIP_ERR_UNSUPPORTED). */
+int dip_dequant_t(const int8_t* qweight, const uint16_t* scales, uint16_t* out, int64_t rows,
+                  int64_t cols, void* stream);
+
 /*
  * Quantize w [rows, cols] (fp32, or bf16 when w_is_bf16) to int4 g128:
  * s = max(max|w_group| / 7, 1e-8) in fp32, q = clamp(round_half_even(w / s),
