@@ -341,7 +341,7 @@ def cache_aware(args) -> int:
         "miss_bytes_per_token": int(miss_bytes / args.steps),
         "pcie_gbs": round(miss_bytes / copy_s / 1e9, 2) if copy_s > 0 else None,
         "copy_ms_per_token": round(copy_s * 1e3 / args.steps, 3),
-        # host gather + queued copies, until the last copy ends
+        # from queueing the stream until its rows are there
         "miss_stream_gbs": round(miss_bytes / stream_s / 1e9, 2) if stream_s > 0 else None,
         "miss_stream_ms_per_token": round(stream_s * 1e3 / args.steps, 3),
     }

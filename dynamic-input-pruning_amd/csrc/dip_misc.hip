@@ -518,8 +518,9 @@ __global__ __launch_bounds__(64 * kDqtWaves) void dequant_t_kernel(const int8_t*
                                                                    int rows, int cols) {
   __shared__ __align__(16) uint32_t tile[kDqtWaves][32][kDqtRows / 2];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int c0 = ((int)blockIdx.x * kDqtWaves + wave) * 32, r0 = (int)blockIdx.y * kDqtRows;
-  if (c0 >= cols) return;  // whole waves: the tiles are the waves' own
+  // waves past the last column repeat it (the same values, stored once more)
+  const int c0 = min(((int)blockIdx.x * kDqtWaves + wave) * 32, cols - 32);
+  const int r0 = (int)blockIdx.y * kDqtRows;
   uint4 w[2];
   uint32_t s[2];
 #pragma unroll

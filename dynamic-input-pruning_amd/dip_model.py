@@ -8,11 +8,12 @@ swap each decoder MLP for a DIP module, then load every other tensor of
 model_int4.safetensors.  One MI355X holds the whole model in HBM, so every
 tensor goes to one device; there is no offload map.
 
-``DIPDecoder`` runs greedy decoding.  The prompt goes through the HF forward
-(the reference's prefill: the DIP modules take their dense route for
-sequences longer than one token), then its key/value cache is copied into a
-static cache and every further token runs one decode step that reads nothing
-from the host: embedding, per layer RMSNorm -> q/k/v projections (int4 GEMV)
+``DIPDecoder`` runs greedy decoding.  The prompt runs like the HF forward (the
+reference's prefill: the DIP modules take their dense route for sequences
+longer than one token), on this library's kernels around the projections and
+MLPs where the model fits them, and leaves its keys and values in a static
+cache; every further token runs one decode step that reads nothing from the
+host: embedding, per layer RMSNorm -> q/k/v projections (int4 GEMV)
 -> q/k RMSNorm -> rotary embedding from a precomputed table -> cache write
 at the device-side position -> attention over the static cache with a
 position mask -> o projection -> RMSNorm -> DIP MLP, then the final norm,
@@ -392,15 +393,15 @@ class DIPDecoder:
         from dip_ca import CADIPMlp
         from dip_stream_predispatch import StreamingDIPMlp
         from torch.nn.modules import module as M
-        if self.model.config._attn_implementation != "sdpa" or M._global_forward_hooks \
-                or M._global_forward_pre_hooks:
+        if getattr(self.model.config, "_attn_implementation", None) != "sdpa" \
+                or M._global_forward_hooks or M._global_forward_pre_hooks:
             return False
         inner = self.model.model
-        passed = [self.model, inner, inner.norm, inner.rotary_emb]
+        passed = [self.model, inner, inner.norm, inner.rotary_emb, self.model.lm_head]
         for L in self.layers:
             a = L.self_attn
             if not isinstance(L.mlp, (StreamingDIPMlp, CADIPMlp)) or \
-                    (a.training and a.attention_dropout):
+                    (a.training and getattr(a, "attention_dropout", 0)):
                 return False
             passed += [L, L.input_layernorm, L.post_attention_layernorm, a, a.q_norm, a.k_norm,
                        a.q_proj, a.k_proj, a.v_proj]

@@ -11,8 +11,9 @@ how the reference uses it at load time (e.g. the one-time down transpose).
 ``QuantLinear`` is the reference's projection layer (qlinear.py:67-88).  On
 the GPU it reads the packed weight once instead of writing and re-reading a
 bf16 copy: the int4 GEMV for one token, the int4 MFMA GEMM for prompts of up
-to GEMM_MAX_TOKENS tokens; longer prompts take the reference's dequant +
-F.linear route.  Both kernels take the weights as exact fp32 q*s (the
+to GEMM_MAX_TOKENS tokens (gate, up and the SwiGLU of an MLP in one launch up
+to GATE_UP_MAX_TOKENS); longer prompts take the reference's dequant + F.linear
+route.  Both kernels take the weights as exact fp32 q*s (the
 reference rounds them to bf16 first), so they differ from dequant + F.linear
 by rounding only.
 ``_replace_linears_with_quant`` and ``load_quantized_qwen3`` build the
@@ -42,10 +43,18 @@ GEMM_MAX_TOKENS = 512
 # Up to this many rows it takes any input, rounded to bf16; beyond, plain bf16
 # tensors only (_plain_bf16).
 _ANY_INPUT_TOKENS = 64
-# The transposed GEMM's limit (us, against dequantize and the library's
-# product: 25600 x 5120, 512 tokens 210 / 338, 1024 tokens 418 / 401; 12288 x
-# 4096, 512 tokens 85 / 128, 1024 tokens 147 / 148).
+# Gate and up in one launch win a little longer (us, against both library
+# products, their dequantisation and the SwiGLU: 25600 x 5120, 512 tokens 338 /
+# 412, 768 tokens 463 / 510, 900 tokens 552 / 535; 12288 x 4096, 512 tokens 135 /
+# 153, 640 tokens 178 / 171, 768 tokens 193 / 202, 900 tokens 226 / 209).
+GATE_UP_MAX_TOKENS = 768
+# The transposed GEMM's limits, for a matrix of GEMM_T_LONG_VALUES weights or
+# more and for smaller ones (us, against dequantize and the library's product:
+# 25600 x 5120, 512 tokens 211 / 339, 768 tokens 263 / 363, 900 tokens 515 / 408;
+# 12288 x 4096, 512 tokens 79 / 92, 576 tokens 125 / 104, 768 tokens 126 / 106).
 GEMM_T_MAX_TOKENS = 768
+GEMM_T_SHORT_TOKENS = 512
+GEMM_T_LONG_VALUES = 100_000_000
 
 
 def _plain_bf16(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -84,11 +93,14 @@ def int4_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor) ->
 def int4_linear_t(x: torch.Tensor, qweight_t: torch.Tensor, scales_t: torch.Tensor) -> torch.Tensor:
     """x @ bf16(q*s) for a matrix stored as rows of the input dimension (the
     transposed down matrix) on the device, in x's dtype: the int4 MFMA GEMM
-    for up to GEMM_T_MAX_TOKENS rows of x, else x @ dequantize (the reference's
-    route, dip_stream_predispatch.py:213-215)."""
+    for up to GEMM_T_MAX_TOKENS rows of x (GEMM_T_SHORT_TOKENS for a smaller
+    matrix), else x @ dequantize (the reference's route,
+    dip_stream_predispatch.py:213-215), on the transpose where that can be."""
     import _dip_hip as K
     rows = x.numel() // x.shape[-1]
-    if rows <= _ANY_INPUT_TOKENS or (rows <= GEMM_T_MAX_TOKENS and _plain_bf16(x, qweight_t)):
+    most = (GEMM_T_MAX_TOKENS if 2 * qweight_t.numel() >= GEMM_T_LONG_VALUES
+            else GEMM_T_SHORT_TOKENS)
+    if rows <= _ANY_INPUT_TOKENS or (rows <= most and _plain_bf16(x, qweight_t)):
         return K.int4_gemm_t(qweight_t, scales_t, x.to(torch.bfloat16)).to(x.dtype)
     if qweight_t.is_cuda and qweight_t.shape[0] % 8 == 0:
         return F.linear(x, K.dequant_t(qweight_t, scales_t).to(x.dtype))
@@ -106,11 +118,11 @@ def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
 
 def int4_gate_up(x, gate_qw, gate_sc, up_qw, up_sc):
     """F.silu(x @ gate^T) * (x @ up^T), or None where that is not one launch: it
-    is for the prompts that int4_linear runs on the int4 MFMA GEMM."""
+    is for plain bf16 prompts of up to GATE_UP_MAX_TOKENS."""
     import _dip_hip as K
     in_f = gate_qw.shape[1] * 2
     rows = x.numel() // in_f
-    if not (1 < rows <= GEMM_MAX_TOKENS and x.shape[-1] == in_f
+    if not (1 < rows <= GATE_UP_MAX_TOKENS and x.shape[-1] == in_f
             and gate_qw.shape == up_qw.shape and _plain_bf16(x, gate_qw)):
         return None
     return K.int4_gemm_swiglu(gate_qw, gate_sc, up_qw, up_sc, x)

@@ -55,7 +55,7 @@ def test_gate_up_tile_edges(m, n, k, odd):
     assert bool(((guard[:m * n].view(m, n).double() - s * u).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("rows", [1, 2, 64, 65, 512, 513])
+@pytest.mark.parametrize("rows", [1, 2, 64, 65, 512, 513, 768, 769])
 def test_dense_route_equals_the_separate_products(rows):
     """StreamingDIPMlp._dense over its dispatch lines against silu(gate) * up of
     the separate routes; inputs the kernel may not stand in for keep them."""

@@ -83,7 +83,7 @@ def test_gemm_t_non_finite_scales():
 
 
 def test_transposed_route_for_longer_prompts():
-    """65 to 768 bf16 rows take the kernel; what it could not stand in for goes
+    """65 to 512 bf16 rows (768 of a large matrix) take the kernel; what it could not stand in for goes
     through torch's matmul, as it did."""
     import torch.autograd.forward_ad as fwd
     import qlinear as Q
@@ -92,7 +92,7 @@ def test_transposed_route_for_longer_prompts():
     sc = dev_bf16(O.f32_to_bf16(rng.uniform(0.001, 0.01, (512, 2)).astype(np.float32)))
     w = Q.dequantize(qw, sc)
     g = torch.Generator(device="cuda").manual_seed(1)
-    for rows in (65, 300, 768, 769):
+    for rows in (65, 300, 512, 513, 768, 769):
         x = torch.randn(rows, 1024, device="cuda", generator=g).to(torch.bfloat16)
         for v in (x[:, :512], x[:, ::2], x[:, :512].reshape(1, rows, 512)):
             got, ref = Q.int4_linear_t(v, qw, sc), v @ w
