@@ -631,7 +631,8 @@ int launch_int4_gemm(const GemmArgs& a, hipStream_t s) {
 // vector instructions to 8 TM MFMAs a slice).  25600 x 5120: 2 tokens 63 -> 32
 // us, 32 tokens 112 -> 39 us, 64 tokens 201 -> 49 us (before: values transposed
 // through LDS a barrier at a time, 64 columns a workgroup), 333 tokens 143 us
-// (dequantize and the library's product: 234), 1024 tokens 418 us (401).
+// (dequantize and the library's product: 233), 768 tokens 263 us (363), 900
+// tokens 515 us (408).
 // ---------------------------------------------------------------------------
 constexpr int kGemmTThreads = 512;
 constexpr int kGemmTCols = 256;  // columns of a workgroup
