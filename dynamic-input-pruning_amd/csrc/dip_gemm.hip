@@ -71,6 +71,13 @@ constexpr int kXcds = 8;  // workgroups go to the 8 XCDs round-robin
 // ---------------------------------------------------------------------------
 constexpr int kScaleRegs = 5;  // scale dwords a thread holds before the first barrier
 
+// Between LDS accesses of one wave's lanes that depend on each other: the LDS
+// keeps a wave's order by itself, this holds the compiler to it.
+DIP_DEV void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // A workgroup's scales, staged in LDS by dwords: the run of its n values of one
 // matrix or (GU) of the gate, and at `stride` (even) that of up.
 template <bool GU>
@@ -165,6 +172,7 @@ __global__ __launch_bounds__(KS * 64, 2) void int4_gemm_split_kernel(
 #pragma unroll
       for (int u = 0; u < RW; ++u) load_w(d, u, min(ks + d * KS, glast));
     stage_x();
+    wave_lds_order();
   }
   if constexpr (SCL) {
 #pragma unroll
@@ -225,7 +233,11 @@ __global__ __launch_bounds__(KS * 64, 2) void int4_gemm_split_kernel(
                 if (u0 + q < RW)
                   v[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                       xa[t][j], b[q][j], j ? v[q][t] : c[t], 0, 0, 0);
-          if (u0 + UB >= RW) stage_x();  // the next group's tile over this one's
+          if (u0 + UB >= RW) {  // the next group's tile over this one's
+            wave_lds_order();
+            stage_x();
+            wave_lds_order();
+          }
 #pragma unroll
           for (int q = 0; q < UB; ++q)
 #pragma unroll
