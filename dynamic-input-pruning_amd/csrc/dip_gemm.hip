@@ -13,7 +13,8 @@
 //   * v_mfma_f32_16x16x32_bf16 sums (24 + q) * x over one 128-column group in
 //     fp32, starting from -24 * sum(x) of the group, which the same MFMA gives
 //     with a constant operand: the result is sum(q * x), scaled by the group's
-//     scale into the fp32 total.
+//     scale into the fp32 total.  (Tokens that leave fp32's range on the way
+//     are computed from plain q * s: plain_dot.)
 // So the weights enter exactly as q * s in fp32 (the reference rounds q * s
 // to bf16 first); the output is rounded to bf16 once.
 #include <algorithm>
@@ -97,6 +98,52 @@ struct ScaleRun {
     return e + 1 < n ? *reinterpret_cast<const uint32_t*>(p + e) : e < n ? p[e] : 0u;
   }
 };
+
+// An output from plain q * s, by one lane: for tokens that 24 * sum(x) takes out
+// of fp32's range (an infinite x, or values near the largest), whose sums above
+// are not finite and stay so whatever follows.  A kernel's last step looks at
+// its sums (one compare each: 333 tokens through a 12288 x 4096 MLP stay within
+// 0.5 %), and the lanes that hold such a one come here for their outputs that are
+// not finite, so other tokens keep their bits.  A sum that is NaN ends the walk.
+DIP_DEV float plain_dot(const int8_t* qw, const uint16_t* sc, const uint16_t* x, int row, int tok,
+                        int K) {
+  const int ngroups = K >> 7;
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(qw + (size_t)row * (K >> 1));
+  const uint4* xv = reinterpret_cast<const uint4*>(x + (size_t)tok * K);
+  float acc = 0.f;
+  for (int g = 0; g < ngroups && acc == acc; ++g) {
+    const float s = bf16_to_f32(sc[(size_t)row * ngroups + g]);
+    float v = 0.f;
+#pragma unroll 2
+    for (int d = 0; d < 16; ++d) {
+      const uint32_t q = w[16 * g + d];
+      const uint4 p = xv[16 * g + d];
+      const uint32_t px[4] = {p.x, p.y, p.z, p.w};
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        v = fmaf((float)(int)__builtin_amdgcn_sbfe(q, 4 * i, 4) * s,
+                 bf16_to_f32(i & 1 ? px[i / 2] >> 16 : px[i / 2] & 0xFFFFu), v);
+    }
+    acc += v;
+  }
+  return acc;
+}
+
+DIP_DEV bool not_finite(float v) { return __builtin_amdgcn_classf(v, 0x207); }  // NaN, inf
+
+// The output of (tok, row) again from plain q * s if the stored one, this lane's
+// own, is not finite.  (With gate and up: whichever of the two was not finite, the
+// stored product is not either, silu(-inf) being NaN.)
+template <bool GU>
+DIP_DEV void redo_output(const int8_t* qw, const uint16_t* sc, const int8_t* qw_up,
+                         const uint16_t* sc_up, const uint16_t* x, uint16_t* out, int N, int K,
+                         int row, int tok) {
+  uint16_t* o = out + (size_t)tok * N + row;
+  if (!not_finite(bf16_to_f32(*o))) return;
+  uint32_t v = f32_to_bf16(plain_dot(qw, sc, x, row, tok, K));
+  if constexpr (GU) v = swiglu_bf16(v, f32_to_bf16(plain_dot(qw_up, sc_up, x, row, tok, K)));
+  *o = (uint16_t)v;
+}
 
 template <int TM, int RW, int KS, int D, bool SCL, bool GU>
 __global__ __launch_bounds__(KS * 64, 2) void int4_gemm_split_kernel(
@@ -262,10 +309,12 @@ __global__ __launch_bounds__(KS * 64, 2) void int4_gemm_split_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) red[(ks * F + (u * TM + t) * 4 + r) * 64] = acc[u][t][r];
   __syncthreads();
+  bool bad = false;
   auto sum = [&](int f) {
     float v = red[f * 64];
 #pragma unroll
     for (int k = 1; k < KS; ++k) v += red[(k * F + f) * 64];
+    bad |= not_finite(v);
     return f32_to_bf16(v);
   };
   for (int f = ks; f < (GU ? F / 2 : F); f += KS) {
@@ -275,6 +324,13 @@ __global__ __launch_bounds__(KS * 64, 2) void int4_gemm_split_kernel(
     const uint32_t v = GU ? swiglu_bf16(sum(fu), sum(fu + 4 * TM)) : sum(fu);
     if (tok < M && l16 < N) out[(size_t)tok * N + tile_row(u) + l16] = (uint16_t)v;
   }
+  if (bad && l16 < N)
+    for (int f = ks; f < (GU ? F / 2 : F); f += KS) {
+      const int r = f & 3, t = (f >> 2) % TM, u = (f >> 2) / TM * (GU ? 2 : 1);
+      const int tok = tok0 + 16 * t + 4 * kb + r;
+      if (tok < M)
+        redo_output<GU>(qw, sc, qw_up, sc_up, x, out, N, K, tile_row(u) + l16, tok);
+    }
 }
 
 constexpr size_t split_lds_bytes(int tm, int rw, int ks, int scale_groups) {
@@ -550,6 +606,7 @@ __global__ __launch_bounds__(KS * 256, 2) void int4_gemm_kernel(
           for (int r = 0; r < 4; ++r)
             acc[u][t][r] += red[((4 * (k - 1) + wr) * F + (u * TM + t) * 4 + r) * 64];
   }
+  bool bad = false;
 #pragma unroll
   for (int t = 0; t < TM; ++t)
 #pragma unroll
@@ -559,10 +616,21 @@ __global__ __launch_bounds__(KS * 256, 2) void int4_gemm_kernel(
 #pragma unroll
         for (int u = 0; u < RW; u += GU ? 2 : 1) {
           uint32_t v = f32_to_bf16(acc[u][t][r]);
-          if constexpr (GU) v = swiglu_bf16(v, f32_to_bf16(acc[u + 1][t][r]));
+          bad |= not_finite(acc[u][t][r]);
+          if constexpr (GU) {
+            v = swiglu_bf16(v, f32_to_bf16(acc[u + 1][t][r]));
+            bad |= not_finite(acc[u + 1][t][r]);
+          }
           out[(size_t)tok * N + tile_row(u) + l16] = (uint16_t)v;
         }
       }
+    }
+  if (bad)  // (a lane whose l16 is no row has not looked)
+    for (int e = 0; e < TM * 4 * RW; e += GU ? 2 : 1) {
+      const int u = e % RW, tr = e / RW;
+      const int tok = tok0 + 16 * (tr >> 2) + 4 * kb + (tr & 3);
+      if (tok < M)
+        redo_output<GU>(qw, sc, qw_up, sc_up, x, out, N, K, tile_row(u) + l16, tok);
     }
 }
 
