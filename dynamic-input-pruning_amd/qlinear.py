@@ -55,13 +55,18 @@ GATE_UP_MAX_TOKENS = 768
 GEMM_T_MAX_TOKENS = 768
 GEMM_T_SHORT_TOKENS = 512
 GEMM_T_LONG_VALUES = 100_000_000
+# What the kernels are built for, where the dequantised product has no such limit:
+# columns of a row, and rows of a matrix dequantised to its transpose.
+_MAX_COLS = 1 << 20
+_MAX_DEQUANT_T_ROWS = 65535 * 128
 
 
 def _plain_bf16(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Whether x is a plain bf16 tensor beside `weight` that nothing
+    """Whether x is a plain bf16 tensor beside `weight` on the device that nothing
     differentiates, batches or traces: what a kernel called on its data may
     take in place of torch ops."""
-    return (type(x) is torch.Tensor and x.dtype == torch.bfloat16 and x.device == weight.device
+    return (type(x) is torch.Tensor and x.dtype == torch.bfloat16 and x.is_cuda
+            and x.device == weight.device
             and not (x.requires_grad and torch.is_grad_enabled())
             and not torch._C._functorch.is_functorch_wrapped_tensor(x)
             and torch.autograd.forward_ad._current_level < 0
@@ -82,7 +87,7 @@ def int4_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor) ->
             y = y.to(x.dtype)
         return y.view(*x.shape[:-1], qweight.shape[0])
     if 1 < rows <= _ANY_INPUT_TOKENS or (1 < rows <= GEMM_MAX_TOKENS and x.shape[-1] == in_f
-                                         and _plain_bf16(x, qweight)):
+                                         and in_f <= _MAX_COLS and _plain_bf16(x, qweight)):
         if x.dtype is torch.bfloat16 and x.shape[-1] == in_f:
             return K.int4_gemm(qweight, scales, x)
         y = K.int4_gemm(qweight, scales, x.reshape(rows, in_f).to(torch.bfloat16))
@@ -100,9 +105,11 @@ def int4_linear_t(x: torch.Tensor, qweight_t: torch.Tensor, scales_t: torch.Tens
     rows = x.numel() // x.shape[-1]
     most = (GEMM_T_MAX_TOKENS if 2 * qweight_t.numel() >= GEMM_T_LONG_VALUES
             else GEMM_T_SHORT_TOKENS)
-    if rows <= _ANY_INPUT_TOKENS or (rows <= most and _plain_bf16(x, qweight_t)):
+    in_f, by8 = qweight_t.shape[0], qweight_t.shape[0] % 8 == 0
+    if rows <= _ANY_INPUT_TOKENS or (rows <= most and by8 and 2 * qweight_t.shape[1] <= _MAX_COLS
+                                     and _plain_bf16(x, qweight_t)):
         return K.int4_gemm_t(qweight_t, scales_t, x.to(torch.bfloat16)).to(x.dtype)
-    if qweight_t.is_cuda and qweight_t.shape[0] % 8 == 0:
+    if qweight_t.is_cuda and by8 and in_f <= _MAX_DEQUANT_T_ROWS:
         return F.linear(x, K.dequant_t(qweight_t, scales_t).to(x.dtype))
     return x @ dequantize(qweight_t, scales_t).to(x.dtype)
 
@@ -122,7 +129,7 @@ def int4_gate_up(x, gate_qw, gate_sc, up_qw, up_sc):
     import _dip_hip as K
     in_f = gate_qw.shape[1] * 2
     rows = x.numel() // in_f
-    if not (1 < rows <= GATE_UP_MAX_TOKENS and x.shape[-1] == in_f
+    if not (1 < rows <= GATE_UP_MAX_TOKENS and x.shape[-1] == in_f and in_f <= _MAX_COLS
             and gate_qw.shape == up_qw.shape and _plain_bf16(x, gate_qw)):
         return None
     return K.int4_gemm_swiglu(gate_qw, gate_sc, up_qw, up_sc, x)
