@@ -61,16 +61,32 @@ _MAX_COLS = 1 << 20
 _MAX_DEQUANT_T_ROWS = 65535 * 128
 
 
+def _torch_watched() -> bool:
+    """Whether the torch ops of a call would do more than compute: an active
+    dispatch or function mode sees them (a default device, itself such a mode,
+    does not count), or autocast gives their results another type than bf16."""
+    if torch._C._len_torch_dispatch_stack():
+        return True
+    if torch._C._len_torch_function_stack():
+        from torch.overrides import _get_current_function_mode_stack
+        from torch.utils._device import DeviceContext
+        if any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()):
+            return True
+    return (torch.is_autocast_enabled("cuda")
+            and torch.get_autocast_dtype("cuda") != torch.bfloat16)
+
+
 def _plain_bf16(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether x is a plain bf16 tensor beside `weight` on the device that nothing
-    differentiates, batches or traces: what a kernel called on its data may
-    take in place of torch ops."""
+    differentiates, batches, traces or watches: what a kernel called on its data
+    may take in place of torch ops."""
     return (type(x) is torch.Tensor and x.dtype == torch.bfloat16 and x.is_cuda
             and x.device == weight.device
             and not (x.requires_grad and torch.is_grad_enabled())
             and not torch._C._functorch.is_functorch_wrapped_tensor(x)
             and torch.autograd.forward_ad._current_level < 0
-            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+            and not _torch_watched())
 
 
 def int4_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor) -> torch.Tensor:

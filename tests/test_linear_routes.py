@@ -20,6 +20,13 @@ def _x(rows, cols, device="cpu"):
     return torch.randn(rows, cols, generator=g).to(torch.bfloat16).to(device)
 
 
+def _mlp(H=256, I=512):
+    from dip_stream_predispatch import SharedBuffers, StreamingDIPMlp
+    shared = SharedBuffers(300, H // 2, H // 128, H, H // 128, "cuda:0")
+    w = [t for i in range(3) for t in _weight(I, H, i)]
+    return StreamingDIPMlp(*w, shared, 0.6, "cuda:0", down_transposed=True)
+
+
 @pytest.mark.parametrize("rows", [65, 200, 512, 513, 768])
 def test_host_tensors_take_the_dequantised_product(rows):
     import qlinear as Q
@@ -40,3 +47,60 @@ def test_shapes_without_a_kernel_keep_their_product(rows):
     qw, sc = _weight(260, 256, device="cuda")
     x = _x(rows, 260, "cuda")
     assert torch.equal(Q.int4_linear_t(x, qw, sc), x @ Q.dequantize(qw, sc))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [65, 300, 600])
+def test_autocast_decides_the_type(rows):
+    """Under autocast the product is torch's, in autocast's type."""
+    import qlinear as Q
+    print(f"autocast, {rows} rows", flush=True)
+    qw, sc = _weight(384, 256, device="cuda")
+    w, x, xt = Q.dequantize(qw, sc), _x(rows, 256, "cuda"), _x(rows, 384, "cuda")
+    m = _mlp()
+    for dtype in (torch.float16, torch.bfloat16):
+        with torch.no_grad(), torch.autocast("cuda", dtype=dtype):
+            got, ref = Q.int4_linear(x, qw, sc), F.linear(x, w)
+            assert got.dtype == ref.dtype == dtype
+            assert float((got - ref).abs().max() / ref.abs().max()) < 1e-2
+            got, ref = Q.int4_linear_t(xt, qw, sc), xt @ w
+            assert got.dtype == ref.dtype == dtype
+            assert float((got - ref).abs().max() / ref.abs().max()) < 1e-2
+            assert m(x.view(1, rows, 256)).dtype == dtype
+
+
+@pytest.mark.gpu
+def test_modes_see_the_product():
+    """A dispatch or function mode sees torch's product; a default device is no
+    such mode."""
+    import _dip_hip as K
+    import qlinear as Q
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    print("modes", flush=True)
+    seen = []
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func.name())
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", str(func)))
+            return func(*args, **(kwargs or {}))
+
+    qw, sc = _weight(384, 256, device="cuda")
+    x, xt, m = _x(100, 256, "cuda"), _x(100, 384, "cuda"), _mlp()
+    for mode, product in ((Dispatch, "mm"), (Function, "linear")):
+        for f in (lambda: Q.int4_linear(x, qw, sc), lambda: m(x.view(1, 100, 256))):
+            seen.clear()
+            with torch.no_grad(), mode():
+                f()
+            assert any(product in s for s in seen), (mode, seen)
+    seen.clear()
+    with torch.no_grad(), Dispatch():
+        Q.int4_linear_t(xt, qw, sc)
+    assert any("mm" in s for s in seen)
+    with torch.no_grad(), torch.device("cuda"):
+        assert torch.equal(Q.int4_linear(x, qw, sc), K.int4_gemm(qw, sc, x))
