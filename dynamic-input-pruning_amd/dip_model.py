@@ -397,7 +397,9 @@ class DIPDecoder:
                 or M._global_forward_hooks or M._global_forward_pre_hooks:
             return False
         inner = self.model.model
-        passed = [self.model, inner, inner.norm, inner.rotary_emb, self.model.lm_head]
+        # (the embedding runs, but what it returns becomes the residual)
+        passed = [self.model, inner, inner.embed_tokens, inner.norm, inner.rotary_emb,
+                  self.model.lm_head]
         for L in self.layers:
             a = L.self_attn
             if not isinstance(L.mlp, (StreamingDIPMlp, CADIPMlp)) or \
@@ -416,7 +418,7 @@ class DIPDecoder:
         from qlinear import int4_linear
         K, inner, hd, nh = self._K, self.model.model, self.hd, self.nh
         plen = ids.shape[1]
-        h = inner.embed_tokens(ids).view(plen, self.hidden)
+        h = inner.embed_tokens(ids).view(plen, self.hidden)  # from here on the residual, in place
         x = torch.empty_like(h)
         q = torch.empty(plen, nh * hd, dtype=self.dtype, device=self.device)
         y = None
@@ -431,8 +433,9 @@ class DIPDecoder:
                 q.view(1, plen, nh, hd).transpose(1, 2), kc[None, :, :plen], vc[None, :, :plen],
                 is_causal=plen > 1, scale=a.scaling, enable_gqa=nh != self.nkv)
             o = a.o_proj(o.transpose(1, 2).reshape(1, plen, nh * hd))
-            K.add_rmsnorm_rows(h, o.reshape(plen, -1), pn.weight, x, pn.variance_epsilon)
-            y = L.mlp(x.view(1, plen, -1)).reshape(plen, -1)
+            m = torch.empty_like(h)  # the MLP's alone: who calls it may keep it
+            K.add_rmsnorm_rows(h, o.reshape(plen, -1), pn.weight, m, pn.variance_epsilon)
+            y = L.mlp(m.view(1, plen, -1)).reshape(plen, -1)
         n = inner.norm
         last = torch.empty(self.hidden, dtype=self.dtype, device=self.device)
         K.add_rmsnorm(h[-1], y[-1], n.weight, last, n.variance_epsilon)

@@ -76,3 +76,89 @@ def test_fused_prefill_matches_hf_forward(tmp_path, kv_heads, tokens):
             for a, b in ((got, ref), (kc, dec.k_cache), (vc, dec.v_cache))]
     print(f"  max_rel {errs}", flush=True)
     assert got.shape == ref.shape and max(errs) < 2e-2
+
+
+def _decoder(tmp_path, kv_heads=2, seed=3, **kw):
+    from dip_model import DIPDecoder
+    from dip_stream_predispatch import load_streaming_dip
+    cfg = tiny_config(hidden=512, inter=1024, heads=4, kv_heads=kv_heads, head_dim=128, vocab=512,
+                      max_pos=1024)
+    write_checkpoint(tiny_model(cfg, seed=seed), tmp_path)
+    model, _, _ = load_streaming_dip(tmp_path, keep_ratio=0.6)
+    return DIPDecoder(model, 600, **kw)
+
+
+def _ids(tokens):
+    return torch.randint(0, 512, (1, tokens), generator=torch.Generator().manual_seed(9))
+
+
+def _fused_against_hf(dec, ids):
+    """max_rel of the logits and caches of the two prefills."""
+    assert dec.fused and dec._prefill_fusible()
+    got, kc, vc = dec.prefill(ids), dec.k_cache.clone(), dec.v_cache.clone()
+    assert int(dec.pos) == ids.shape[1] and int(dec.tok) == int(got.argmax())
+    handle = dec.model.model.norm.register_forward_hook(lambda *a: None)
+    ref = dec.prefill(ids)
+    handle.remove()
+    return max(max_rel(a.float(), b.float())
+               for a, b in ((got, ref), (kc, dec.k_cache), (vc, dec.v_cache)))
+
+
+@pytest.mark.parametrize("tokens", [1, 2])
+def test_fused_prefill_of_one_token(tmp_path, tokens):
+    """One token takes the modules' decode step on both routes.  There the top-k
+    picks channels, and a swapped one moves the logits by more than rounding: the
+    bound is the sparse decode's against the modules, 8e-2."""
+    print(f"prefill {tokens} token(s)", flush=True)
+    assert _fused_against_hf(_decoder(tmp_path), _ids(tokens)) < (8e-2 if tokens == 1 else 2e-2)
+
+
+@pytest.mark.parametrize("tokens", [1, 40, 300])
+@pytest.mark.parametrize("resident", [False, True])
+def test_fused_prefill_of_a_cache_aware_model(tmp_path, tokens, resident):
+    from dip_ca import load_dip_ca
+    from dip_model import DIPDecoder
+    print(f"cache-aware prefill {tokens} tokens, resident channels {resident}", flush=True)
+    cfg = tiny_config(hidden=512, inter=1024, heads=4, kv_heads=2, head_dim=128, vocab=512,
+                      max_pos=1024)
+    write_checkpoint(tiny_model(cfg, seed=4), tmp_path)
+    model, _, cas = load_dip_ca(tmp_path, keep_ratio=0.6, cache_frac=0.3)
+    if resident:
+        for c in cas:
+            c.set_cache(torch.randperm(c.inter, generator=torch.Generator().manual_seed(1)))
+    dec = DIPDecoder(model, 600, use_graph=False)
+    sparse = tokens == 1 and resident
+    assert _fused_against_hf(dec, _ids(tokens)) < (8e-2 if sparse else 2e-2)
+
+
+@pytest.mark.parametrize("what", ["hooks", "wrapped forward"])
+@pytest.mark.parametrize("whose", ["embedding", "layers"])
+def test_kept_inputs_and_outputs_stay_as_they_were(tmp_path, what, whose):
+    """Whoever keeps what the embedding, the MLPs and the o projections take and
+    give finds it unchanged after the prompt; the layers' keep the fused route."""
+    print(f"prefill with kept tensors: {what} of the {whose}", flush=True)
+    dec = _decoder(tmp_path)
+    inner = dec.model.model
+    mods = ([inner.embed_tokens] if whose == "embedding" else
+            [m for L in inner.layers for m in (L.mlp, L.self_attn.o_proj)])
+    kept = []
+
+    def keep(*tensors):
+        kept.extend((t, t.clone()) for t in tensors)
+
+    handles = []
+    for m in mods:
+        if what == "hooks":
+            handles.append(m.register_forward_hook(lambda mod, a, out: keep(a[0], out)))
+        else:
+            def forward(x, f=m.forward):
+                out = f(x)
+                keep(x, out)
+                return out
+            m.forward = forward
+    assert dec._prefill_fusible() == (whose == "layers")
+    dec.prefill(_ids(65))
+    assert len(kept) == 2 * len(mods)
+    assert all(torch.equal(t, was) for t, was in kept)
+    for h in handles:
+        h.remove()
