@@ -308,6 +308,10 @@ class DIPDecoder:
         self._qkv_w = []
         for L in self.layers:
             a = L.self_attn
+            joined = self._qkv_joined(a)
+            if joined is not None:
+                self._qkv_w.append(joined)
+                continue
             parts = (a.q_proj, a.k_proj, a.v_proj)
             qw = torch.cat([p.qweight for p in parts])
             sc = torch.cat([p.scales for p in parts])
@@ -339,6 +343,7 @@ class DIPDecoder:
         # (one workgroup per kv head); longer ones split the cache over many
         # workgroups (three launches)
         self._attn_one_launch = self.max_len <= K.decode_attention_fused_max_len()
+        self._passed = self._passed_by()
 
     def _body_fused(self) -> torch.Tensor:
         K = self._K
@@ -389,26 +394,81 @@ class DIPDecoder:
     def _prefill_fusible(self) -> bool:
         """Whether a prompt may pass by the HF modules around the projections
         and MLPs: the attention is the one _prefill_fused makes, without
-        dropout, and nobody observes or replaced a module it passes by."""
+        dropout; the modules it passes by are the published ones, with the
+        weights they had when this decoder was made, and nobody hooks them; and
+        no mode or autocast acts on their torch ops."""
+        from torch.nn.modules import module as M
         from dip_ca import CADIPMlp
         from dip_stream_predispatch import StreamingDIPMlp
-        from torch.nn.modules import module as M
-        if getattr(self.model.config, "_attn_implementation", None) != "sdpa" \
-                or M._global_forward_hooks or M._global_forward_pre_hooks:
+        from qlinear import _torch_watched
+        if not self._passed or getattr(self.model.config, "_attn_implementation", None) != "sdpa" \
+                or M._global_forward_hooks or M._global_forward_pre_hooks or _torch_watched():
             return False
+        classes, modules, buffers = self._passed
+        return (all(cls.forward is fwd for cls, fwd in classes.items())
+                and len(self.model.model.layers) == len(self.layers)
+                and all(parent.get(name) is m and type(m) is cls and not m._forward_hooks
+                        and not m._forward_pre_hooks and "forward" not in m.__dict__
+                        for parent, name, m, cls in modules)
+                and all(parent.get(name) is t for parent, name, t in buffers)
+                and all(isinstance(L.mlp, (StreamingDIPMlp, CADIPMlp))
+                        and not (L.self_attn.training and L.self_attn.attention_dropout)
+                        for L in self.layers))
+
+    def _passed_by(self):
+        """What _prefill_fused stands in for: the forward of each class, the
+        modules (and the embedding, whose output it takes over) and the
+        projections' weights, each with where it hangs; None where one is not of
+        the class it knows, or that class's forward is not its own."""
+        from transformers.models.qwen3 import modeling_qwen3 as Q
+        from qlinear import QuantLinear
         inner = self.model.model
-        # (the embedding runs, but what it returns becomes the residual)
-        passed = [self.model, inner, inner.embed_tokens, inner.norm, inner.rotary_emb,
-                  self.model.lm_head]
-        for L in self.layers:
+        found = [({"": self.model}, "", Q.Qwen3ForCausalLM), (self.model._modules, "model", Q.Qwen3Model),
+                 (self.model._modules, "lm_head", nn.Linear),
+                 (inner._modules, "embed_tokens", nn.Embedding),
+                 (inner._modules, "norm", Q.Qwen3RMSNorm),
+                 (inner._modules, "rotary_emb", Q.Qwen3RotaryEmbedding),
+                 (inner._modules, "layers", nn.ModuleList)]
+        buffers = []
+        for i, L in enumerate(self.layers):
             a = L.self_attn
-            if not isinstance(L.mlp, (StreamingDIPMlp, CADIPMlp)) or \
-                    (a.training and getattr(a, "attention_dropout", 0)):
-                return False
-            passed += [L, L.input_layernorm, L.post_attention_layernorm, a, a.q_norm, a.k_norm,
-                       a.q_proj, a.k_proj, a.v_proj]
-        return not any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__
-                       for m in passed)
+            found += [(inner.layers._modules, str(i), Q.Qwen3DecoderLayer),
+                      (L._modules, "input_layernorm", Q.Qwen3RMSNorm),
+                      (L._modules, "post_attention_layernorm", Q.Qwen3RMSNorm),
+                      (L._modules, "self_attn", Q.Qwen3Attention),
+                      (a._modules, "q_norm", Q.Qwen3RMSNorm),
+                      (a._modules, "k_norm", Q.Qwen3RMSNorm)]
+            for p in ("q_proj", "k_proj", "v_proj"):
+                found.append((a._modules, p, QuantLinear))
+                buffers += [(getattr(a, p)._buffers, n, getattr(a, p)._buffers[n])
+                            for n in ("qweight", "scales")]
+        modules = [(d, n, d.get(n), cls) for d, n, cls in found]
+        classes = {cls: cls.forward for _, _, _, cls in modules}
+        if any(type(m) is not cls for _, _, m, cls in modules) or any(
+                f.__module__ != cls.__module__ for cls, f in classes.items()
+                if cls is not nn.ModuleList):
+            return None
+        return classes, modules, buffers
+
+    @staticmethod
+    def _qkv_joined(a):
+        """The q, k and v projections' weights as one aligned [q|k|v] matrix and
+        its scales where they are the rows of one already (another decoder of
+        the model joined them), else None."""
+        out = []
+        for name in ("qweight", "scales"):
+            ts = [getattr(p, name) for p in (a.q_proj, a.k_proj, a.v_proj)]
+            q, end = ts[0], ts[0].data_ptr()
+            if end % 16:
+                return None
+            for t in ts:
+                if (t.shape[1:] != q.shape[1:] or t.dtype != q.dtype or not t.is_contiguous()
+                        or t.data_ptr() != end
+                        or t.untyped_storage().data_ptr() != q.untyped_storage().data_ptr()):
+                    return None
+                end += t.numel() * t.element_size()
+            out.append(q.as_strided((sum(t.shape[0] for t in ts), q.shape[1]), q.stride()))
+        return tuple(out)
 
     def _prefill_fused(self, ids: torch.Tensor) -> torch.Tensor:
         """prefill with the decode kernels' prompt forms around the

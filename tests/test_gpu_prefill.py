@@ -162,3 +162,121 @@ def test_kept_inputs_and_outputs_stay_as_they_were(tmp_path, what, whose):
     assert all(torch.equal(t, was) for t, was in kept)
     for h in handles:
         h.remove()
+
+
+def _replacements():
+    import torch.nn as nn
+    from transformers.models.qwen3 import modeling_qwen3 as Q
+
+    class Wrapped(nn.Module):  # an adapter, a probe: anything around a module
+        def __init__(self, inner, calls):
+            super().__init__()
+            self.inner, self.calls = inner, calls
+
+        def __getattr__(self, name):
+            try:
+                return super().__getattr__(name)
+            except AttributeError:
+                return getattr(super().__getattr__("inner"), name)
+
+        def forward(self, *a, **kw):
+            self.calls.append(1)
+            return self.inner(*a, **kw)
+
+    def swap(parent, name):
+        def do(dec, calls, monkeypatch):
+            p = parent(dec)
+            setattr(p, name, Wrapped(getattr(p, name), calls))
+        return do
+
+    def layer(dec, calls, monkeypatch):
+        dec.model.model.layers[1] = Wrapped(dec.model.model.layers[1], calls)
+
+    def class_forward(cls):
+        def do(dec, calls, monkeypatch):
+            orig = cls.forward
+
+            def forward(self, *a, **kw):
+                calls.append(1)
+                return orig(self, *a, **kw)
+            monkeypatch.setattr(cls, "forward", forward)
+        return do
+
+    def subclass(dec, calls, monkeypatch):
+        norm = dec.model.model.layers[0].input_layernorm
+
+        class Other(type(norm)):
+            def forward(self, x):
+                calls.append(1)
+                return super().forward(x)
+        norm.__class__ = Other
+
+    def weights(dec, calls, monkeypatch):
+        p = dec.model.model.layers[1].self_attn.k_proj
+        p.qweight = torch.roll(p.qweight, 1, 0)
+        calls.append(1)
+
+    L0 = lambda dec: dec.model.model.layers[0]
+    A0 = lambda dec: dec.model.model.layers[0].self_attn
+    return {"input norm": swap(L0, "input_layernorm"),
+            "post-attention norm": swap(L0, "post_attention_layernorm"),
+            "q norm": swap(A0, "q_norm"), "k projection": swap(A0, "k_proj"),
+            "attention": swap(L0, "self_attn"), "layer": layer,
+            "final norm": swap(lambda d: d.model.model, "norm"),
+            "embedding": swap(lambda d: d.model.model, "embed_tokens"),
+            "norm class": class_forward(Q.Qwen3RMSNorm),
+            "attention class": class_forward(Q.Qwen3Attention),
+            "layer class": class_forward(Q.Qwen3DecoderLayer),
+            "norm subclass": subclass, "projection weights": weights}
+
+
+@pytest.mark.parametrize("what", ["input norm", "post-attention norm", "q norm", "k projection",
+                                  "attention", "layer", "final norm", "embedding", "norm class",
+                                  "attention class", "layer class", "norm subclass",
+                                  "projection weights"])
+def test_replaced_modules_run(tmp_path, what, monkeypatch):
+    """A module, class method or weight replaced after the decoder was made
+    serves its prompts: the logits are the model's own, now."""
+    print(f"prefill with a replaced {what}", flush=True)
+    dec = _decoder(tmp_path)
+    ids = _ids(65)
+    calls = []
+    _replacements()[what](dec, calls, monkeypatch)
+    assert not calls or what == "projection weights"
+    got = dec.prefill(ids)
+    assert calls
+    with torch.no_grad():
+        ref = dec.model(ids.cuda()).logits[0, -1]
+    assert max_rel(got.float(), ref.float()) < 2e-2
+
+
+def test_prefill_under_modes_runs_the_model(tmp_path):
+    """Autocast to another type and dispatch modes act on the model's own ops."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    print("prefill under modes", flush=True)
+    dec = _decoder(tmp_path)
+    seen = []
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func.name())
+            return func(*args, **(kwargs or {}))
+
+    with Dispatch():
+        dec.prefill(_ids(65))
+    assert any("rsqrt" in s for s in seen)  # the norms
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert not dec._prefill_fusible()
+    assert dec._prefill_fusible()
+
+
+def test_two_decoders_of_one_model(tmp_path):
+    """A second decoder of the model leaves the first one's prompts as they were."""
+    from dip_model import DIPDecoder
+    print("prefill of two decoders", flush=True)
+    first = _decoder(tmp_path)
+    before = first.prefill(_ids(65))
+    second = DIPDecoder(first.model, 300)
+    for dec in (first, second):
+        assert dec._prefill_fusible()
+        assert torch.equal(dec.prefill(_ids(65)), before)
