@@ -353,11 +353,11 @@ struct GemmArgs {
 
 template <int TM, int RW, int KS, int D, bool SCL, bool GU>
 int launch_split(const GemmArgs& a, hipStream_t s) {
-  static const bool lds_ok =
-      hipFuncSetAttribute(
-          reinterpret_cast<const void*>(&int4_gemm_split_kernel<TM, RW, KS, D, SCL, GU>),
-          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemmLds) == hipSuccess;
-  if (!lds_ok) return hip_status(hipGetLastError());
+  static std::atomic<uint64_t> granted{0};
+  if (const int st = allow_lds(
+          granted, reinterpret_cast<const void*>(&int4_gemm_split_kernel<TM, RW, KS, D, SCL, GU>),
+          (int)kGemmLds))
+    return st;
   constexpr int kRows = GU ? 8 * RW : 16 * RW;
   const int row_blocks = (a.N + kRows - 1) / kRows;
   const unsigned grid = (unsigned)row_blocks * (unsigned)((a.M + 16 * TM - 1) / (16 * TM));
@@ -642,10 +642,10 @@ constexpr size_t gemm_lds_bytes(int rw, int ks, int ngroups) {
 
 template <int RW, int KS, bool GU>
 int launch_gemm(const GemmArgs& a, hipStream_t s) {
-  static const bool lds_ok =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&int4_gemm_kernel<RW, KS, GU>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemmLds) == hipSuccess;
-  if (!lds_ok) return hip_status(hipGetLastError());
+  static std::atomic<uint64_t> granted{0};
+  if (const int st = allow_lds(
+          granted, reinterpret_cast<const void*>(&int4_gemm_kernel<RW, KS, GU>), (int)kGemmLds))
+    return st;
   constexpr int kRows = GU ? 32 * RW : 64 * RW;
   const int rbs = (a.N + kRows - 1) / kRows, tbs = (a.M + kTileTokens - 1) / kTileTokens;
   const unsigned grid = (unsigned)((rbs + kXcds - 1) / kXcds * kXcds) * (unsigned)tbs;
@@ -964,10 +964,10 @@ __global__ __launch_bounds__(256) void int4_gemm_t_reduce_kernel(const float* __
 template <int TM>
 int launch_gemm_t(const int8_t* qw, const uint16_t* sc, const uint16_t* x, uint16_t* out, float* part,
                   int M, int N, int K, int splits, int part_slices, hipStream_t s) {
-  static const bool lds_ok =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&int4_gemm_t_kernel<TM>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemmLds) == hipSuccess;
-  if (!lds_ok) return hip_status(hipGetLastError());
+  static std::atomic<uint64_t> granted{0};
+  if (const int st = allow_lds(
+          granted, reinterpret_cast<const void*>(&int4_gemm_t_kernel<TM>), (int)kGemmLds))
+    return st;
   const dim3 grid((unsigned)((N + kGemmTCols - 1) / kGemmTCols), (unsigned)((M + 16 * TM - 1) / (16 * TM)),
                   (unsigned)splits);
   hipLaunchKernelGGL(int4_gemm_t_kernel<TM>, grid, dim3(kGemmTThreads), gemm_t_lds_bytes(TM), s, qw, sc,

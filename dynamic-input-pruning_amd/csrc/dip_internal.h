@@ -5,6 +5,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "../../include/dip_hip.h"
 
 namespace dip {
@@ -171,5 +173,23 @@ int device_cus();
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 inline int hip_status(hipError_t e) { return e == hipSuccess ? DIP_OK : (int)e; }
+
+// Lets `kernel` take up to `bytes` of dynamic LDS on the current device.
+// `granted`, the kernel's own, has a bit for each device that has agreed; one
+// that refused is asked again, and its refusal returned, on every call.
+inline int allow_lds(std::atomic<uint64_t>& granted, const void* kernel, int bytes) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  const uint64_t bit = dev >= 0 && dev < 64 ? (uint64_t)1 << dev : 0;
+  if (e == hipSuccess && (granted.load(std::memory_order_relaxed) & bit)) return DIP_OK;
+  if (e == hipSuccess)
+    e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // returned here, so not again by the next launch's check
+    return (int)e;
+  }
+  granted.fetch_or(bit, std::memory_order_relaxed);
+  return DIP_OK;
+}
 
 }  // namespace dip

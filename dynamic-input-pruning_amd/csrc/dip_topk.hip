@@ -618,19 +618,18 @@ __global__ __launch_bounds__(kThreads) void topk_spec_kernel(
 
 int launch_topk_select(const uint16_t* s, int64_t n, int64_t k, int32_t* idx, void* ws,
                        hipStream_t stream) {
-  static const bool lds_ok = [] {
-    const int bytes = kFineBins * (int)sizeof(uint32_t);
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(&topk_select_kernel<4>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess &&
-           hipFuncSetAttribute(reinterpret_cast<const void*>(&topk_select_kernel<8>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
-  }();
-  if (!lds_ok) return hip_status(hipGetLastError());
+  static std::atomic<uint64_t> granted[2];
+  const bool small = n <= 4 * 8 * kThreads;
+  if (const int st = allow_lds(granted[small ? 0 : 1],
+                               small ? reinterpret_cast<const void*>(&topk_select_kernel<4>)
+                                     : reinterpret_cast<const void*>(&topk_select_kernel<8>),
+                               kFineBins * (int)sizeof(uint32_t)))
+    return st;
   TopkMeta* meta = reinterpret_cast<TopkMeta*>(ws);
   const unsigned blocks = (unsigned)(n > 0 ? (n + kSlice - 1) / kSlice : 1);
   const int stamps = tuning(DIP_TUNE_TOPK_STAMPS);
   const size_t lds = kFineBins * sizeof(uint32_t);
-  if (n <= 4 * 8 * kThreads)
+  if (small)
     hipLaunchKernelGGL((topk_select_kernel<4>), dim3(blocks), dim3(kThreads), lds, stream, s,
                        (int)n, (int)k, idx, meta, stamps);
   else
@@ -644,11 +643,11 @@ namespace {
 template <int R, int LPR, int CH>
 int launch_spec_variant(const uint16_t* s, int n, int k, int32_t* idx, TopkMeta* meta,
                         const SpecArgs& sp, int blocks, hipStream_t stream) {
-  static const bool lds_ok =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&topk_spec_kernel<R, LPR, CH>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize,
-                          kFineBins * (int)sizeof(uint32_t)) == hipSuccess;
-  if (!lds_ok) return hip_status(hipGetLastError());
+  static std::atomic<uint64_t> granted{0};
+  if (const int st = allow_lds(
+          granted, reinterpret_cast<const void*>(&topk_spec_kernel<R, LPR, CH>),
+          kFineBins * (int)sizeof(uint32_t)))
+    return st;
   hipLaunchKernelGGL((topk_spec_kernel<R, LPR, CH>), dim3(blocks), dim3(kThreads),
                      kFineBins * sizeof(uint32_t), stream, s, n, k, idx, meta,
                      tuning(DIP_TUNE_TOPK_STAMPS), sp);
