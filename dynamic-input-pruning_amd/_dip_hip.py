@@ -97,18 +97,17 @@ _SIGS = {
     "dip_timeline_read": ([_i32, _p], _i32),
     "dip_get_tuning": ([_i32], _i32),
 }
+# The argument lists above follow this version of include/dip_hip.h
+# (DIP_VERSION); a library built from another one would be called with
+# shifted arguments, or lack an entry point, so it is refused here.
+ABI_VERSION = 305
+if lib.dip_version() != ABI_VERSION:
+    raise ImportError(f"{LIB_PATH} reports ABI version {lib.dip_version()}, these bindings "
+                      f"are written for {ABI_VERSION}; rebuild the library")
 for _name, (_args, _res) in _SIGS.items():
     _fn = getattr(lib, _name)
     _fn.argtypes = _args
     _fn.restype = _res
-
-# The argument lists above follow this version of include/dip_hip.h
-# (DIP_VERSION); a library built from another one would be called with
-# shifted arguments, so it is refused here.
-ABI_VERSION = 304
-if lib.dip_version() != ABI_VERSION:
-    raise ImportError(f"{LIB_PATH} reports ABI version {lib.dip_version()}, these bindings "
-                      f"are written for {ABI_VERSION}; rebuild the library")
 
 GROUP_SIZE = 128
 

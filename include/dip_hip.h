@@ -52,7 +52,9 @@ const char* dip_status_string(int status);
  * Library version as an integer (major * 10000 + minor * 100 + patch).  The
  * minor number changes whenever an entry point's argument list changes, so
  * a binding written against this header checks dip_version() == DIP_VERSION
- * before its first call.  0.3.4: dip_int4_gather_down_by_channel takes
+ * before its first call.  0.3.5 adds dip_int4_gemm_swiglu, dip_swiglu,
+ * dip_dequant_t, dip_stream_rows, dip_add_rmsnorm_rows and
+ * dip_qk_norm_rope_cache_rows.  0.3.4: dip_int4_gather_down_by_channel takes
  * indices == NULL (every row in order; it was an error).  0.3.3 adds the
  * DIP_TUNE_ROW_TIERS knob (no argument list changes).  0.3.2: the down and decode workspaces grow by
  * 8 KB of arrival counters (the sizes functions report it).  0.3.1 adds
@@ -61,7 +63,7 @@ const char* dip_status_string(int status);
  * down_t_sc_gm to the decode and gather-down entry points and g_len to
  * dip_ca_fused_gemv.
  */
-#define DIP_VERSION 304
+#define DIP_VERSION 305
 int dip_version(void);
 
 /* Highest row count the top-k supports (its keys are staged in LDS). */

@@ -35,6 +35,20 @@ def test_status_strings():
     assert K.lib.dip_topk_max_n() == 65536
 
 
+def test_older_library_is_refused_by_its_version(tmp_path):
+    """A library of another version is refused by that, whatever it exports."""
+    import os
+    import subprocess
+    import sys
+    src, so = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text("int dip_version(void) { return 304; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    r = subprocess.run([sys.executable, "-c", "import _dip_hip"], capture_output=True, text=True,
+                       cwd=os.path.dirname(K.__file__), env=dict(os.environ, DIP_HIP_LIB=str(so)),
+                       timeout=120)
+    assert r.returncode != 0 and "ImportError" in r.stderr and "ABI version 304" in r.stderr
+
+
 def _fake(n=16):
     """An aligned host pointer that is never dereferenced by a rejected call."""
     buf = (ctypes.c_uint8 * (n + 16))()
