@@ -276,6 +276,12 @@ def int4_gemm_swiglu(gate_qw, gate_sc, up_qw, up_sc, x):
     return out
 
 
+def int4_gemm_t_splits(m: int, out_features: int, in_features: int) -> int:
+    """The parts of K that dip_int4_gemm_t adds up in its workspace."""
+    nbytes = lib.dip_int4_gemm_t_workspace_size(m, out_features, in_features)
+    return max(1, nbytes // (4 * m * out_features))
+
+
 def int4_gemm_t(qweight_t, scales_t, x, out=None):
     """out [M, N] = bf16(x [M, K] @ bf16(q*s)) for W stored as K rows of N
     (the transposed down matrix), on bf16 MFMA."""

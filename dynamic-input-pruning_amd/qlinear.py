@@ -22,6 +22,7 @@ resident on one device.
 """
 from __future__ import annotations
 
+import functools
 from pathlib import Path
 
 import torch
@@ -34,31 +35,78 @@ _QUANT_SUBSTRINGS = ("q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_pr
 # 32-column chunks split over 4..32 lanes per row).
 _GEMV_COLS = frozenset((128, 256, 512, 1024, 1536, 2048, 2560, 3072, 4096, 5120, 6144, 8192))
 # Prompts of up to this many tokens run the int4 MFMA GEMM (weights read
-# once as nibbles); longer ones dequantize once and use the library GEMM,
-# which wins once the bf16 copy is amortised over enough tokens (us, int4
-# GEMM against both steps of the library route: 25600 x 5120, 512 tokens 180
-# / 191, 700 tokens 228 / 237, 1024 tokens 313 / 300; 12288 x 4096, 512 tokens
-# 69 / 77, 700 tokens 104 / 95).
+# once as nibbles) where _gemm_serves; longer ones dequantize once and use the
+# library GEMM, which wins once the bf16 copy is amortised over enough tokens
+# (us, int4 GEMM / both steps of the library route, each in a graph over layers
+# that do not fit the caches: 25600 x 5120, 512 tokens 197 / 201, 704 tokens 247 /
+# 263, 900 tokens 322 / 270; 12288 x 4096, 512 tokens 70 / 72, 576 tokens 91 / 80;
+# 9728 x 2560, 512 tokens 44 / 47, 640 tokens 58 / 50).
 GEMM_MAX_TOKENS = 512
 # Up to this many rows it takes any input, rounded to bf16; beyond, plain bf16
 # tensors only (_plain_bf16).
 _ANY_INPUT_TOKENS = 64
-# Gate and up in one launch win a little longer (us, against both library
-# products, their dequantisation and the SwiGLU: 25600 x 5120, 512 tokens 338 /
-# 412, 768 tokens 463 / 510, 900 tokens 552 / 535; 12288 x 4096, 512 tokens 135 /
-# 153, 640 tokens 178 / 171, 768 tokens 193 / 202, 900 tokens 226 / 209).
+# Gate and up in one launch win a little longer, whatever the shape (us, against
+# both library products, their dequantisation and the SwiGLU, at 512 / 704 / 768 /
+# 900 tokens: 25600 x 5120 374 / 426, 486 / 545, 512 / 539, 622 / 569; 12288 x 4096
+# 145 / 164, 201 / 211, 210 / 201, 250 / 227; 9728 x 2560 74 / 101, 107 / 118, 124 /
+# 124, 135 / 143; 3072 x 1024 18 / 41, 23 / 42, 24 / 42, 24 / 45.  Over ten shapes and
+# 65 to 768 tokens the one launch is at most 8 % behind, at 17408 x 5120 and 768).
 GATE_UP_MAX_TOKENS = 768
-# The transposed GEMM's limits, for a matrix of GEMM_T_LONG_VALUES weights or
-# more and for smaller ones (us, against dequantize and the library's product:
-# 25600 x 5120, 512 tokens 211 / 339, 768 tokens 263 / 363, 900 tokens 515 / 408;
-# 12288 x 4096, 512 tokens 79 / 92, 576 tokens 125 / 104, 768 tokens 126 / 106).
+# The transposed GEMM's limits, for a K of GEMM_T_LONG_ROWS or more, over which the
+# library's product does not fill the chip (768 tokens, dequantize and product:
+# 25600 x 5120 371 us, 17408 x 5120 242, 2.7 us per million weights), and for
+# shorter ones (14336 x 4096 128 us, 2.2 per million).  Within them _gemm_t_serves.
 GEMM_T_MAX_TOKENS = 768
 GEMM_T_SHORT_TOKENS = 512
-GEMM_T_LONG_VALUES = 100_000_000
+GEMM_T_LONG_ROWS = 16384
 # What the kernels are built for, where the dequantised product has no such limit:
 # columns of a row, and rows of a matrix dequantised to its transpose.
 _MAX_COLS = 1 << 20
 _MAX_DEQUANT_T_ROWS = 65535 * 128
+
+
+@functools.lru_cache(maxsize=None)
+def _cus(device_index: int) -> int:
+    return torch.cuda.get_device_properties(device_index).multi_processor_count
+
+
+def _gemm_serves(rows: int, out_f: int, in_f: int, cus: int) -> bool:
+    """Whether the int4 GEMM beats dequantize + the library for 65 rows or more.
+    Its workgroups are 128 weight rows x 64 tokens.  Just past one to a CU they
+    lose their second part of K, and a CU with one of them waits on memory:
+    beyond 256 tokens the library is faster there (us, 448 tokens: 5120 x 8192,
+    280 workgroups, 87 / 72; 5120 x 25600, 280, 363 / 328; 6144 x 4096, 336, 46 /
+    43), but for a short K (384 tokens: 6144 x 2048, 288 workgroups, 26 / 31; 9728 x
+    2560, 456, 34 / 42).  At 1.5 to a CU the two are level (10240 x 5120, 384 tokens,
+    480 workgroups, 63 / 69), and up to one the GEMM wins (5120 x 8192, 384
+    tokens, 240 workgroups, 51 / 65)."""
+    if rows > GEMM_MAX_TOKENS:
+        return False
+    workgroups = -(-out_f // 128) * -(-rows // 64)
+    return rows <= 256 or in_f < 4096 or not cus < workgroups <= 1.5 * cus
+
+
+def _gemm_t_serves(rows: int, in_f: int, out_f: int, splits: int, cus: int) -> bool:
+    """Whether the transposed int4 GEMM, in `splits` parts of K, beats
+    dequantize + the library for 65 rows or more.  Its workgroups (256 columns x
+    64 tokens x a part) run in rounds of one to a CU, 11 ns per row of K each, so
+    a round that is nearly empty costs a whole one; the parts' sums make another
+    pass.  The library takes the dequantisation and 2.1 us per thousand tokens
+    and million weights.  (us, kernel / library: 6144 x 5120, 384 tokens, two
+    parts in one round, 51 / 55, 448 tokens, one part, 78 / 63; 17408 x 5120, 384
+    tokens 124 / 177, 768 tokens 208 / 242; 25600 x 5120, 512 tokens 226 / 345, 768
+    tokens 290 / 371, 832 tokens, two rounds, 548 / 403; 12288 x 4096, 512 tokens 87 /
+    98; 9728 x 2560, 512 tokens 53 / 59; 3072 x 1024, 192 tokens 22 / 16.  Over eleven
+    shapes and 65 to 1024 tokens the choice is at most 20 % from the faster, at
+    6144 x 2048 and 128 tokens, and 0.6 % on average.)"""
+    long = in_f >= GEMM_T_LONG_ROWS
+    if rows > (GEMM_T_MAX_TOKENS if long else GEMM_T_SHORT_TOKENS):
+        return False
+    rounds = -(-(-(-out_f // 256) * -(-rows // 64) * splits) // cus)
+    kernel = 11e-3 * in_f * rounds / splits
+    if splits > 1:
+        kernel += 4.0 + 1.8e-6 * splits * rows * out_f
+    return kernel < 4.0 + 1e-6 * in_f * out_f * ((1.3 if long else 0.8) + 2.1e-3 * rows)
 
 
 def _torch_watched() -> bool:
@@ -102,8 +150,10 @@ def int4_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor) ->
         if y.dtype is not x.dtype:
             y = y.to(x.dtype)
         return y.view(*x.shape[:-1], qweight.shape[0])
-    if 1 < rows <= _ANY_INPUT_TOKENS or (1 < rows <= GEMM_MAX_TOKENS and x.shape[-1] == in_f
-                                         and in_f <= _MAX_COLS and _plain_bf16(x, qweight)):
+    if 1 < rows <= _ANY_INPUT_TOKENS or (
+            1 < rows <= GEMM_MAX_TOKENS and x.shape[-1] == in_f and in_f <= _MAX_COLS
+            and _plain_bf16(x, qweight)
+            and _gemm_serves(rows, qweight.shape[0], in_f, _cus(x.device.index))):
         if x.dtype is torch.bfloat16 and x.shape[-1] == in_f:
             return K.int4_gemm(qweight, scales, x)
         y = K.int4_gemm(qweight, scales, x.reshape(rows, in_f).to(torch.bfloat16))
@@ -114,16 +164,17 @@ def int4_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor) ->
 def int4_linear_t(x: torch.Tensor, qweight_t: torch.Tensor, scales_t: torch.Tensor) -> torch.Tensor:
     """x @ bf16(q*s) for a matrix stored as rows of the input dimension (the
     transposed down matrix) on the device, in x's dtype: the int4 MFMA GEMM
-    for up to GEMM_T_MAX_TOKENS rows of x (GEMM_T_SHORT_TOKENS for a smaller
-    matrix), else x @ dequantize (the reference's route,
+    for up to GEMM_T_MAX_TOKENS rows of x (GEMM_T_SHORT_TOKENS for a shorter K)
+    where it is the faster, else x @ dequantize (the reference's route,
     dip_stream_predispatch.py:213-215), on the transpose where that can be."""
     import _dip_hip as K
     rows = x.numel() // x.shape[-1]
-    most = (GEMM_T_MAX_TOKENS if 2 * qweight_t.numel() >= GEMM_T_LONG_VALUES
-            else GEMM_T_SHORT_TOKENS)
-    in_f, by8 = qweight_t.shape[0], qweight_t.shape[0] % 8 == 0
-    if rows <= _ANY_INPUT_TOKENS or (rows <= most and by8 and 2 * qweight_t.shape[1] <= _MAX_COLS
-                                     and _plain_bf16(x, qweight_t)):
+    in_f, out_f = qweight_t.shape[0], 2 * qweight_t.shape[1]
+    by8 = in_f % 8 == 0
+    if rows <= _ANY_INPUT_TOKENS or (
+            rows <= GEMM_T_MAX_TOKENS and by8 and out_f <= _MAX_COLS and _plain_bf16(x, qweight_t)
+            and _gemm_t_serves(rows, in_f, out_f, K.int4_gemm_t_splits(rows, out_f, in_f),
+                               _cus(x.device.index))):
         return K.int4_gemm_t(qweight_t, scales_t, x.to(torch.bfloat16)).to(x.dtype)
     if qweight_t.is_cuda and by8 and in_f <= _MAX_DEQUANT_T_ROWS:
         return F.linear(x, K.dequant_t(qweight_t, scales_t).to(x.dtype))

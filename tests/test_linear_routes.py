@@ -104,3 +104,74 @@ def test_modes_see_the_product():
     assert any("mm" in s for s in seen)
     with torch.no_grad(), torch.device("cuda"):
         assert torch.equal(Q.int4_linear(x, qw, sc), K.int4_gemm(qw, sc, x))
+
+
+# (rows, out, in, serves) on 256 CUs: both sides of each line
+@pytest.mark.parametrize("rows,out_f,in_f,serves", [
+    (384, 5120, 8192, True), (448, 5120, 8192, False), (512, 5120, 8192, False),
+    (256, 10240, 5120, True), (257, 6528, 4096, True), (257, 6656, 4096, False),
+    (448, 6144, 4096, False), (448, 6144, 2048, True), (320, 9728, 2560, True),
+    (448, 7040, 4096, True), (448, 4608, 4096, True), (512, 25600, 5120, True),
+    (513, 25600, 5120, False), (65, 1024, 5120, True)])
+def test_linear_rule(rows, out_f, in_f, serves):
+    import qlinear as Q
+    assert Q._gemm_serves(rows, out_f, in_f, 256) == serves
+
+
+@pytest.mark.parametrize("rows,in_f,out_f,serves", [
+    (512, 25600, 5120, True), (768, 25600, 5120, True), (769, 25600, 5120, False),
+    (768, 17408, 5120, True), (832, 17408, 5120, False), (384, 6144, 5120, True),
+    (448, 6144, 5120, False), (512, 12288, 4096, True), (513, 12288, 4096, False),
+    (320, 12288, 4096, True), (768, 16384, 2560, True), (192, 3072, 1024, False),
+    (512, 9728, 2560, True)])
+def test_transposed_rule(rows, in_f, out_f, serves):
+    import _dip_hip as K
+    import qlinear as Q
+    splits = K.int4_gemm_t_splits(rows, out_f, in_f)  # 256 CUs, here and on the device
+    assert Q._gemm_t_serves(rows, in_f, out_f, splits, 256) == serves
+
+
+def _calls(monkeypatch, *names):
+    import _dip_hip as K
+    seen = []
+    for n in names:
+        def wrapped(*a, n=n, f=getattr(K, n), **kw):
+            seen.append(n)
+            return f(*a, **kw)
+        monkeypatch.setattr(K, n, wrapped)
+    return seen
+
+
+def _close(got, x, w):
+    """One bf16 rounding and fp32 sums, against fp64 (the weights are the
+    route's: exact q * s, or rounded to bf16 once, 2^-9 of each term)."""
+    ref, terms = x.double() @ w.double(), x.double().abs() @ w.double().abs()
+    return bool(((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -9 * terms).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,entry", [(513, "int4_gemm_t"), (768, "int4_gemm_t"),
+                                        (769, "dequant_t")])
+def test_transposed_route_of_a_long_matrix(rows, entry, monkeypatch):
+    import qlinear as Q
+    print(f"transposed route, 16384 x 2560, {rows} rows", flush=True)
+    qw, sc = _weight(16384, 2560, device="cuda")
+    x = _x(rows, 16384, "cuda")
+    w = Q.dequantize(qw, sc)
+    seen = _calls(monkeypatch, "int4_gemm_t", "dequant_t")
+    got = Q.int4_linear_t(x, qw, sc)
+    assert seen == [entry] and _close(got, x, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,in_f,entry", [(384, 4096, "int4_gemm"), (448, 4096, "dequant_rows"),
+                                             (448, 2048, "int4_gemm"), (513, 2048, "dequant_rows")])
+def test_linear_route_by_workgroups(rows, in_f, entry, monkeypatch):
+    import qlinear as Q
+    print(f"linear route, 5120 x {in_f}, {rows} rows", flush=True)
+    qw, sc = _weight(5120, in_f, device="cuda")
+    x = _x(rows, in_f, "cuda")
+    w = Q.dequantize(qw, sc).t()
+    seen = _calls(monkeypatch, "int4_gemm", "dequant_rows")
+    got = Q.int4_linear(x, qw, sc)
+    assert seen == [entry] and _close(got, x, w)
