@@ -408,14 +408,22 @@ int launch_split_tokens(const GemmArgs& a, hipStream_t s) {
   if (!scales_by_dword(a) ||
       split_lds_bytes(TM, rw, few ? 8 : 4, a.K / kGroupSize) > kGemmLds / (few ? 1 : 2))
     return launch_split<TM, 2, 4, 1, false, GU>(a, s);
+  // two pairs of gate and up tiles come with more than 1.5 workgroups per CU
+  if constexpr (GU) {
+    if (rw == 4) return launch_split<TM, 4, 4, 2, true, GU>(a, s);
+    return few ? launch_split<TM, 2, 8, 2, true, GU>(a, s) : launch_split<TM, 2, 4, 2, true, GU>(a, s);
+  } else {
 #define DIP_SPLIT(R)                                                    \
   if (rw == (R))                                                        \
     return few ? launch_split<TM, R, 8, 2, true, GU>(a, s)              \
                : launch_split<TM, R, 4, 2, true, GU>(a, s);
-  DIP_SPLIT(2) DIP_SPLIT(4)
-  if constexpr (!GU) { DIP_SPLIT(1) DIP_SPLIT(3) }
+    DIP_SPLIT(2) DIP_SPLIT(3) DIP_SPLIT(4)
 #undef DIP_SPLIT
-  return DIP_ERR_UNSUPPORTED;
+    // one block of tokens has a single tile a workgroup only while those are few:
+    // beyond one to a CU two tiles or more cost less
+    if constexpr (TM == 1) return launch_split<TM, 1, 8, 2, true, GU>(a, s);
+    else return few ? launch_split<TM, 1, 8, 2, true, GU>(a, s) : launch_split<TM, 1, 4, 2, true, GU>(a, s);
+  }
 }
 
 // ---------------------------------------------------------------------------

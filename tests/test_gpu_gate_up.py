@@ -16,7 +16,8 @@ from gpu_util import dev, dev_bf16, random_bf16, random_int4
 pytestmark = pytest.mark.gpu
 
 CASES = [(2, 5, 128), (2, 16, 384), (3, 17, 128), (16, 31, 640), (17, 1000, 256), (31, 40, 1152),
-         (16, 7000, 384), (32, 6161, 256),                  # split kernel, two pairs of tiles
+         (16, 7000, 384), (32, 6161, 256),                  # split kernel, a pair of tiles, 4 waves
+         (16, 12322, 384), (9, 12321, 256), (32, 14343, 256),  # two pairs of tiles
          (33, 8, 512), (48, 1003, 384), (65, 1285, 640),    # split kernel, several token blocks
          (64, 10241, 256), (100, 5135, 384),                # tiled, two K parts
          (64, 20481, 128), (333, 3500, 640),                # tiled, one K part

@@ -19,7 +19,11 @@ CASES = [(1, 5, 128), (2, 16, 384), (3, 17, 128), (16, 31, 640), (17, 1000, 256)
          (64, 20480, 256), (100, 10249, 384), (129, 9000, 512),  # tiled, two K parts
          (64, 40961, 128), (333, 7000, 640), (130, 25600, 128),  # tiled, one K part
          (700, 24001, 256),                                # tiled, four row tiles a wave
-         (7, 48, 1 << 17), (40, 33, 40960)]                # scales from memory
+         (7, 48, 1 << 17), (40, 33, 40960),                # scales from memory
+         (9, 4271, 256), (16, 8279, 256), (9, 12501, 256),  # split, 8 waves: two to four tiles
+         (20, 4271, 256), (32, 8279, 256), (20, 12501, 256),
+         (9, 36971, 256), (16, 16507, 256), (9, 24739, 256),  # split, 4 waves
+         (768, 331, 256), (201, 2307, 256), (100, 5125, 256), (20, 16507, 256), (32, 24739, 256)]
 
 
 @pytest.mark.parametrize("m,n,k", CASES)

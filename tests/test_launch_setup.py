@@ -21,7 +21,9 @@ int hipGetDevice(int* d) { *d = device; return 0; }
 int hipDeviceGetAttribute(int* v, int a, int d) { *v = 256; return 0; }
 int hipGetLastError(void) { int e = last; last = 0; return e; }
 int hipFuncSetAttribute(const void* f, int a, int v) { ++asked; return refused ? (last = 1) : 0; }
-int hipLaunchKernel(const void* f, ...) { ++launches; return 0; }
+int __hipPushCallConfiguration() { return 0; }
+int __hipPopCallConfiguration() { return 0; }
+int hipLaunchKernel(const void* f) { ++launches; return 0; }
 """
 
 CALLS = r"""
@@ -61,9 +63,9 @@ def test_failed_setup_is_reported_every_time(tmp_path, call):
 def test_setup_runs_once_per_device(tmp_path, call):
     out = _run(tmp_path, f"""
 f = calls[{call!r}]
-assert f() != 0          # refused
+assert f() != 0 and shim.shim_launches() == 0  # refused
 shim.shim_refuse(0)
-assert f() == 0          # asked again, and granted
+assert f() == 0 and shim.shim_launches() > 0  # asked again, and granted
 seen = shim.shim_asked()
 assert f() == 0 and shim.shim_asked() == seen
 shim.shim_device(1)      # another device of the same process
