@@ -57,12 +57,9 @@ class CABuffers:
         dev = self.device
         self.gpu_up_qw = torch.empty(k, up_in_packed, dtype=torch.int8, device=dev)
         self.gpu_up_sc = torch.empty(k, up_ngroups, dtype=torch.bfloat16, device=dev)
-        self.pin_up_qw = torch.empty(k, up_in_packed, dtype=torch.int8).pin_memory()
-        self.pin_up_sc = torch.empty(k, up_ngroups, dtype=torch.bfloat16).pin_memory()
         self.gpu_dn_qw = torch.empty(k, down_out // 2, dtype=torch.int8, device=dev)
         self.gpu_dn_sc = torch.empty(k, down_ngroups, dtype=torch.bfloat16, device=dev)
-        self.pin_dn_qw = torch.empty(k, down_out // 2, dtype=torch.int8).pin_memory()
-        self.pin_dn_sc = torch.empty(k, down_ngroups, dtype=torch.bfloat16).pin_memory()
+        self._pins = None
         self.copy_stream = torch.cuda.Stream(device=dev)
         self.h = torch.empty(k, dtype=torch.bfloat16, device=dev)
         self._g = {}
@@ -92,6 +89,20 @@ class CABuffers:
         if t is None:
             t = self._g[inter] = torch.empty(inter, dtype=torch.bfloat16, device=self.device)
         return t
+
+    def pins(self):
+        """Pinned staging for the host gather: the shape of the device's up and
+        down rows and scales, k of each (about 80 MB at the 32B shape, keep 0.6),
+        made when a matrix that the device cannot read first needs it."""
+        if self._pins is None:
+            rows = (self.gpu_up_qw, self.gpu_up_sc, self.gpu_dn_qw, self.gpu_dn_sc)
+            self._pins = tuple(torch.empty(r.shape, dtype=r.dtype, pin_memory=True) for r in rows)
+        return self._pins
+
+    pin_up_qw = property(lambda self: self.pins()[0])
+    pin_up_sc = property(lambda self: self.pins()[1])
+    pin_dn_qw = property(lambda self: self.pins()[2])
+    pin_dn_sc = property(lambda self: self.pins()[3])
 
 
 class CADIPMlp(nn.Module):
@@ -160,7 +171,7 @@ class CADIPMlp(nn.Module):
         chunk's copies are queued as soon as it is gathered, so they run
         while the next chunk is gathered."""
         b = self.buf
-        pins = (b.pin_up_qw, b.pin_up_sc, b.pin_dn_qw, b.pin_dn_sc)
+        pins = b.pins()
         # No wait on the compute stream: _decode_host_gather synchronised it on the
         # host before the read-back, so the previous layer's reads of the
         # staging rows are done, and the hits' GEMV queued since reads only

@@ -81,3 +81,28 @@ def test_module_with_pinned_and_pageable_matrices():
     print("pageable", flush=True)
     assert torch.equal(m(x), y)
     assert (m.buf.last_n_hit, m.buf.last_n_miss) == counts
+
+
+def test_host_gather_chunks_and_its_staging():
+    """The host gather's chunk size moves when rows are copied, never a bit; its
+    pinned staging exists only once a matrix has needed it."""
+    from dip_ca import CABuffers, CADIPMlp
+    H, I, keep = 1024, 3072, 0.6
+    L = O.make_layer(H, I, seed=9)
+    k = O.keep_count(I, keep)
+    d = torch.device("cuda:0")
+    buf = CABuffers(k, H // 2, H // 128, H, H // 128, d)
+    m = CADIPMlp(dev(L["gate_qw"]), dev_bf16(L["gate_sc"]), dev(L["up_qw"]),
+                 dev_bf16(L["up_sc"]), dev(L["down_t_qw"]), dev_bf16(L["down_t_sc"]), buf, keep,
+                 0.3, d, down_transposed=True)
+    m.set_cache(torch.arange(I))
+    x = dev_bf16(O.make_x(H, seed=4)).reshape(1, 1, -1)
+    print("read by the device", flush=True)
+    y = m(x)
+    assert buf._pins is None
+    m.up_qw = m.up_qw.clone()  # pageable
+    for chunk in (k, 333, 64, 2048):
+        print(f"host gather, chunks of {chunk}", flush=True)
+        buf.stream_chunk = chunk
+        assert torch.equal(m(x), y)
+    assert buf.pin_up_qw.is_pinned() and buf.pin_dn_sc.shape == (k, H // 128)
