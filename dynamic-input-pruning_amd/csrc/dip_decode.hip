@@ -430,8 +430,8 @@ __global__ __launch_bounds__(4 * kHeadDim) void attn_combine_kernel(
 //      that cover 64 (256) contiguous bytes of a row, the next chunk's while
 //      this one is worked on;
 //   3. the NW waves' partials are merged through LDS in a fixed order.
-// Bound by what one CU can fetch (each query head's workgroup reads its kv
-// head's rows).  64 / 8 heads, us in a graph: 121 rows of 128 7.1 -> 5.5, 101
+// Bound by what one CU can fetch: one workgroup per query head occupies 32 or
+// 64 CUs of the chip, and each reads its kv head's rows.  64 / 8 heads, us in a graph: 121 rows of 128 7.1 -> 5.5, 101
 // rows of 1024 7.3 -> 5.5, 501 rows 11.8 -> 10.0, 701 rows 15.3 -> 11.9, 1021
 // rows 18.5 -> 14.7 (before: 16 waves without room for a chunk ahead, 16-byte
 // pieces of 64 lines per key load, 4-byte value loads; two chunks ahead on 8

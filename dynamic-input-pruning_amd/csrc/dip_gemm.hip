@@ -677,7 +677,7 @@ int launch_gemm(const GemmArgs& a, hipStream_t s) {
 // (25600 x 5120, 64 tokens, 200 workgroups: 35, with one part 41), else with one
 // (100 tokens, 400 workgroups: 57, with two parts 63; 5120 x 8192, 400 tokens,
 // 280 workgroups: two parts 93), and with four row tiles per wave from 1024
-// workgroups of them (25600 x 5120: 333 tokens, 600 of them, 151 against 138
+// workgroups of them (25600 x 5120: 333 tokens, 600 of them, 148 against 132
 // with two; 2048 tokens, 3200 of them, 639 against 718).
 // Gate and up with the SwiGLU between them (GU) follow the same lines with
 // their rows counted together; us against the two products and dip_swiglu:

@@ -113,8 +113,8 @@ __global__ __launch_bounds__(kAsmThreads) void ca_assemble_kernel(
 // own count ends the run: the host learns it only afterwards.  5161 rows of
 // 4224 bytes 420 us, 52 GB/s, the rate of a plain copy over the link (64 to
 // 1024 blocks and 1 to 8 vectors a lane are within 4 %).  A layer's whole
-// token, 12288 x 4096, 5161 misses: 765 us with host threads gathering into
-// staging for DMA copies, 500 us so.
+// token, 12288 x 4096, 5161 misses: 759 us with host threads gathering into
+// staging for DMA copies, 487 us so.
 // ---------------------------------------------------------------------------
 constexpr int kStreamPieces = 8;
 constexpr int kStreamBlocks = 256;
