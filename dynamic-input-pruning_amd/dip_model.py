@@ -423,23 +423,23 @@ class DIPDecoder:
         from transformers.models.qwen3 import modeling_qwen3 as Q
         from qlinear import QuantLinear
         inner = self.model.model
-        found = [({"": self.model}, "", Q.Qwen3ForCausalLM), (self.model._modules, "model", Q.Qwen3Model),
-                 (self.model._modules, "lm_head", nn.Linear),
-                 (inner._modules, "embed_tokens", nn.Embedding),
-                 (inner._modules, "norm", Q.Qwen3RMSNorm),
-                 (inner._modules, "rotary_emb", Q.Qwen3RotaryEmbedding),
-                 (inner._modules, "layers", nn.ModuleList)]
+        under = lambda m: getattr(m, "_modules", {})  # (a stand-in for a module has none)
+        found = [({"": self.model}, "", Q.Qwen3ForCausalLM), (under(self.model), "model", Q.Qwen3Model),
+                 (under(self.model), "lm_head", nn.Linear),
+                 (under(inner), "embed_tokens", nn.Embedding),
+                 (under(inner), "norm", Q.Qwen3RMSNorm),
+                 (under(inner), "rotary_emb", Q.Qwen3RotaryEmbedding),
+                 (under(inner), "layers", nn.ModuleList)]
         buffers = []
         for i, L in enumerate(self.layers):
             a = L.self_attn
-            found += [(inner.layers._modules, str(i), Q.Qwen3DecoderLayer),
-                      (L._modules, "input_layernorm", Q.Qwen3RMSNorm),
-                      (L._modules, "post_attention_layernorm", Q.Qwen3RMSNorm),
-                      (L._modules, "self_attn", Q.Qwen3Attention),
-                      (a._modules, "q_norm", Q.Qwen3RMSNorm),
-                      (a._modules, "k_norm", Q.Qwen3RMSNorm)]
+            found += [(under(inner.layers), str(i), Q.Qwen3DecoderLayer),
+                      (under(L), "input_layernorm", Q.Qwen3RMSNorm),
+                      (under(L), "post_attention_layernorm", Q.Qwen3RMSNorm),
+                      (under(L), "self_attn", Q.Qwen3Attention),
+                      (under(a), "q_norm", Q.Qwen3RMSNorm), (under(a), "k_norm", Q.Qwen3RMSNorm)]
             for p in ("q_proj", "k_proj", "v_proj"):
-                found.append((a._modules, p, QuantLinear))
+                found.append((under(a), p, QuantLinear))
                 buffers += [(getattr(a, p)._buffers, n, getattr(a, p)._buffers[n])
                             for n in ("qweight", "scales")]
         modules = [(d, n, d.get(n), cls) for d, n, cls in found]

@@ -280,3 +280,28 @@ def test_two_decoders_of_one_model(tmp_path):
     for dec in (first, second):
         assert dec._prefill_fusible()
         assert torch.equal(dec.prefill(_ids(65)), before)
+
+
+def test_stand_in_for_the_model(tmp_path):
+    """An object with the model's parts, but no module of its class, decodes with
+    the fused steps and runs its own forward for prompts."""
+    from types import SimpleNamespace
+    from dip_model import DIPDecoder
+    print("prefill of a stand-in", flush=True)
+    dec = _decoder(tmp_path)
+    want, step = dec.prefill(_ids(65)), dec.step()
+    m, calls = dec.model, []
+
+    class StandIn:
+        config, lm_head = m.config, m.lm_head
+        model = SimpleNamespace(layers=list(m.model.layers), embed_tokens=m.model.embed_tokens,
+                                norm=m.model.norm, rotary_emb=m.model.rotary_emb)
+
+        def __call__(self, **kw):
+            calls.append(1)
+            return m(**kw)
+
+    other = DIPDecoder(StandIn(), 600)
+    assert other.fused and not other._prefill_fusible()
+    assert max_rel(other.prefill(_ids(65)).float(), want.float()) < 2e-2 and calls
+    assert max_rel(other.step().float(), step.float()) < 8e-2  # the sparse bound
