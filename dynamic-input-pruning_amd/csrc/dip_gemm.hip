@@ -105,7 +105,8 @@ struct ScaleRun {
 // sums with one instruction each (gate and up of 12288 x 4096, 333 tokens 108.9 ->
 // 109.1 us; with a class compare and its mask 109.6), and the lanes that hold such
 // a one come here for their outputs that are not finite, so other tokens keep
-// their bits.  A sum that is NaN ends the walk.
+// their bits.  A sum that is NaN ends the walk (512 tokens through 25600 x 5120:
+// 190 us, one of them infinite 570, all NaN 510, an infinity in each 13 ms).
 DIP_DEV float plain_dot(const int8_t* qw, const uint16_t* sc, const uint16_t* x, int row, int tok,
                         int K) {
   const int ngroups = K >> 7;
