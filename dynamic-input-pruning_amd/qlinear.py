@@ -52,10 +52,10 @@ _ANY_INPUT_TOKENS = 64
 # 124, 135 / 143; 3072 x 1024 18 / 41, 23 / 42, 24 / 42, 24 / 45.  Over ten shapes and
 # 65 to 768 tokens the one launch is at most 8 % behind, at 17408 x 5120 and 768).
 GATE_UP_MAX_TOKENS = 768
-# The transposed GEMM's limits, for a K of GEMM_T_LONG_ROWS or more, over which the
-# library's product does not fill the chip (768 tokens, dequantize and product:
-# 25600 x 5120 371 us, 17408 x 5120 242, 2.7 us per million weights), and for
-# shorter ones (14336 x 4096 128 us, 2.2 per million).  Within them _gemm_t_serves.
+# The transposed GEMM's limits, for a K beyond GEMM_T_LONG_ROWS, where the library
+# slows down (576 tokens, dequantize and product, us per million weights: 16384 x
+# 5120 1.77, 17408 x 5120 2.49, 25600 x 5120 2.59), and for a shorter one.  Within
+# them _gemm_t_serves.
 GEMM_T_MAX_TOKENS = 768
 GEMM_T_SHORT_TOKENS = 512
 GEMM_T_LONG_ROWS = 16384
@@ -65,25 +65,31 @@ _MAX_COLS = 1 << 20
 _MAX_DEQUANT_T_ROWS = 65535 * 128
 
 
-@functools.lru_cache(maxsize=None)
-def _cus(device_index: int) -> int:
-    return torch.cuda.get_device_properties(device_index).multi_processor_count
-
-
 def _gemm_serves(rows: int, out_f: int, in_f: int, cus: int) -> bool:
     """Whether the int4 GEMM beats dequantize + the library for 65 rows or more.
-    Its workgroups are 128 weight rows x 64 tokens.  Just past one to a CU they
-    lose their second part of K, and a CU with one of them waits on memory:
-    beyond 256 tokens the library is faster there (us, 448 tokens: 5120 x 8192,
-    280 workgroups, 87 / 72; 5120 x 25600, 280, 363 / 328; 6144 x 4096, 336, 46 /
-    43), but for a short K (384 tokens: 6144 x 2048, 288 workgroups, 26 / 31; 9728 x
-    2560, 456, 34 / 42).  At 1.5 to a CU the two are level (10240 x 5120, 384 tokens,
-    480 workgroups, 63 / 69), and up to one the GEMM wins (5120 x 8192, 384
-    tokens, 240 workgroups, 51 / 65)."""
+    Its workgroups are 128 weight rows x 64 tokens, the row blocks dealt to 8
+    XCDs.  Up to 256 tokens it always does; beyond, where
+      * at most one comes to a CU, if no XCD has more of them than CUs (us, GEMM /
+        library: 5120 x 8192, 384 tokens, 240 workgroups, 51 / 65; 6400 x 5120, 320
+        tokens, 250, 35 of them on an XCD, 63 / 50);
+      * more come, and run in rounds of one to a CU, two at least (a CU with one
+        waits on memory), if these are full enough: 92 % from K 6144 (5120 x 8192,
+        448 tokens, 55 %, 87 / 72; 7424 x 8192, 512, 91 %, 96 / 90; 8704 x 8192, 448,
+        93 %, 97 / 100), 72 % of three or more from K 4096 (8704 x 4096, 512, 71 %,
+        65 / 59; 10240 x 5120, 448, 73 %, 79 / 78).  Two rounds of a shorter K win or
+        lose by a tenth, as the library's steps fall (5632 x 5120, 448 tokens, 56 /
+        60, 512 56 / 53), and short rows win (6144 x 2048, 384, 56 %, 26 / 31)."""
     if rows > GEMM_MAX_TOKENS:
         return False
-    workgroups = -(-out_f // 128) * -(-rows // 64)
-    return rows <= 256 or in_f < 4096 or not cus < workgroups <= 1.5 * cus
+    row_blocks, token_blocks = -(-out_f // 128), -(-rows // 64)
+    workgroups = row_blocks * token_blocks
+    if rows <= 256:
+        return True
+    if workgroups <= cus:
+        return 8 * -(-row_blocks // 8) * token_blocks <= cus
+    rounds = max(2, -(-workgroups // cus))
+    full = 0.92 if in_f >= 6144 else 0.72 if in_f >= 4096 and rounds > 2 else 0.0
+    return workgroups >= full * cus * rounds
 
 
 def _gemm_t_serves(rows: int, in_f: int, out_f: int, splits: int, cus: int) -> bool:
@@ -91,50 +97,72 @@ def _gemm_t_serves(rows: int, in_f: int, out_f: int, splits: int, cus: int) -> b
     dequantize + the library for 65 rows or more.  Its workgroups (256 columns x
     64 tokens x a part) run in rounds of one to a CU, 11 ns per row of K each, so
     a round that is nearly empty costs a whole one; the parts' sums make another
-    pass.  The library takes the dequantisation and 2.1 us per thousand tokens
-    and million weights.  (us, kernel / library: 6144 x 5120, 384 tokens, two
-    parts in one round, 51 / 55, 448 tokens, one part, 78 / 63; 17408 x 5120, 384
-    tokens 124 / 177, 768 tokens 208 / 242; 25600 x 5120, 512 tokens 226 / 345, 768
-    tokens 290 / 371, 832 tokens, two rounds, 548 / 403; 12288 x 4096, 512 tokens 87 /
-    98; 9728 x 2560, 512 tokens 53 / 59; 3072 x 1024, 192 tokens 22 / 16.  Over eleven
-    shapes and 65 to 1024 tokens the choice is at most 20 % from the faster, at
-    6144 x 2048 and 128 tokens, and 0.6 % on average.)"""
-    long = in_f >= GEMM_T_LONG_ROWS
+    pass.  The library takes 1.0 us per million weights (1.2 where K is long) and
+    2.3 more per thousand tokens.  (us, kernel / library: 6144 x 5120, 384 tokens,
+    two parts in one round, 51 / 55, 448 tokens, one part, 78 / 63; 17408 x 5120,
+    384 tokens 124 / 177, 768 tokens 208 / 242; 25600 x 5120, 512 tokens 226 / 345,
+    768 tokens 290 / 371, 832 tokens, two rounds, 548 / 403; 12288 x 4096, 512
+    tokens 87 / 98; 3072 x 1024, 192 tokens 22 / 16.  Over 28 shapes and 65 to 1024
+    tokens the choice is 0.7 % from the faster on average, 28 points of 487 more
+    than 4 %, the worst 2048 x 4096, 256 tokens, 28 / 19.)"""
+    long = in_f > GEMM_T_LONG_ROWS
     if rows > (GEMM_T_MAX_TOKENS if long else GEMM_T_SHORT_TOKENS):
         return False
     rounds = -(-(-(-out_f // 256) * -(-rows // 64) * splits) // cus)
     kernel = 11e-3 * in_f * rounds / splits
     if splits > 1:
-        kernel += 4.0 + 1.8e-6 * splits * rows * out_f
-    return kernel < 4.0 + 1e-6 * in_f * out_f * ((1.3 if long else 0.8) + 2.1e-3 * rows)
+        kernel += 2.0 + 1.5e-6 * splits * rows * out_f
+    return kernel < 2.0 + 1e-6 * in_f * out_f * ((1.2 if long else 1.0) + 2.3e-3 * rows)
+
+
+@functools.lru_cache(maxsize=4096)
+def _gemm_route(rows: int, out_f: int, in_f: int, device_index: int) -> bool:
+    cus = torch.cuda.get_device_properties(device_index).multi_processor_count
+    return in_f <= _MAX_COLS and _gemm_serves(rows, out_f, in_f, cus)
+
+
+@functools.lru_cache(maxsize=4096)
+def _gemm_t_route(rows: int, in_f: int, out_f: int, device_index: int) -> bool:
+    import _dip_hip as K
+    cus = torch.cuda.get_device_properties(device_index).multi_processor_count
+    return (in_f % 8 == 0 and out_f <= _MAX_COLS
+            and _gemm_t_serves(rows, in_f, out_f, K.int4_gemm_t_splits(rows, out_f, in_f), cus))
+
+
+# (bound once: a small prompt's call is host time, 1.3 us of it these checks)
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_modes = torch._C._len_torch_function_stack
+_any_autocast = torch._C._is_any_autocast_enabled
+_functorch_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+_forward_ad = torch.autograd.forward_ad
+_is_tracing = torch._C._is_tracing
+_is_compiling = torch.compiler.is_compiling
+_is_grad_enabled = torch.is_grad_enabled
 
 
 def _torch_watched() -> bool:
     """Whether the torch ops of a call would do more than compute: an active
     dispatch or function mode sees them (a default device, itself such a mode,
     does not count), or autocast gives their results another type than bf16."""
-    if torch._C._len_torch_dispatch_stack():
+    if _dispatch_modes():
         return True
-    if torch._C._len_torch_function_stack():
+    if _function_modes():
         from torch.overrides import _get_current_function_mode_stack
         from torch.utils._device import DeviceContext
         if any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()):
             return True
-    return (torch.is_autocast_enabled("cuda")
+    return (_any_autocast() and torch.is_autocast_enabled("cuda")
             and torch.get_autocast_dtype("cuda") != torch.bfloat16)
 
 
-def _plain_bf16(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Whether x is a plain bf16 tensor beside `weight` on the device that nothing
-    differentiates, batches, traces or watches: what a kernel called on its data
-    may take in place of torch ops."""
-    return (type(x) is torch.Tensor and x.dtype == torch.bfloat16 and x.is_cuda
-            and x.device == weight.device
-            and not (x.requires_grad and torch.is_grad_enabled())
-            and not torch._C._functorch.is_functorch_wrapped_tensor(x)
-            and torch.autograd.forward_ad._current_level < 0
-            and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
-            and not _torch_watched())
+def _plain_bf16(x: torch.Tensor) -> bool:
+    """Whether x is a plain bf16 tensor on the device that nothing differentiates,
+    batches, traces or watches: what a kernel called on its data may take in
+    place of torch ops.  (Both refuse a weight on another device.)"""
+    return (type(x) is torch.Tensor and x.dtype is torch.bfloat16 and x.is_cuda
+            and not (x.requires_grad and _is_grad_enabled())
+            and not _functorch_wrapped(x) and _forward_ad._current_level < 0
+            and not _is_tracing() and not _is_compiling() and not _torch_watched())
 
 
 def int4_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor) -> torch.Tensor:
@@ -150,10 +178,11 @@ def int4_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor) ->
         if y.dtype is not x.dtype:
             y = y.to(x.dtype)
         return y.view(*x.shape[:-1], qweight.shape[0])
-    if 1 < rows <= _ANY_INPUT_TOKENS or (
-            1 < rows <= GEMM_MAX_TOKENS and x.shape[-1] == in_f and in_f <= _MAX_COLS
-            and _plain_bf16(x, qweight)
-            and _gemm_serves(rows, qweight.shape[0], in_f, _cus(x.device.index))):
+    if rows > _ANY_INPUT_TOKENS:
+        if (rows <= GEMM_MAX_TOKENS and x.shape[-1] == in_f and _plain_bf16(x)
+                and _gemm_route(rows, qweight.shape[0], in_f, x.device.index)):
+            return K.int4_gemm(qweight, scales, x)
+    elif rows > 1:
         if x.dtype is torch.bfloat16 and x.shape[-1] == in_f:
             return K.int4_gemm(qweight, scales, x)
         y = K.int4_gemm(qweight, scales, x.reshape(rows, in_f).to(torch.bfloat16))
@@ -168,15 +197,12 @@ def int4_linear_t(x: torch.Tensor, qweight_t: torch.Tensor, scales_t: torch.Tens
     where it is the faster, else x @ dequantize (the reference's route,
     dip_stream_predispatch.py:213-215), on the transpose where that can be."""
     import _dip_hip as K
-    rows = x.numel() // x.shape[-1]
-    in_f, out_f = qweight_t.shape[0], 2 * qweight_t.shape[1]
-    by8 = in_f % 8 == 0
+    rows, in_f = x.numel() // x.shape[-1], qweight_t.shape[0]
     if rows <= _ANY_INPUT_TOKENS or (
-            rows <= GEMM_T_MAX_TOKENS and by8 and out_f <= _MAX_COLS and _plain_bf16(x, qweight_t)
-            and _gemm_t_serves(rows, in_f, out_f, K.int4_gemm_t_splits(rows, out_f, in_f),
-                               _cus(x.device.index))):
+            rows <= GEMM_T_MAX_TOKENS and _plain_bf16(x)
+            and _gemm_t_route(rows, in_f, 2 * qweight_t.shape[1], x.device.index)):
         return K.int4_gemm_t(qweight_t, scales_t, x.to(torch.bfloat16)).to(x.dtype)
-    if qweight_t.is_cuda and by8 and in_f <= _MAX_DEQUANT_T_ROWS:
+    if qweight_t.is_cuda and in_f % 8 == 0 and in_f <= _MAX_DEQUANT_T_ROWS:
         return F.linear(x, K.dequant_t(qweight_t, scales_t).to(x.dtype))
     return x @ dequantize(qweight_t, scales_t).to(x.dtype)
 
@@ -184,7 +210,7 @@ def int4_linear_t(x: torch.Tensor, qweight_t: torch.Tensor, scales_t: torch.Tens
 def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """F.silu(gate) * up, in one launch for plain bf16 tensors on the device
     (the same roundings)."""
-    if gate.is_cuda and gate.shape == up.shape and _plain_bf16(gate, up) and _plain_bf16(up, gate):
+    if gate.is_cuda and gate.shape == up.shape and _plain_bf16(gate) and _plain_bf16(up):
         import _dip_hip as K
         return K.swiglu(gate, up)
     return F.silu(gate) * up
@@ -197,7 +223,7 @@ def int4_gate_up(x, gate_qw, gate_sc, up_qw, up_sc):
     in_f = gate_qw.shape[1] * 2
     rows = x.numel() // in_f
     if not (1 < rows <= GATE_UP_MAX_TOKENS and x.shape[-1] == in_f and in_f <= _MAX_COLS
-            and gate_qw.shape == up_qw.shape and _plain_bf16(x, gate_qw)):
+            and gate_qw.shape == up_qw.shape and _plain_bf16(x)):
         return None
     return K.int4_gemm_swiglu(gate_qw, gate_sc, up_qw, up_sc, x)
 

@@ -109,10 +109,12 @@ def test_modes_see_the_product():
 # (rows, out, in, serves) on 256 CUs: both sides of each line
 @pytest.mark.parametrize("rows,out_f,in_f,serves", [
     (384, 5120, 8192, True), (448, 5120, 8192, False), (512, 5120, 8192, False),
-    (256, 10240, 5120, True), (257, 6528, 4096, True), (257, 6656, 4096, False),
-    (448, 6144, 4096, False), (448, 6144, 2048, True), (320, 9728, 2560, True),
-    (448, 7040, 4096, True), (448, 4608, 4096, True), (512, 25600, 5120, True),
-    (513, 25600, 5120, False), (65, 1024, 5120, True)])
+    (256, 10240, 5120, True), (257, 6144, 4096, True), (257, 6528, 4096, False),
+    (257, 6656, 4096, True), (448, 4096, 4096, True), (448, 4608, 4096, False),
+    (448, 6144, 4096, True), (449, 8704, 4096, False), (449, 8704, 2048, True), (449, 9600, 4096, True), (320, 9728, 2560, True),
+    (448, 7040, 4096, True), (512, 7424, 8192, False), (448, 8704, 8192, True), (448, 8704, 6144, True), (384, 8704, 6144, False),
+    (512, 8704, 8192, False), (512, 25600, 5120, True), (513, 25600, 5120, False),
+    (65, 1024, 5120, True)])
 def test_linear_rule(rows, out_f, in_f, serves):
     import qlinear as Q
     assert Q._gemm_serves(rows, out_f, in_f, 256) == serves
@@ -122,7 +124,7 @@ def test_linear_rule(rows, out_f, in_f, serves):
     (512, 25600, 5120, True), (768, 25600, 5120, True), (769, 25600, 5120, False),
     (768, 17408, 5120, True), (832, 17408, 5120, False), (384, 6144, 5120, True),
     (448, 6144, 5120, False), (512, 12288, 4096, True), (513, 12288, 4096, False),
-    (320, 12288, 4096, True), (768, 16384, 2560, True), (192, 3072, 1024, False),
+    (320, 12288, 4096, True), (768, 17408, 2560, True), (513, 16384, 2560, False), (192, 3072, 1024, False),
     (512, 9728, 2560, True)])
 def test_transposed_rule(rows, in_f, out_f, serves):
     import _dip_hip as K
@@ -154,9 +156,9 @@ def _close(got, x, w):
                                         (769, "dequant_t")])
 def test_transposed_route_of_a_long_matrix(rows, entry, monkeypatch):
     import qlinear as Q
-    print(f"transposed route, 16384 x 2560, {rows} rows", flush=True)
-    qw, sc = _weight(16384, 2560, device="cuda")
-    x = _x(rows, 16384, "cuda")
+    print(f"transposed route, 16640 x 2560, {rows} rows", flush=True)
+    qw, sc = _weight(16640, 2560, device="cuda")
+    x = _x(rows, 16640, "cuda")
     w = Q.dequantize(qw, sc)
     seen = _calls(monkeypatch, "int4_gemm_t", "dequant_t")
     got = Q.int4_linear_t(x, qw, sc)
@@ -164,8 +166,8 @@ def test_transposed_route_of_a_long_matrix(rows, entry, monkeypatch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,in_f,entry", [(384, 4096, "int4_gemm"), (448, 4096, "dequant_rows"),
-                                             (448, 2048, "int4_gemm"), (513, 2048, "dequant_rows")])
+@pytest.mark.parametrize("rows,in_f,entry", [(384, 6144, "int4_gemm"), (448, 6144, "dequant_rows"),
+                                             (448, 4096, "int4_gemm"), (513, 4096, "dequant_rows")])
 def test_linear_route_by_workgroups(rows, in_f, entry, monkeypatch):
     import qlinear as Q
     print(f"linear route, 5120 x {in_f}, {rows} rows", flush=True)
