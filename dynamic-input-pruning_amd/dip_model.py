@@ -479,12 +479,14 @@ class DIPDecoder:
         K, inner, hd, nh = self._K, self.model.model, self.hd, self.nh
         plen = ids.shape[1]
         h = inner.embed_tokens(ids).view(plen, self.hidden)  # from here on the residual, in place
-        x = torch.empty_like(h)
         q = torch.empty(plen, nh * hd, dtype=self.dtype, device=self.device)
-        y = None
+        x = y = None
         for i, L in enumerate(self.layers):
             a, n_in, pn = L.self_attn, L.input_layernorm, L.post_attention_layernorm
             kc, vc = self.k_cache[i], self.v_cache[i]
+            # a layer's own, as who calls its MLP may keep it; else the same memory again
+            x = None
+            x = torch.empty_like(h)
             K.add_rmsnorm_rows(h, y, n_in.weight, x, n_in.variance_epsilon)
             qkv = int4_linear(x, *self._qkv_w[i])
             K.qk_norm_rope_cache_rows(qkv, a.q_norm.weight, a.k_norm.weight, self.cos, self.sin, q,
@@ -493,9 +495,8 @@ class DIPDecoder:
                 q.view(1, plen, nh, hd).transpose(1, 2), kc[None, :, :plen], vc[None, :, :plen],
                 is_causal=plen > 1, scale=a.scaling, enable_gqa=nh != self.nkv)
             o = a.o_proj(o.transpose(1, 2).reshape(1, plen, nh * hd))
-            m = torch.empty_like(h)  # the MLP's alone: who calls it may keep it
-            K.add_rmsnorm_rows(h, o.reshape(plen, -1), pn.weight, m, pn.variance_epsilon)
-            y = L.mlp(m.view(1, plen, -1)).reshape(plen, -1)
+            K.add_rmsnorm_rows(h, o.reshape(plen, -1), pn.weight, x, pn.variance_epsilon)
+            y = L.mlp(x.view(1, plen, -1)).reshape(plen, -1)
         n = inner.norm
         last = torch.empty(self.hidden, dtype=self.dtype, device=self.device)
         K.add_rmsnorm(h[-1], y[-1], n.weight, last, n.variance_epsilon)
